@@ -476,6 +476,24 @@ ESA_API int esa_linear_f32(const float* x, int rows, int in_features, int n_out,
                    const float* const* weight, const float* const* bias, float* const* y,
                    const int* out_features, void* stream);
 
+/* Weight and bias gradients of n (1-3) of the blocks' Linear layers over    */
+/* one batch of rows (the autograd of nn.Linear, esa/mha.py:12-15,           */
+/* esa/mlp_utils.py:18-37): dW_i = g_i^T x_i [out_i, in_i] and, where db_i   */
+/* is not null, db_i [out_i] = the column sums of g_i, for g_i [rows, out_i] */
+/* and x_i [rows, in_i], all ESA_BF16 or all ESA_F32, row-major and          */
+/* contiguous (the x_i may be one tensor: fc_q / fc_k / fc_v).  Products are */
+/* accumulated in fp32 and dW_i, db_i are fp32; fixed summation order        */
+/* (deterministic).  out_i and in_i are multiples of 8 (bf16) or 4 (fp32) up */
+/* to 16384, rows >= 1, device pointers 16-byte aligned.  g, x, dw, db,      */
+/* out_features and in_features are host arrays of n entries; workspace size */
+/* from the query.                                                           */
+ESA_API int esa_weight_grad_workspace_size(long long rows, int n, const int* out_features,
+                   const int* in_features, int dtype, size_t* bytes);
+ESA_API int esa_weight_grad(long long rows, int n, const void* const* g, const void* const* x,
+                   const int* out_features, const int* in_features, int dtype,
+                   float* const* dw, float* const* db, void* workspace, size_t workspace_bytes,
+                   void* stream);
+
 /* ------------------------------------------------------------------------ */
 /* Profiling hook (no counterpart in the reference; used by the benchmark).  */
 /* While enabled, every kernel launch of the entry points above is           */
@@ -484,7 +502,7 @@ ESA_API int esa_linear_f32(const float* x, int rows, int in_features, int n_out,
 /* launch count per kernel id (capacity >= ESA_PROFILE_KERNELS) and clears   */
 /* the record.  Not for concurrent use from several threads.                 */
 /* ------------------------------------------------------------------------ */
-#define ESA_PROFILE_KERNELS 23
+#define ESA_PROFILE_KERNELS 24
 ESA_API int esa_profile_enable(int on);
 ESA_API int esa_profile_collect(float* total_ms, int* launches, int capacity);
 ESA_API const char* esa_profile_kernel_name(int kernel);

@@ -103,6 +103,12 @@ _PROTOS = {
     # x rows in n_out | weight[] bias[] y[] out_features[] stream
     "esa_linear_f32": (_c_int, [_vp, _c_int, _c_int, _c_int, ctypes.POINTER(_vp), ctypes.POINTER(_vp),
                                 ctypes.POINTER(_vp), ctypes.POINTER(_c_int), _vp]),
+    "esa_weight_grad_workspace_size": (_c_int, [_c_i64, _c_int, ctypes.POINTER(_c_int), ctypes.POINTER(_c_int), _c_int,
+                                                ctypes.POINTER(_c_sz)]),
+    # rows n | g[] x[] out_features[] in_features[] dtype | dw[] db[] ws bytes stream
+    "esa_weight_grad": (_c_int, [_c_i64, _c_int, ctypes.POINTER(_vp), ctypes.POINTER(_vp), ctypes.POINTER(_c_int),
+                                 ctypes.POINTER(_c_int), _c_int, ctypes.POINTER(_vp), ctypes.POINTER(_vp), _vp, _c_sz,
+                                 _vp]),
     "esa_mab_residual_fwd": (_c_int, [_vp, _vp, _vp, _c_i64, _c_int, _vp, _vp]),
     "esa_mab_residual_bwd": (_c_int, [_vp, _vp, _c_i64, _c_int, _vp, _vp, _vp]),
     "esa_profile_enable": (_c_int, [_c_int]),
@@ -110,7 +116,7 @@ _PROTOS = {
     "esa_profile_kernel_name": (ctypes.c_char_p, [_c_int]),
 }
 
-PROFILE_KERNELS = 23
+PROFILE_KERNELS = 24
 
 _lock = threading.Lock()
 _lib = None

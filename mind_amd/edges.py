@@ -356,7 +356,7 @@ class _EdgeTokenLinear(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, g):
-        from .esa.linear import column_sum, weight_grad
+        from .esa.linear import column_sum, weight_bias_grads
         x, w2, src, dst, edge_attr, w_e = ctx.saved_tensors
         src_csr, dst_csr = ctx.csrs
         n, f = x.shape
@@ -372,10 +372,10 @@ class _EdgeTokenLinear(torch.autograd.Function):
         dx = dpq @ w2 if ctx.needs_input_grad[0] else None
         dweight = None
         if ctx.needs_input_grad[1]:
-            dw2 = weight_grad(dpq, x).to(w2.dtype)                # [2D, F]
+            dw2 = weight_bias_grads([(dpq, x)], [True], [False])[0][0].to(w2.dtype)   # [2D, F]
             parts = [dw2[:d], dw2[d:]]
             if edge_attr is not None:
-                parts.append(weight_grad(g, edge_attr).to(w2.dtype))   # [D, F_e]
+                parts.append(weight_bias_grads([(g, edge_attr)], [True], [False])[0][0].to(w2.dtype))   # [D, F_e]
             dweight = torch.cat(parts, 1)                          # [D, 2F (+ F_e)]
         dbias = column_sum(g).to(g.dtype) if ctx.has_bias and ctx.needs_input_grad[2] else None
         dattr = g @ w_e if edge_attr is not None and ctx.needs_input_grad[7] else None

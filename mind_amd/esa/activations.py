@@ -92,7 +92,7 @@ class _MabEpilogue(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, g):
-        from .linear import column_sum, weight_grad   # deferred: linear.py is a sibling with its own imports
+        from .linear import weight_bias_grads   # deferred: linear.py is a sibling with its own imports
         o, weight, z = ctx.saved_tensors
         lib, st, code = _lib.load(), _lib.stream_of(z), _DTYPES[z.dtype]
         dz = torch.empty_like(z)
@@ -107,9 +107,9 @@ class _MabEpilogue(torch.autograd.Function):
                        "esa_mish_bwd")
         wdt, bdt = ctx.dtypes
         do = torch.addmm(g_o, dz, weight) if ctx.needs_input_grad[0] else None
-        dw = weight_grad(dz, o).to(wdt) if ctx.needs_input_grad[1] else None
-        db = column_sum(dz).to(bdt) if bdt is not None and ctx.needs_input_grad[2] else None
-        return do, dw, db, (g if ctx.has_x and ctx.needs_input_grad[3] else None)
+        ((dw, db),) = weight_bias_grads([(dz, o)], [ctx.needs_input_grad[1]],
+                                        [bdt is not None and ctx.needs_input_grad[2]])
+        return do, None if dw is None else dw.to(wdt), None if db is None else db.to(bdt), (g if ctx.has_x and ctx.needs_input_grad[3] else None)
 
 
 def mab_epilogue(o: torch.Tensor, fc_o: nn.Linear, residual: torch.Tensor | None = None) -> torch.Tensor:
@@ -131,13 +131,10 @@ def mab_epilogue(o: torch.Tensor, fc_o: nn.Linear, residual: torch.Tensor | None
     return _MabEpilogue.apply(o, w, b, None if residual is None else residual.contiguous())
 
 
-_FUSED_COLSUM_MIN_COLS = 1024
-
-
 class _LinearMish(torch.autograd.Function):
     """y = mish(x W^T + b), an MLP's Linear -> Mish (esa/mlp_utils.py:18-37).  Forward: the GEMM, then
-    esa_mish_fwd.  Backward: esa_mish_bwd_colsum writes dz and the bias gradient (dz's column sums) in one
-    pass; dx = dz W and the split-K weight gradient follow.  Parameters enter in their own dtype and are cast
+    esa_mish_fwd.  Backward: esa_mish_bwd writes dz; dx = dz W and the weight and bias gradients (one kernel,
+    weight_bias_grads) follow.  Parameters enter in their own dtype and are cast
     inside, so their gradients are returned in it (fp32 under autocast)."""
 
     @staticmethod
@@ -154,33 +151,17 @@ class _LinearMish(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, g):
-        import ctypes
-
-        from .linear import column_sum, weight_grad
+        from .linear import weight_bias_grads   # deferred: linear.py is a sibling with its own imports
         x, w, z = ctx.saved_tensors
         wdt, bdt = ctx.dtypes
-        lib, st, code = _lib.load(), _lib.stream_of(z), _DTYPES[z.dtype]
         g = g.to(z.dtype).contiguous()
         dz = torch.empty_like(z)
-        rows, cols = z.shape
-        db = None
-        # fused from 1024 columns (129,850 x 2048 bf16: 334 vs 397 us for the two kernels); at 512 columns the
-        # two cost the same (104 vs 105 us) and the two kernels run
-        if bdt is not None and ctx.needs_input_grad[2] and cols % 4 == 0 and cols >= _FUSED_COLSUM_MIN_COLS:
-            n = ctypes.c_size_t(0)
-            _lib.check(lib.esa_column_sum_workspace_size(rows, cols, ctypes.byref(n)), "esa_column_sum_workspace_size")
-            ws = torch.empty(int(n.value), dtype=torch.uint8, device=z.device)
-            db = torch.empty(cols, dtype=torch.float32, device=z.device)
-            _lib.check(lib.esa_mish_bwd_colsum(z.data_ptr(), g.data_ptr(), rows, cols, code, dz.data_ptr(),
-                                               db.data_ptr(), ws.data_ptr(), ws.numel(), st), "esa_mish_bwd_colsum")
-        else:
-            _lib.check(lib.esa_mish_bwd(z.data_ptr(), g.data_ptr(), z.numel(), code, dz.data_ptr(), st),
-                       "esa_mish_bwd")
-            if bdt is not None and ctx.needs_input_grad[2]:
-                db = column_sum(dz)
+        _lib.check(_lib.load().esa_mish_bwd(z.data_ptr(), g.data_ptr(), z.numel(), _DTYPES[z.dtype], dz.data_ptr(),
+                                            _lib.stream_of(z)), "esa_mish_bwd")
         dx = dz.mm(w) if ctx.needs_input_grad[0] else None
-        dw = weight_grad(dz, x).to(wdt) if ctx.needs_input_grad[1] else None
-        return dx, dw, None if db is None else db.to(bdt)
+        ((dw, db),) = weight_bias_grads([(dz, x)], [ctx.needs_input_grad[1]],
+                                        [bdt is not None and ctx.needs_input_grad[2]])
+        return dx, None if dw is None else dw.to(wdt), None if db is None else db.to(bdt)
 
 
 def linear_mish(x: torch.Tensor, layer: nn.Linear) -> torch.Tensor:

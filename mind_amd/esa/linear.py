@@ -1,13 +1,14 @@
-"""nn.Linear for the packed ESA blocks, with a split-K weight gradient.
+"""nn.Linear for the packed ESA blocks, with weight and bias gradients of their own.
 
 On packed edge tokens a Linear's weight gradient dW = g^T x reduces over all
 T tokens of the batch (T = 131,072 in the encoder-stack benchmark) into a
 small [out, in] matrix: one GEMM with K = T has only a few dozen output tiles
-for 256 CUs.  ``linear`` computes it instead as S batched GEMMs over token
-chunks (``torch.bmm`` with fp32 outputs) and sums the S fp32 partials, so the
-reduction fills the chip and is rounded to the weight's dtype once, as the
-single GEMM's fp32 accumulator is.  Forward (F.linear) and dx = g W are
-unchanged; the bias gradient is a deterministic column sum (esa_column_sum).
+for 256 CUs.  ``weight_bias_grads`` cuts it over the tokens in one kernel that
+also sums the bias gradient's columns (esa_weight_grad: two launches for up to
+three Linears that share their rows), in fp32 and rounded to the weight's
+dtype once, as the single GEMM's fp32 accumulator is.  Shapes and dtypes
+outside the kernel's run as S batched GEMMs over token chunks (``weight_grad``)
+and a column sum.  Forward (F.linear) and dx = g W are unchanged.
 Under autocast the inputs are cast as autocast casts F.linear's (x, weight
 and bias to the autocast dtype); the autograd functions take the parameters
 in their own dtype and cast them inside, so the fp32 weight and bias
@@ -45,7 +46,8 @@ def split_count(tokens: int, out_features: int, in_features: int) -> int:
 
 
 def weight_grad(g: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
-    """g^T x for g [T, out], x [T, in] (same dtype) in fp32, by split_count(T, out, in) token chunks."""
+    """g^T x for g [T, out], x [T, in] (same dtype) in fp32, by split_count(T, out, in) token chunks: the shapes
+    and dtypes that esa_weight_grad does not take."""
     t, o = g.shape
     i = x.shape[1]
     s = split_count(t, o, i)
@@ -83,10 +85,63 @@ def column_sum(g: torch.Tensor) -> torch.Tensor:
 
 
 _MAX_LINEAR_OUT = 3
+_MAX_FEATURES = 16384
+
+
+def _wgrad_ok(pairs) -> bool:
+    """Whether esa_weight_grad takes every (g, x): fp32 or bf16 device tensors of one dtype, [rows, features]
+    contiguous with the same rows >= 1, feature counts multiples of 8 (bf16) or 4 (fp32), 16-byte aligned."""
+    g0 = pairs[0][0]
+    code = _CODES.get(g0.dtype)
+    if code is None or not g0.is_cuda or g0.shape[0] < 1:
+        return False
+    unit = 8 if code == _lib.ESA_BF16 else 4
+    for g, x in pairs:
+        for t in (g, x):
+            if (t.dtype != g0.dtype or t.device != g0.device or t.dim() != 2 or t.shape[0] != g0.shape[0]
+                    or t.shape[1] < unit or t.shape[1] % unit or t.shape[1] > _MAX_FEATURES
+                    or not t.is_contiguous() or not _aligned(t)):
+                return False
+    return True
+
+
+def esa_weight_grad(pairs, bias) -> list[tuple[torch.Tensor, torch.Tensor | None]]:
+    """[(g^T x, g.sum(0) or None)] in fp32 for 1-3 (g, x) over the same rows (the shapes ``_wgrad_ok`` accepts)
+    through esa_weight_grad; ``bias`` says per pair whether the column sums are wanted."""
+    n, (rows, dev) = len(pairs), (pairs[0][0].shape[0], pairs[0][0].device)
+    code = _CODES[pairs[0][0].dtype]
+    vp, ci = ctypes.c_void_p * n, ctypes.c_int * n
+    o, i = ci(*[g.shape[1] for g, _ in pairs]), ci(*[x.shape[1] for _, x in pairs])
+    lib = _lib.load()
+    nbytes = ctypes.c_size_t(0)
+    _lib.check(lib.esa_weight_grad_workspace_size(rows, n, o, i, code, ctypes.byref(nbytes)),
+               "esa_weight_grad_workspace_size")
+    ws = torch.empty(max(int(nbytes.value), 16), dtype=torch.uint8, device=dev)
+    dw = [torch.empty(g.shape[1], x.shape[1], dtype=torch.float32, device=dev) for g, x in pairs]
+    db = [torch.empty(g.shape[1], dtype=torch.float32, device=dev) if b else None for (g, _), b in zip(pairs, bias)]
+    _lib.check(lib.esa_weight_grad(rows, n, vp(*[g.data_ptr() for g, _ in pairs]), vp(*[x.data_ptr() for _, x in pairs]),
+                                   o, i, code, vp(*[w.data_ptr() for w in dw]), vp(*[_lib.ptr(b) for b in db]),
+                                   ws.data_ptr(), ws.numel(), _lib.stream_of(pairs[0][0])), "esa_weight_grad")
+    return list(zip(dw, db))
 
 
 def _aligned(t: torch.Tensor) -> bool:
     return t.data_ptr() % 16 == 0
+
+
+def weight_bias_grads(pairs, need_w, need_b) -> list[tuple[torch.Tensor | None, torch.Tensor | None]]:
+    """[(g^T x, g.sum(0))] in fp32 for 1-3 (g, x) over the same rows, None where ``need_w`` / ``need_b`` says a
+    gradient is not wanted: one call of esa_weight_grad where it takes them, else ``weight_grad`` and
+    ``column_sum`` one by one (also where the gradients are to be differentiated again: ``weight_grad`` is made
+    of torch operations)."""
+    wanted = [p for p, w in zip(pairs, need_w) if w]
+    again = torch.is_grad_enabled() and any(t.requires_grad for p in wanted for t in p)
+    if wanted and not again and _wgrad_ok(wanted):
+        got = iter(esa_weight_grad(wanted, [b for w, b in zip(need_w, need_b) if w]))
+        return [next(got) if w else (None, column_sum(g) if b else None)
+                for (g, _), w, b in zip(pairs, need_w, need_b)]
+    return [(weight_grad(g, x) if w else None, column_sum(g) if b else None)
+            for (g, x), w, b in zip(pairs, need_w, need_b)]
 
 
 def _f32_linear_ok(x: torch.Tensor, pairs) -> bool:
@@ -208,9 +263,9 @@ class _Linear(torch.autograd.Function):
         wdt, bdt = ctx.dtypes
         g = g.contiguous()
         dx = g.mm(w) if ctx.needs_input_grad[0] else None
-        dw = weight_grad(g, x).to(wdt) if ctx.needs_input_grad[1] else None
-        db = column_sum(g).to(bdt) if bdt is not None and ctx.needs_input_grad[2] else None
-        return dx, dw, db
+        ((dw, db),) = weight_bias_grads([(g, x)], [ctx.needs_input_grad[1]],
+                                        [bdt is not None and ctx.needs_input_grad[2]])
+        return dx, None if dw is None else dw.to(wdt), None if db is None else db.to(bdt)
 
 
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
@@ -264,12 +319,18 @@ class _QKV(torch.autograd.Function):
             if ctx.needs_input_grad[1]:
                 dxk = gk.mm(wk)
                 dxk.addmm_(gv, wv)
+        pairs = [(gq, xq), (gk, xk), (gv, xk)]
+        need_w = [ctx.needs_input_grad[2 + 2 * i] for i in range(3)]
+        need_b = [ctx.params[2 * i + 1] is not None and ctx.needs_input_grad[3 + 2 * i] for i in range(3)]
+        if ctx.same:
+            parts = weight_bias_grads(pairs, need_w, need_b)
+        else:   # the seeds' rows are not the keys'
+            parts = (weight_bias_grads(pairs[:1], need_w[:1], need_b[:1])
+                     + weight_bias_grads(pairs[1:], need_w[1:], need_b[1:]))
         grads = [dxq, dxk]
-        for i, (g, x) in enumerate(((gq, xq), (gk, xk), (gv, xk))):
-            wdt, bdt = ctx.params[2 * i], ctx.params[2 * i + 1]
-            dw = weight_grad(g, x).to(wdt) if ctx.needs_input_grad[2 + 2 * i] else None
-            db = column_sum(g).to(bdt) if bdt is not None and ctx.needs_input_grad[3 + 2 * i] else None
-            grads += [dw, db]
+        for i, (dw, db) in enumerate(parts):
+            grads += [None if dw is None else dw.to(ctx.params[2 * i]),
+                      None if db is None else db.to(ctx.params[2 * i + 1])]
         return tuple(grads)
 
 
