@@ -166,7 +166,7 @@ def ptr(t: torch.Tensor | None) -> int | None:
 
 
 def stream_of(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(t.get_device())   # current_stream(t.device).cuda_stream, without the object
 
 
 def version() -> str:

@@ -16,6 +16,7 @@ from typing import Optional
 import torch
 
 from . import _lib
+from .esa.eager import call
 
 _DTYPES = {torch.float32: _lib.ESA_F32, torch.bfloat16: _lib.ESA_BF16}
 
@@ -249,7 +250,7 @@ def scatter_add(src: torch.Tensor, index: torch.Tensor, dim: int = 0, dim_size: 
         csr = CSR.build(index, dim_size)
     elif csr.num_nodes != dim_size:
         raise ValueError("csr was built for another dim_size")
-    return _ScatterAdd.apply(src, index, dim_size, csr)
+    return call(_ScatterAdd, src, index, dim_size, csr)
 
 
 def segment_minmax_csr(y: torch.Tensor, indptr: torch.Tensor, perm: torch.Tensor | None = None,
@@ -315,7 +316,7 @@ def _scatter_minmax(src, index, dim, out, dim_size, csr, maximum, name):
         csr = CSR.build(index, dim_size)
     elif csr.num_nodes != dim_size:
         raise ValueError("csr was built for another dim_size")
-    return _ScatterMinMax.apply(src, dim_size, csr, maximum)
+    return call(_ScatterMinMax, src, dim_size, csr, maximum)
 
 
 def scatter_min(src: torch.Tensor, index: torch.Tensor, dim: int = 0, out: torch.Tensor | None = None,
@@ -411,8 +412,8 @@ def edge_token_linear(x: torch.Tensor, src: torch.Tensor, dst: torch.Tensor, wei
         raise ValueError("src and dst must be 1-D and of equal length")
     if edge_attr is not None and (edge_attr.dim() != 2 or edge_attr.shape[0] != src.shape[0]):
         raise ValueError("edge_attr must be [E, F_e]")
-    return _EdgeTokenLinear.apply(x, weight, bias, src, dst, src_csr, dst_csr,
-                                  None if edge_attr is None else edge_attr.contiguous())
+    return call(_EdgeTokenLinear, x, weight, bias, src, dst, src_csr, dst_csr,
+                None if edge_attr is None else edge_attr.contiguous())
 
 
 class EdgeTokenLinear(torch.nn.Module):

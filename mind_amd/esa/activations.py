@@ -23,34 +23,56 @@ from torch import nn
 from torch.nn import functional as F
 
 from .. import _lib
+from .eager import call
 
 _DTYPES = {torch.float32: _lib.ESA_F32, torch.bfloat16: _lib.ESA_BF16}
+
+
+def mish_forward(z, residual=None):
+    """esa_mish_fwd: residual + mish(z) of contiguous tensors of one dtype (mish(z) without a residual)."""
+    y = torch.empty_like(z)
+    _lib.check(_lib.load().esa_mish_fwd(z.data_ptr(), _lib.ptr(residual), z.numel(), _DTYPES[z.dtype], y.data_ptr(),
+                                        _lib.stream_of(z)), "esa_mish_fwd")
+    return y
+
+
+def mish_backward(z, g):
+    """esa_mish_bwd: g mish'(z), contiguous tensors of one dtype."""
+    dz = torch.empty_like(z)
+    _lib.check(_lib.load().esa_mish_bwd(z.data_ptr(), g.data_ptr(), z.numel(), _DTYPES[z.dtype], dz.data_ptr(),
+                                        _lib.stream_of(z)), "esa_mish_bwd")
+    return dz
+
+
+def mab_residual_forward(z, o, x):
+    """esa_mab_residual_fwd: x + r(o + mish(z)), x and the result fp32, r() the rounding to o's dtype."""
+    y = torch.empty(x.shape, dtype=torch.float32, device=x.device)
+    _lib.check(_lib.load().esa_mab_residual_fwd(z.data_ptr(), o.data_ptr(), x.data_ptr(), z.numel(), _DTYPES[o.dtype],
+                                                y.data_ptr(), _lib.stream_of(o)), "esa_mab_residual_fwd")
+    return y
+
+
+def mab_residual_backward(z, g):
+    """esa_mab_residual_bwd: (g mish'(z), r(g)) of the fp32 gradient g, in z's dtype."""
+    dz, g_o = torch.empty_like(z), torch.empty_like(z)
+    _lib.check(_lib.load().esa_mab_residual_bwd(z.data_ptr(), g.data_ptr(), z.numel(), _DTYPES[z.dtype], dz.data_ptr(),
+                                                g_o.data_ptr(), _lib.stream_of(z)), "esa_mab_residual_bwd")
+    return dz, g_o
 
 
 class _Mish(torch.autograd.Function):
     @staticmethod
     def forward(ctx, z, residual):
-        code = _DTYPES[z.dtype]
         z = z.contiguous()
-        if residual is not None:
-            residual = residual.contiguous()
-        y = torch.empty_like(z)
-        rc = _lib.load().esa_mish_fwd(z.data_ptr(), _lib.ptr(residual), z.numel(), code, y.data_ptr(),
-                                      _lib.stream_of(z))
-        _lib.check(rc, "esa_mish_fwd")
         ctx.save_for_backward(z)
         ctx.has_residual = residual is not None
-        return y
+        return mish_forward(z, None if residual is None else residual.contiguous())
 
     @staticmethod
     def backward(ctx, g):
         (z,) = ctx.saved_tensors
         g = g.to(z.dtype).contiguous()
-        dz = torch.empty_like(z)
-        rc = _lib.load().esa_mish_bwd(z.data_ptr(), g.data_ptr(), z.numel(), _DTYPES[z.dtype], dz.data_ptr(),
-                                      _lib.stream_of(z))
-        _lib.check(rc, "esa_mish_bwd")
-        return dz, (g if ctx.has_residual else None)
+        return mish_backward(z, g), (g if ctx.has_residual else None)
 
 
 def mish(z: torch.Tensor, residual: torch.Tensor | None = None) -> torch.Tensor:
@@ -61,8 +83,8 @@ def mish(z: torch.Tensor, residual: torch.Tensor | None = None) -> torch.Tensor:
         raise TypeError(f"mish: unsupported dtype {z.dtype}; use float32 or bfloat16")
     if residual is not None and (residual.dtype != z.dtype or residual.shape != z.shape):
         # Mixed precision or broadcasting: torch's promotion rules for the add.
-        return residual + _Mish.apply(z, None)
-    return _Mish.apply(z, residual)
+        return residual + call(_Mish, z, None)
+    return call(_Mish, z, residual)
 
 
 class _MabEpilogue(torch.autograd.Function):
@@ -77,15 +99,7 @@ class _MabEpilogue(torch.autograd.Function):
         ctx.dtypes = (weight.dtype, None if bias is None else bias.dtype)   # the gradients are returned in these
         weight, bias = cast_param(weight, o.dtype), cast_param(bias, o.dtype)
         (z,) = linear_fwd(o, [(weight, bias)])
-        lib, st, code = _lib.load(), _lib.stream_of(o), _DTYPES[o.dtype]
-        if x is None:
-            y = torch.empty_like(z)
-            _lib.check(lib.esa_mish_fwd(z.data_ptr(), o.data_ptr(), z.numel(), code, y.data_ptr(), st),
-                       "esa_mish_fwd")
-        else:
-            y = torch.empty(x.shape, dtype=torch.float32, device=x.device)
-            _lib.check(lib.esa_mab_residual_fwd(z.data_ptr(), o.data_ptr(), x.data_ptr(), z.numel(), code,
-                                                y.data_ptr(), st), "esa_mab_residual_fwd")
+        y = mish_forward(z, o) if x is None else mab_residual_forward(z, o, x)
         ctx.save_for_backward(o, weight, z)
         ctx.has_x = x is not None
         return y
@@ -94,17 +108,12 @@ class _MabEpilogue(torch.autograd.Function):
     def backward(ctx, g):
         from .linear import weight_bias_grads   # deferred: linear.py is a sibling with its own imports
         o, weight, z = ctx.saved_tensors
-        lib, st, code = _lib.load(), _lib.stream_of(z), _DTYPES[z.dtype]
-        dz = torch.empty_like(z)
         if ctx.has_x:
             g = g.float().contiguous()
-            g_o = torch.empty_like(z)
-            _lib.check(lib.esa_mab_residual_bwd(z.data_ptr(), g.data_ptr(), z.numel(), code, dz.data_ptr(),
-                                                g_o.data_ptr(), st), "esa_mab_residual_bwd")
+            dz, g_o = mab_residual_backward(z, g)
         else:
             g_o = g.to(z.dtype).contiguous()
-            _lib.check(lib.esa_mish_bwd(z.data_ptr(), g_o.data_ptr(), z.numel(), code, dz.data_ptr(), st),
-                       "esa_mish_bwd")
+            dz = mish_backward(z, g_o)
         wdt, bdt = ctx.dtypes
         do = torch.addmm(g_o, dz, weight) if ctx.needs_input_grad[0] else None
         ((dw, db),) = weight_bias_grads([(dz, o)], [ctx.needs_input_grad[1]],
@@ -127,8 +136,8 @@ def mab_epilogue(o: torch.Tensor, fc_o: nn.Linear, residual: torch.Tensor | None
         return y if residual is None else residual + y
     o = o.to(dt).contiguous()
     if residual is not None and (residual.dtype != torch.float32 or residual.shape != o.shape):
-        return residual + _MabEpilogue.apply(o, w, b, None)
-    return _MabEpilogue.apply(o, w, b, None if residual is None else residual.contiguous())
+        return residual + call(_MabEpilogue, o, w, b, None)
+    return call(_MabEpilogue, o, w, b, None if residual is None else residual.contiguous())
 
 
 class _LinearMish(torch.autograd.Function):
@@ -143,11 +152,8 @@ class _LinearMish(torch.autograd.Function):
         ctx.dtypes = (weight.dtype, None if bias is None else bias.dtype)
         w, b = cast_param(weight, x.dtype), cast_param(bias, x.dtype)
         (z,) = linear_fwd(x, [(w, b)])
-        y = torch.empty_like(z)
-        _lib.check(_lib.load().esa_mish_fwd(z.data_ptr(), None, z.numel(), _DTYPES[z.dtype], y.data_ptr(),
-                                            _lib.stream_of(z)), "esa_mish_fwd")
         ctx.save_for_backward(x, w, z)
-        return y
+        return mish_forward(z)
 
     @staticmethod
     def backward(ctx, g):
@@ -155,9 +161,7 @@ class _LinearMish(torch.autograd.Function):
         x, w, z = ctx.saved_tensors
         wdt, bdt = ctx.dtypes
         g = g.to(z.dtype).contiguous()
-        dz = torch.empty_like(z)
-        _lib.check(_lib.load().esa_mish_bwd(z.data_ptr(), g.data_ptr(), z.numel(), _DTYPES[z.dtype], dz.data_ptr(),
-                                            _lib.stream_of(z)), "esa_mish_bwd")
+        dz = mish_backward(z, g)
         dx = dz.mm(w) if ctx.needs_input_grad[0] else None
         ((dw, db),) = weight_bias_grads([(dz, x)], [ctx.needs_input_grad[1]],
                                         [bdt is not None and ctx.needs_input_grad[2]])
@@ -174,7 +178,7 @@ def linear_mish(x: torch.Tensor, layer: nn.Linear) -> torch.Tensor:
         return mish(linear(x, layer.weight, layer.bias))
     x = x.to(dt)
     lead = x.shape[:-1]
-    y = _LinearMish.apply(x.reshape(-1, x.shape[-1]).contiguous(), layer.weight, layer.bias)
+    y = call(_LinearMish, x.reshape(-1, x.shape[-1]).contiguous(), layer.weight, layer.bias)
     return y.view(*lead, layer.weight.shape[0])
 
 

@@ -17,6 +17,7 @@ from typing import Optional
 import torch
 
 from .. import _lib
+from .eager import call, plain, records
 
 HEAD_DIMS = (16, 24, 32, 64)   # head dims the kernels take
 _SEED_MASK = (1 << 63) - 1
@@ -352,6 +353,29 @@ def _varlen_backward(ctx, dout, _dlse):
 torch.library.register_autograd("esa_hip::varlen_attn_fwd", _varlen_backward, setup_context=_varlen_setup)
 
 
+class _VarlenAttention(torch.autograd.Function):
+    """The forward operator's autograd in plain eager execution: the same calls without the operators' dispatch
+    (fwd + bwd of 1,000 tokens 138 -> 60 us of host time) and without a gradient materialised for the lse."""
+
+    @staticmethod
+    def forward(ctx, *args):
+        out, lse = attn_fwd(*args)
+        ctx.set_materialize_grads(False)
+        _varlen_setup(ctx, args, (out, lse))
+        return out, lse
+
+    @staticmethod
+    def backward(ctx, dout, _dlse):
+        q, k, v, out, lse, cu_q, cu_k, *masks = ctx.saved_tensors
+        if dout is None:   # only the lse was used, whose gradient is not defined: zeros, as the operator gives
+            return (torch.zeros_like(q), torch.zeros_like(k), torch.zeros_like(v)) + (None,) * 13
+        if torch.is_grad_enabled() or not plain(dout, q):   # to be differentiated again, or seen as an operation
+            return _varlen_backward(ctx, dout, _dlse)
+        max_q, max_k, scale, dropout_p, dropout_seed = ctx.meta
+        return attn_bwd(dout.contiguous(), q, k, v, out, lse, cu_q, cu_k, max_q, max_k, scale, *masks, dropout_p,
+                        dropout_seed) + (None,) * 13
+
+
 def varlen_attention(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, dropout_p=0.0,
                      softmax_scale=None, causal=False, edge_src=None, edge_dst=None, return_lse=False,
                      adj_indptr=None, adj_indices=None, edge_plan=None, adj_plan=None, dropout_seed=None):
@@ -387,10 +411,14 @@ def varlen_attention(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seql
         raise ValueError("edge_src and edge_dst must be given together")
     if (adj_indptr is None) != (adj_indices is None):
         raise ValueError("adj_indptr and adj_indices must be given together")
-    out, lse = torch.ops.esa_hip.varlen_attn_fwd(q, k, v, cu_seqlens_q, cu_seqlens_k, int(max_seqlen_q),
-                                                 int(max_seqlen_k), float(softmax_scale), edge_src, edge_dst,
-                                                 adj_indptr, adj_indices, edge_plan, adj_plan, dropout_p,
-                                                 int(dropout_seed or 0) & _SEED_MASK)
+    args = (q, k, v, cu_seqlens_q, cu_seqlens_k, int(max_seqlen_q), int(max_seqlen_k), float(softmax_scale), edge_src,
+            edge_dst, adj_indptr, adj_indices, edge_plan, adj_plan, dropout_p, int(dropout_seed or 0) & _SEED_MASK)
+    if not plain(*args):
+        out, lse = torch.ops.esa_hip.varlen_attn_fwd(*args)
+    elif records(q, k, v):
+        out, lse = _VarlenAttention.apply(*args)
+    else:
+        out, lse = attn_fwd(*args)
     return (out, lse) if return_lse else out
 
 
@@ -402,18 +430,38 @@ def _pma_workspace(device, batch, k_seeds, total_k, heads, head_dim, dtype, back
     return torch.empty(max(int(n.value), 256), dtype=torch.uint8, device=device)
 
 
+def pma_forward(q, k, v, cu_k, max_k, scale, dropout_p, dropout_seed):
+    """esa_pma_fwd: (out [B * k, H, hd], lse) of seeds q [k, H, hd] over the sets' keys."""
+    batch, k_seeds, heads, hd = cu_k.numel() - 1, q.shape[0], q.shape[1], q.shape[2]
+    dt = _dtype_code(q)
+    out = torch.empty((batch * k_seeds, heads, hd), dtype=q.dtype, device=q.device)
+    lse = torch.empty((heads, batch * k_seeds), dtype=torch.float32, device=q.device)
+    ws = _pma_workspace(q.device, batch, k_seeds, k.shape[0], heads, hd, dt, False)
+    rc = _lib.load().esa_pma_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), cu_k.data_ptr(), batch, k_seeds,
+                                 k.shape[0], int(max_k), heads, hd, dt, float(scale), dropout_p, dropout_seed,
+                                 out.data_ptr(), lse.data_ptr(), ws.data_ptr(), ws.numel(), _lib.stream_of(q))
+    _lib.check(rc, "esa_pma_fwd")
+    return out, lse
+
+
+def pma_backward(g, q, k, v, out, lse, cu_k, max_k, scale, dropout_p, dropout_seed):
+    """esa_pma_bwd: (dq, dk, dv), dq summed over the sets; g contiguous in q's dtype."""
+    batch, k_seeds, heads, hd = cu_k.numel() - 1, q.shape[0], q.shape[1], q.shape[2]
+    dt = _dtype_code(q)
+    dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
+    ws = _pma_workspace(q.device, batch, k_seeds, k.shape[0], heads, hd, dt, True)
+    rc = _lib.load().esa_pma_bwd(g.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
+                                 lse.data_ptr(), cu_k.data_ptr(), batch, k_seeds, k.shape[0], int(max_k), heads,
+                                 hd, dt, float(scale), dropout_p, dropout_seed, dq.data_ptr(), dk.data_ptr(),
+                                 dv.data_ptr(), ws.data_ptr(), ws.numel(), _lib.stream_of(q))
+    _lib.check(rc, "esa_pma_bwd")
+    return dq, dk, dv
+
+
 class _PMAAttention(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v, cu_k, max_k, scale, dropout_p, dropout_seed):
-        batch, k_seeds, heads, hd = cu_k.numel() - 1, q.shape[0], q.shape[1], q.shape[2]
-        dt = _dtype_code(q)
-        out = torch.empty((batch * k_seeds, heads, hd), dtype=q.dtype, device=q.device)
-        lse = torch.empty((heads, batch * k_seeds), dtype=torch.float32, device=q.device)
-        ws = _pma_workspace(q.device, batch, k_seeds, k.shape[0], heads, hd, dt, False)
-        rc = _lib.load().esa_pma_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), cu_k.data_ptr(), batch, k_seeds,
-                                     k.shape[0], int(max_k), heads, hd, dt, float(scale), dropout_p, dropout_seed,
-                                     out.data_ptr(), lse.data_ptr(), ws.data_ptr(), ws.numel(), _lib.stream_of(q))
-        _lib.check(rc, "esa_pma_fwd")
+        out, lse = pma_forward(q, k, v, cu_k, max_k, scale, dropout_p, dropout_seed)
         ctx.save_for_backward(q, k, v, out, lse, cu_k)
         ctx.meta = (max_k, scale, dropout_p, dropout_seed)
         return out
@@ -421,18 +469,7 @@ class _PMAAttention(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g):
         q, k, v, out, lse, cu_k = ctx.saved_tensors
-        max_k, scale, dropout_p, dropout_seed = ctx.meta
-        batch, k_seeds, heads, hd = cu_k.numel() - 1, q.shape[0], q.shape[1], q.shape[2]
-        dt = _dtype_code(q)
-        g = g.to(q.dtype).contiguous()
-        dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-        ws = _pma_workspace(q.device, batch, k_seeds, k.shape[0], heads, hd, dt, True)
-        rc = _lib.load().esa_pma_bwd(g.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
-                                     lse.data_ptr(), cu_k.data_ptr(), batch, k_seeds, k.shape[0], int(max_k), heads,
-                                     hd, dt, float(scale), dropout_p, dropout_seed, dq.data_ptr(), dk.data_ptr(),
-                                     dv.data_ptr(), ws.data_ptr(), ws.numel(), _lib.stream_of(q))
-        _lib.check(rc, "esa_pma_bwd")
-        return dq, dk, dv, None, None, None, None, None
+        return pma_backward(g.to(q.dtype).contiguous(), q, k, v, out, lse, cu_k, *ctx.meta) + (None,) * 5
 
 
 def pma_attention(q, k, v, cu_seqlens_k, max_seqlen_k, softmax_scale=None, dropout_p=0.0, dropout_seed=None):
@@ -453,8 +490,8 @@ def pma_attention(q, k, v, cu_seqlens_k, max_seqlen_k, softmax_scale=None, dropo
     dropout_p = _check_dropout(dropout_p)
     if dropout_p > 0.0 and dropout_seed is None:
         dropout_seed = draw_dropout_seed()
-    return _PMAAttention.apply(q, k, v, cu_seqlens_k, max_seqlen_k, float(softmax_scale), dropout_p,
-                               int(dropout_seed or 0) & _SEED_MASK)
+    return call(_PMAAttention, q, k, v, cu_seqlens_k, max_seqlen_k, float(softmax_scale), dropout_p,
+                int(dropout_seed or 0) & _SEED_MASK)
 
 
 def edge_mask_dense(edge_src, edge_dst, cu_seqlens, max_items):

@@ -1,0 +1,283 @@
+"""The packed pre-norm blocks as one autograd function each.
+
+``sab_block`` and ``pma_block`` run the computation of
+``masked_layers._sab_forward_packed`` / ``_pma_forward_packed`` (the
+reference's SABComplete.forward and PMAComplete.forward,
+esa/masked_layers.py:418-483, 574-621) on the same kernels, in the same order,
+but record one autograd node for a block instead of seven, and call the
+kernels without the layers between.  A small batch's step is bound by the
+host: a block's forward and backward issue about 35 launches, and an autograd
+function around each costs more than the launch (64 small molecules in fp32,
+three blocks: 3.3 -> 2.2 ms per train step).  The gradients of a block's
+shared inputs are added inside its GEMMs and kernels, with at most the
+roundings of the separate nodes.
+
+They take the calls that nothing else has to see as single operations
+(``eager.plain``), over the dtypes the kernels compute in: bf16 autocast with
+fp32 parameters, or fp32 throughout.  Everything else stays with the separate
+functions, which also serve a backward that is differentiated again.
+"""
+from __future__ import annotations
+
+import math
+
+import torch
+from torch import nn
+
+from . import attention
+from .activations import Mish, mab_residual_backward, mab_residual_forward, mish_backward, mish_forward
+from .attention import HEAD_DIMS, attn_bwd, attn_fwd, pma_backward, pma_forward
+from .eager import call, plain
+from .layer_norm import f32_values, ln_backward, ln_forward, supported
+from .linear import cast_param, hookless, linear_fwd, weight_bias_grads
+from .mlp_utils import SmallMLP
+
+
+def _mlp_layers(blk) -> list[nn.Linear] | None:
+    """The Linears of the block's MLP when it is Linear (-> Mish -> Linear)* without hooks, [] without an MLP, None
+    for any other."""
+    if not blk.use_mlp:
+        return []
+    glob = nn.modules.module
+    if (type(blk.mlp) is not SmallMLP or not hookless(blk.mlp) or blk.mlp._backward_hooks
+            or blk.mlp._backward_pre_hooks or glob._global_forward_hooks or glob._global_forward_pre_hooks
+            or glob._global_backward_hooks or glob._global_backward_pre_hooks):
+        return None
+    layers = list(blk.mlp.mlp)
+    for i, m in enumerate(layers):
+        if type(m) not in ((nn.Linear,) if i % 2 == 0 else (Mish, nn.Mish)) or not hookless(m):
+            return None
+    return layers[::2] if len(layers) % 2 else None
+
+
+def _compute_dtype(x: torch.Tensor, params):
+    """The dtype the block's GEMMs run in: bf16 under bf16 autocast, fp32 where everything is fp32; None where the
+    block is not taken."""
+    if not x.is_cuda or x.dtype != torch.float32 or x.shape[0] == 0:
+        return None
+    if any(p is not None and p.dtype != torch.float32 for p in params):
+        return None
+    if not torch.is_autocast_enabled("cuda"):
+        return torch.float32
+    return torch.bfloat16 if torch.get_autocast_dtype("cuda") == torch.bfloat16 else None
+
+
+def _block_args(blk, mab, mlp):
+    """The block's parameters in the functions' order."""
+    args = [blk.norm.ln.weight, blk.norm.ln.bias]
+    for fc in (mab.fc_q, mab.fc_k, mab.fc_v, mab.fc_o):
+        args += (fc.weight, fc.bias)
+    if mlp:
+        args += (blk.norm_mlp.ln.weight, blk.norm_mlp.ln.bias)
+    for fc in mlp:
+        args += (fc.weight, fc.bias)
+    return args
+
+
+class _Setup:
+    """What a block's function needs besides tensors."""
+
+    def __init__(self, blk, tokens, mab, mlp, dt, dropout_p, again):
+        self.eps = (blk.norm.ln.eps, blk.norm_mlp.ln.eps)
+        self.heads, self.max_items, self.cu = mab.num_heads, tokens.max_items, tokens.cu_seqlens
+        self.dt, self.amp, self.n_mlp = dt, dt != torch.float32, len(mlp)
+        self.dropout = (dropout_p, attention.draw_dropout_seed() if dropout_p > 0.0 else 0)
+        self.again = again   # (x, seed) -> the block's output through the separate functions
+        self.mask = {}
+
+
+def _rebuilt(setup, inputs, g, needs):
+    """The inputs' gradients by the separate functions, for a backward that is itself differentiated."""
+    with torch.enable_grad(), torch.autocast("cuda", setup.dt if setup.amp else None, enabled=setup.amp):
+        out = setup.again(inputs[0], setup.dropout[1])
+        wanted = [t for t, n in zip(inputs, needs) if n]
+        got = iter(torch.autograd.grad(out, wanted, g, create_graph=True, allow_unused=True))
+    return tuple(next(got) if n else None for n in needs)
+
+
+def _norm(setup, x, w, b, eps, full):
+    """(ln(x) in fp32 or None, the rows its Linear takes, statistics)."""
+    if setup.amp:
+        return ln_forward(x, f32_values(w), f32_values(b), eps, torch.float32, full, True)
+    y, _, stats = ln_forward(x, f32_values(w), f32_values(b), eps, x.dtype, True, False)
+    return y, y, stats
+
+
+def _mlp_forward(x, params):
+    """Linear (-> Mish -> Linear)*: (output, [the tensors _mlp_backward takes: input, weight and, before a Mish, z])."""
+    saved = []
+    for i in range(0, len(params), 2):
+        w, b = cast_param(params[i], x.dtype), cast_param(params[i + 1], x.dtype)
+        (z,) = linear_fwd(x, [(w, b)])
+        saved += (x, w)
+        if i + 2 < len(params):
+            saved.append(z)
+            x = mish_forward(z)
+    return z, saved
+
+
+def _mlp_backward(g, saved, needs):
+    """(dx, the parameters' gradients) for the output gradient g in the compute dtype."""
+    grads = [None] * len(needs)
+    layers = [saved[i:i + 3] for i in range(0, len(saved), 3)]
+    for i in range(len(layers) - 1, -1, -1):
+        x, w = layers[i][:2]
+        if len(layers[i]) == 3:
+            g = mish_backward(layers[i][2], g)
+        ((grads[2 * i], grads[2 * i + 1]),) = weight_bias_grads([(g, x)], needs[2 * i:2 * i + 1],
+                                                                needs[2 * i + 1:2 * i + 2])
+        g = g.mm(w)
+    return g, grads
+
+
+class _SabBlock(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, setup, x, *params):
+        ln_w, ln_b, wq, bq, wk, bk, wv, bv, wo, bo = params[:10]
+        t, d, h = x.shape[0], x.shape[1], setup.heads
+        x1, xm, stats = _norm(setup, x, ln_w, ln_b, setup.eps[0], True)
+        weights = [cast_param(p, setup.dt) for p in (wq, wk, wv, wo)]
+        biases = [cast_param(p, setup.dt) for p in (bq, bk, bv, bo)]
+        q, k, v = (y.view(t, h, d // h) for y in linear_fwd(xm, list(zip(weights[:3], biases[:3]))))
+        cu, n, (p, seed) = setup.cu, setup.max_items, setup.dropout
+        o, lse = attn_fwd(q, k, v, cu, cu, n, n, 1.0 / math.sqrt(d // h), dropout_p=p, dropout_seed=seed, **setup.mask)
+        (z,) = linear_fwd(o.view(t, d), [(weights[3], biases[3])])
+        x2 = mab_residual_forward(z, o, x1)
+        keep = [x, f32_values(ln_w), stats, xm, q, k, v, o, lse, z] + weights
+        out = x2
+        if setup.n_mlp:
+            ln_w2, ln_b2 = params[10:12]
+            _, ym, stats2 = _norm(setup, x2, ln_w2, ln_b2, setup.eps[1], False)
+            y, saved = _mlp_forward(ym, params[12:])
+            out = y + x2
+            keep += [x2, f32_values(ln_w2), stats2] + saved
+        ctx.setup, ctx.n_keep, ctx.mask_keys = setup, len(keep), list(setup.mask)
+        ctx.save_for_backward(*keep, cu, *setup.mask.values(), *params)
+        return out
+
+    @staticmethod
+    def backward(ctx, g):
+        setup, needs, tensors = ctx.setup, ctx.needs_input_grad[1:], ctx.saved_tensors
+        if torch.is_grad_enabled():
+            n = ctx.n_keep + 1 + len(ctx.mask_keys)
+            return (None,) + _rebuilt(setup, (tensors[0],) + tensors[n:], g, needs)
+        x, ln_w, stats, xm, q, k, v, o, lse, z, wq, wk, wv, wo = tensors[:14]
+        cu, mask = tensors[ctx.n_keep], dict(zip(ctx.mask_keys, tensors[ctx.n_keep + 1:]))
+        t, d = x.shape
+        g = g.contiguous()
+        mlp_grads = ()
+        if setup.n_mlp:
+            x2, ln_w2, stats2 = tensors[14:17]
+            dy, mlp_grads = _mlp_backward(g.to(setup.dt), tensors[17:ctx.n_keep], needs[13:])
+            g, dw, db = ln_backward(x2, ln_w2, stats2, None if setup.amp else dy, dy if setup.amp else None, g,
+                                    needs[11], needs[12])
+            mlp_grads = (dw, db, *mlp_grads)
+        dz, g_o = mab_residual_backward(z, g)
+        do = torch.addmm(g_o, dz, wo).view_as(o)
+        grads_o = weight_bias_grads([(dz, o.view(t, d))], needs[9:10], needs[10:11])
+        n, (p, seed) = setup.max_items, setup.dropout
+        gq, gk, gv = (y.view(t, d) for y in attn_bwd(do, q, k, v, o, lse, cu, cu, n, n, 1.0 / math.sqrt(d // setup.heads),
+                                                     dropout_p=p, dropout_seed=seed, **mask))
+        # fp32: the norm's one output feeds the projections and the residual, whose gradient g starts the sum
+        dxm = gq.mm(wq) if setup.amp else torch.addmm(g, gq, wq)
+        dxm.addmm_(gk, wk)
+        dxm.addmm_(gv, wv)
+        grads = weight_bias_grads([(gq, xm), (gk, xm), (gv, xm)], needs[3:9:2], needs[4:9:2])
+        dx, dw, db = ln_backward(x, ln_w, stats, g if setup.amp else dxm, dxm if setup.amp else None, None, needs[1],
+                                 needs[2])
+        return (None, dx, dw, db, *(y for pair in grads + grads_o for y in pair), *mlp_grads)
+
+
+def sab_block(blk, x: torch.Tensor, tokens, masked: bool, attn_p: float, again) -> torch.Tensor | None:
+    """The SABComplete block ``blk`` on packed tokens x [T, D], or None where this path does not take the call.
+    ``again(x, seed)`` computes the same through the separate functions."""
+    mab, ln = blk.sab.mab, blk.norm.ln
+    mlp = _mlp_layers(blk)
+    if mlp is None or blk.residual_dropout > 0 or x.dim() != 2 or mab.dim_V != x.shape[1]:
+        return None
+    d, h = x.shape[1], mab.num_heads
+    params = _block_args(blk, mab, mlp)
+    dt = _compute_dtype(x, params)
+    if (dt is None or d % h or d // h not in HEAD_DIMS or not supported(x, ln) or not supported(x, blk.norm_mlp.ln)
+            or not plain(x, *params)):
+        return None
+    setup = _Setup(blk, tokens, mab, mlp, dt, attn_p, again)
+    if masked:
+        setup.mask = tokens.kernel_mask(padded=False)
+    return call(_SabBlock, setup, x.contiguous(), *params)
+
+
+class _PmaBlock(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, setup, x, seeds, *params):
+        ln_w, ln_b, wq, bq, wk, bk, wv, bv, wo, bo = params[:10]
+        (k_seeds, d), h = seeds.shape[1:], setup.heads
+        _, xm, stats = _norm(setup, x, ln_w, ln_b, setup.eps[0], False)
+        s = cast_param(seeds, setup.dt).reshape(k_seeds, d)
+        weights = [cast_param(p, setup.dt) for p in (wq, wk, wv, wo)]
+        biases = [cast_param(p, setup.dt) for p in (bq, bk, bv, bo)]
+        (q,) = linear_fwd(s, [(weights[0], biases[0])])
+        k, v = linear_fwd(xm, list(zip(weights[1:3], biases[1:3])))
+        q, k, v = (y.view(-1, h, d // h) for y in (q, k, v))
+        o, lse = pma_forward(q, k, v, setup.cu, setup.max_items, 1.0 / math.sqrt(d // h), *setup.dropout)
+        (z,) = linear_fwd(o.view(-1, d), [(weights[3], biases[3])])
+        x2 = mish_forward(z, o.view(-1, d))
+        keep = [x, f32_values(ln_w), stats, xm, s, q, k, v, o, lse, z] + weights
+        out = x2
+        if setup.n_mlp:
+            ln_w2, ln_b2 = params[10:12]
+            _, ym, stats2 = _norm(setup, x2, ln_w2, ln_b2, setup.eps[1], False)
+            y, saved = _mlp_forward(ym, params[12:])
+            out = y + x2
+            keep += [x2, f32_values(ln_w2), stats2] + saved
+        ctx.setup, ctx.n_keep = setup, len(keep)
+        ctx.save_for_backward(*keep, setup.cu, seeds, *params)
+        return out.view(-1, k_seeds, d)
+
+    @staticmethod
+    def backward(ctx, g):
+        setup, needs, tensors = ctx.setup, ctx.needs_input_grad[1:], ctx.saved_tensors
+        if torch.is_grad_enabled():
+            return (None,) + _rebuilt(setup, (tensors[0],) + tensors[ctx.n_keep + 1:], g, needs)
+        x, ln_w, stats, xm, s, q, k, v, o, lse, z, wq, wk, wv, wo = tensors[:15]
+        cu, seeds = tensors[ctx.n_keep:ctx.n_keep + 2]
+        d = x.shape[1]
+        g = g.contiguous().view(-1, d)
+        mlp_grads = ()
+        if setup.n_mlp:
+            x2, ln_w2, stats2 = tensors[15:18]
+            dy, mlp_grads = _mlp_backward(g, tensors[18:ctx.n_keep], needs[14:])
+            g, dw, db = ln_backward(x2, ln_w2, stats2, None if setup.amp else dy, dy if setup.amp else None, g,
+                                    needs[12], needs[13])
+            mlp_grads = (dw, db, *mlp_grads)
+        dz = mish_backward(z, g)
+        do = torch.addmm(g, dz, wo).view_as(o)
+        grads_o = weight_bias_grads([(dz, o.view(-1, d))], needs[10:11], needs[11:12])
+        gq, gk, gv = (y.view(-1, d) for y in pma_backward(do, q, k, v, o, lse, cu, setup.max_items,
+                                                          1.0 / math.sqrt(d // setup.heads), *setup.dropout))
+        dseeds = gq.mm(wq).view(seeds.shape).to(seeds.dtype) if needs[1] else None
+        dxm = gk.mm(wk)
+        dxm.addmm_(gv, wv)
+        grads = (weight_bias_grads([(gq, s)], needs[4:5], needs[5:6])
+                 + weight_bias_grads([(gk, xm), (gv, xm)], needs[6:10:2], needs[7:10:2]))
+        dx, dw, db = ln_backward(x, ln_w, stats, None if setup.amp else dxm, dxm if setup.amp else None, None, needs[2],
+                                 needs[3])
+        return (None, dx, dseeds, dw, db, *(y for pair in grads + grads_o for y in pair), *mlp_grads)
+
+
+def pma_block(blk, x: torch.Tensor, tokens, attn_p: float, again) -> torch.Tensor | None:
+    """The PMAComplete block ``blk`` over packed keys x [T, D] -> [B, k, D], or None where this path does not take
+    the call (as ``sab_block``; a seed count equal to the sets' padded size has a residual of its own)."""
+    mab, seeds, ln = blk.pma.mab, blk.pma.S, blk.norm.ln
+    mlp = _mlp_layers(blk)
+    if mlp is None or blk.residual_dropout > 0 or x.dim() != 2 or seeds.shape[1] == tokens.max_items:
+        return None
+    d, h = x.shape[1], mab.num_heads
+    if mab.dim_V != d or seeds.shape[2] != d or tokens.batch_size < 1:
+        return None
+    params = _block_args(blk, mab, mlp)
+    dt = _compute_dtype(x, [seeds] + params)
+    if (dt is None or d % h or d // h not in HEAD_DIMS or not supported(x, ln) or not supported(x, blk.norm_mlp.ln)
+            or not plain(x, seeds, *params)):
+        return None
+    return call(_PmaBlock, _Setup(blk, tokens, mab, mlp, dt, attn_p, again), x.contiguous(), seeds, *params)

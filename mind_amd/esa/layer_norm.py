@@ -26,6 +26,7 @@ import torch
 from torch import nn
 
 from .. import _lib
+from .eager import call
 
 _CODES = {torch.float32: _lib.ESA_F32, torch.bfloat16: _lib.ESA_BF16}
 MAX_FEATURES = 2048
@@ -37,23 +38,55 @@ def supported(x: torch.Tensor, ln: nn.LayerNorm) -> bool:
             and 4 <= d <= MAX_FEATURES)
 
 
+def f32_values(p: torch.Tensor | None) -> torch.Tensor | None:
+    """The parameter's values as contiguous fp32."""
+    return p if p is None or (p.dtype == torch.float32 and p.is_contiguous()) else p.detach().float().contiguous()
+
+
+def ln_forward(x, w32, b32, eps: float, y_dtype, full: bool, lowp: bool):
+    """esa_layer_norm_fwd over contiguous x: (y or None, bf16 rows or None, [2, rows] mean and 1 / std)."""
+    d = x.shape[-1]
+    rows = x.numel() // d
+    y = torch.empty(x.shape, dtype=y_dtype, device=x.device) if full else None
+    ylp = torch.empty(x.shape, dtype=torch.bfloat16, device=x.device) if lowp else None
+    stats = torch.empty(2, rows, dtype=torch.float32, device=x.device)
+    rc = _lib.load().esa_layer_norm_fwd(x.data_ptr(), _CODES[x.dtype], _lib.ptr(w32), _lib.ptr(b32), rows, d,
+                                        float(eps), _lib.ptr(y), _CODES[y_dtype], _lib.ptr(ylp), stats.data_ptr(),
+                                        stats.data_ptr() + 4 * rows, _lib.stream_of(x))
+    _lib.check(rc, "esa_layer_norm_fwd")
+    return y, ylp, stats
+
+
+def ln_backward(x, w32, stats, gy, gl, gr, need_w: bool, need_b: bool):
+    """esa_layer_norm_bwd: (dx, dweight, dbias) of the outputs' gradients gy (fp32 or bf16) and gl (bf16), gr
+    (x's dtype) added to dx; all contiguous, any of them None (not both gy and gl)."""
+    d = x.shape[-1]
+    rows = x.numel() // d
+    dx = torch.empty_like(x)
+    dw = torch.empty(d, dtype=torch.float32, device=x.device) if need_w else None
+    db = torch.empty(d, dtype=torch.float32, device=x.device) if need_b else None
+    lib = _lib.load()
+    ws = None
+    if need_w or need_b:
+        n = ctypes.c_size_t(0)
+        _lib.check(lib.esa_layer_norm_bwd_workspace_size(rows, d, ctypes.byref(n)), "esa_layer_norm_bwd_workspace_size")
+        ws = torch.empty(max(int(n.value), 1), dtype=torch.uint8, device=x.device)
+    rc = lib.esa_layer_norm_bwd(x.data_ptr(), _CODES[x.dtype], _lib.ptr(w32), stats.data_ptr(),
+                                stats.data_ptr() + 4 * rows, _lib.ptr(gy),
+                                _CODES[gy.dtype] if gy is not None else _lib.ESA_F32, _lib.ptr(gl), _lib.ptr(gr), rows,
+                                d, dx.data_ptr(), _lib.ptr(dw), _lib.ptr(db), _lib.ptr(ws),
+                                0 if ws is None else ws.numel(), _lib.stream_of(x))
+    _lib.check(rc, "esa_layer_norm_bwd")
+    return dx, dw, db
+
+
 class _LayerNorm(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x_in, weight, bias, eps, y_dtype, full, lowp, passthrough):
         x = x_in.contiguous()
-        d = x.shape[-1]
-        rows = x.numel() // d
-        w32 = None if weight is None else weight.detach().float().contiguous()
-        b32 = None if bias is None else bias.detach().float().contiguous()
-        y = torch.empty(x.shape, dtype=y_dtype, device=x.device) if full else None
-        ylp = torch.empty(x.shape, dtype=torch.bfloat16, device=x.device) if lowp else None
-        mean = torch.empty(rows, dtype=torch.float32, device=x.device)
-        rstd = torch.empty(rows, dtype=torch.float32, device=x.device)
-        rc = _lib.load().esa_layer_norm_fwd(x.data_ptr(), _CODES[x.dtype], _lib.ptr(w32), _lib.ptr(b32), rows, d,
-                                            float(eps), _lib.ptr(y), _CODES[y_dtype], _lib.ptr(ylp),
-                                            mean.data_ptr(), rstd.data_ptr(), _lib.stream_of(x))
-        _lib.check(rc, "esa_layer_norm_fwd")
-        ctx.save_for_backward(x, w32, mean, rstd)
+        w32, b32 = f32_values(weight), f32_values(bias)
+        y, ylp, stats = ln_forward(x, w32, b32, eps, y_dtype, full, lowp)
+        ctx.save_for_backward(x, w32, stats)
         ctx.set_materialize_grads(False)   # an unused output's gradient stays None (no zero tensor is read)
         ctx.param_dtypes = (None if weight is None else weight.dtype, None if bias is None else bias.dtype)
         ctx.outputs = (full, lowp, passthrough)
@@ -62,7 +95,7 @@ class _LayerNorm(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, *grads):
-        x, w32, mean, rstd = ctx.saved_tensors
+        x, w32, stats = ctx.saved_tensors
         full, lowp, passthrough = ctx.outputs
         grads = list(grads)
         gy = grads.pop(0) if full else None
@@ -76,25 +109,11 @@ class _LayerNorm(torch.autograd.Function):
             gl = gl.to(torch.bfloat16).contiguous()
         if gr is not None:
             gr = gr.to(x.dtype).contiguous()
-        d = x.shape[-1]
-        rows = x.numel() // d
-        dx = torch.empty_like(x)
-        wdt, bdt = ctx.param_dtypes
-        need_w = wdt is not None and ctx.needs_input_grad[1]
-        need_b = bdt is not None and ctx.needs_input_grad[2]
         if gy is None and gl is None:
             return (torch.zeros_like(x) if gr is None else gr), None, None, None, None, None, None, None
-        dw = torch.empty(d, dtype=torch.float32, device=x.device) if need_w else None
-        db = torch.empty(d, dtype=torch.float32, device=x.device) if need_b else None
-        lib = _lib.load()
-        n = ctypes.c_size_t(0)
-        _lib.check(lib.esa_layer_norm_bwd_workspace_size(rows, d, ctypes.byref(n)), "esa_layer_norm_bwd_workspace_size")
-        ws = torch.empty(max(int(n.value), 1), dtype=torch.uint8, device=x.device) if (need_w or need_b) else None
-        rc = lib.esa_layer_norm_bwd(x.data_ptr(), _CODES[x.dtype], _lib.ptr(w32), mean.data_ptr(), rstd.data_ptr(),
-                                    _lib.ptr(gy), _CODES[gy.dtype] if gy is not None else _lib.ESA_F32, _lib.ptr(gl),
-                                    _lib.ptr(gr), rows, d, dx.data_ptr(), _lib.ptr(dw), _lib.ptr(db), _lib.ptr(ws),
-                                    0 if ws is None else ws.numel(), _lib.stream_of(x))
-        _lib.check(rc, "esa_layer_norm_bwd")
+        wdt, bdt = ctx.param_dtypes
+        dx, dw, db = ln_backward(x, w32, stats, gy, gl, gr, wdt is not None and ctx.needs_input_grad[1],
+                                 bdt is not None and ctx.needs_input_grad[2])
         return (dx, None if dw is None else dw.to(wdt), None if db is None else db.to(bdt), None, None, None, None,
                 None)
 
@@ -113,7 +132,7 @@ def layer_norm(x: torch.Tensor, ln: nn.LayerNorm, full: bool = True, lowp: bool 
         lowp = False
         full = True
     y_dtype = torch.float32 if amp else x.dtype
-    out = _LayerNorm.apply(x, ln.weight, ln.bias, ln.eps, y_dtype, full, lowp, passthrough)
+    out = call(_LayerNorm, x, ln.weight, ln.bias, ln.eps, y_dtype, full, lowp, passthrough)
     if not isinstance(out, tuple):
         out = (out,)
     out = list(out)

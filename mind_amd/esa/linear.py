@@ -29,6 +29,7 @@ from torch import nn
 from torch.nn import functional as F
 
 from .. import _lib
+from .eager import call
 
 _MIN_CHUNK = 4096               # tokens per chunk: below, a chunk's GEMM is too short to pay
 _MAX_PARTIAL = 16 * 1024 * 1024  # fp32 values of all partials (64 MiB)
@@ -230,18 +231,17 @@ def param_casts(params, dt: torch.dtype):
     if not ps:
         yield
         return
-    pad = torch.zeros(_CAST_ALIGN, dtype=torch.float32, device=ps[0].device)
-    pieces, offsets, off = [], [], 0
-    for p in ps:
+    slots = [p.numel() + -p.numel() % _CAST_ALIGN for p in ps]
+    pieces, pad = [], None
+    for p, slot in zip(ps, slots):
         pieces.append(p.detach().reshape(-1))
-        offsets.append(off)
-        off += p.numel()
-        r = -off % _CAST_ALIGN
-        if r:
-            pieces.append(pad[:r])
-            off += r
-    flat = torch.cat(pieces).to(dt)
-    cache = {id(p): (p, flat[o:o + p.numel()].view(p.shape)) for p, o in zip(ps, offsets)}
+        if slot > p.numel():
+            pad = torch.zeros(_CAST_ALIGN, dtype=torch.float32, device=p.device) if pad is None else pad
+            pieces.append(pad[:slot - p.numel()])
+    cache = {}
+    for p, flat in zip(ps, torch.cat(pieces).to(dt).split(slots)):
+        flat = flat if flat.numel() == p.numel() else flat[:p.numel()]
+        cache[id(p)] = (p, flat if p.dim() == 1 else flat.view(p.shape))
     token = _CAST_CACHE.set(cache)
     try:
         yield
@@ -275,7 +275,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = No
         return F.linear(x, weight, bias)   # CPU, or mixed dtypes: torch's own type checks and errors
     x = x.to(dt)
     lead = x.shape[:-1]
-    y = _Linear.apply(x.reshape(-1, x.shape[-1]).contiguous(), weight, bias)
+    y = call(_Linear, x.reshape(-1, x.shape[-1]).contiguous(), weight, bias)
     return y.view(*lead, weight.shape[0])
 
 
@@ -344,7 +344,7 @@ def qkv_projection(fc_q: nn.Linear, fc_k: nn.Linear, fc_v: nn.Linear, xq: torch.
         return fc_q(xq), fc_k(xk), fc_v(xk)
     xq = xq.to(dt)
     xk_ = None if same else xk.to(dt).contiguous()
-    return _QKV.apply(xq.contiguous(), xk_, *params)
+    return call(_QKV, xq.contiguous(), xk_, *params)
 
 
 def hookless(layer: nn.Module) -> bool:

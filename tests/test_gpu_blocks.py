@@ -1,0 +1,119 @@
+"""The packed blocks recorded as one autograd node (mind_amd.esa.blocks) against the separate functions on the same
+kernels: outputs bit for bit, gradients of every input.
+
+Bar of the gradients, norm-wise per tensor: the two differ in where partial gradients are added and rounded.  fp32:
+one more or less rounding of 2^-24 per addition, far below 1e-5.  bf16 autocast: a gradient rounded to bf16 once
+more or once less, 2^-9 of its magnitude per rounding, at most four of them on any path: 2^-7."""
+import numpy as np
+import pytest
+import torch
+
+from mind_amd import generators
+from mind_amd.esa import attention, blocks, masked_layers
+from mind_amd.esa.packing import EdgeAdjacency, NodeAdjacency
+
+pytestmark = pytest.mark.gpu
+
+
+def _tokens(device, node, seed=0, graphs=5):
+    gb, _ = generators.small_molecules(seed=seed, num_graphs=graphs)
+    ei, bm = torch.as_tensor(gb.edge_index).to(device), torch.as_tensor(gb.batch).to(device)
+    cls, n = (NodeAdjacency, gb.node_counts.max()) if node else (EdgeAdjacency, gb.edge_counts.max())
+    return cls.from_edge_index(ei, bm, gb.num_graphs, int(n) + 3)
+
+
+def _sab(device, idx, mlp_layers, dropout=0.0, d=64):
+    torch.manual_seed(3)
+    blk = masked_layers.SABComplete(d, d, 4, dropout, idx, "LN", use_mlp=mlp_layers > 0, mlp_hidden_size=96,
+                                    num_mlp_layers=max(mlp_layers, 2), xformers_or_torch_attn="hip").to(device)
+    return blk.train()
+
+
+def _both(one, separate, x, params, g, amp):
+    res = []
+    for fn in (one, separate):
+        with torch.autocast("cuda", torch.bfloat16, enabled=amp):
+            out = fn()
+        assert out is not None
+        res.append((out, torch.autograd.grad(out, [x] + params, g.to(out.dtype))))
+    (o1, g1), (o2, g2) = res
+    assert torch.equal(o1, o2)
+    size = 0.0
+    for a, b in zip(g1, g2):
+        assert a.dtype == b.dtype and a.shape == b.shape
+        # a bias sums the rows that its weight (the tensor before it) sums against inputs of about 1; fc_k's is zero
+        # but for rounding, the softmax being unchanged by it
+        size = max(float(b.double().norm()), size if b.dim() == 1 else 0.0)
+        assert float((a.double() - b.double()).norm()) <= (2.0 ** -7 if amp else 1e-5) * size
+
+
+@pytest.mark.parametrize("amp", [False, True])
+@pytest.mark.parametrize("idx,node,mlp_layers,dropout", [(0, False, 2, 0.0), (1, False, 2, 0.0), (1, True, 3, 0.1),
+                                                         (0, False, 0, 0.0), (0, False, 2, 0.2)])
+def test_sab_block(device, amp, idx, node, mlp_layers, dropout):
+    tokens, blk = _tokens(device, node), _sab(device, idx, mlp_layers, dropout)
+    x = torch.randn(tokens.num_tokens, 64, device=device, requires_grad=True)
+    g = torch.randn(tokens.num_tokens, 64, device=device)
+    params = [p for n, p in blk.named_parameters() if mlp_layers or "norm_mlp" not in n]
+    seeds = []
+
+    def one():
+        return blocks.sab_block(blk, x, tokens, idx == 1, dropout, lambda a, seed: seeds.append(seed))
+
+    def separate():
+        return masked_layers._sab_separate(blk, x, tokens, seed)
+
+    state = torch.get_rng_state()
+    seed = attention.draw_dropout_seed() if dropout else None   # what the block draws from the same state
+    torch.set_rng_state(state)
+    _both(one, separate, x, params, g, amp)
+
+
+@pytest.mark.parametrize("amp", [False, True])
+@pytest.mark.parametrize("k_seeds,dropout", [(1, 0.0), (4, 0.1)])
+def test_pma_block(device, amp, k_seeds, dropout):
+    tokens = _tokens(device, False)
+    torch.manual_seed(4)
+    blk = masked_layers.PMAComplete(64, 4, k_seeds, "LN", dropout=dropout, use_mlp=True, mlp_hidden_size=96,
+                                    num_mlp_layers=2, xformers_or_torch_attn="hip").to(device).train()
+    x = torch.randn(tokens.num_tokens, 64, device=device, requires_grad=True)
+    g = torch.randn(tokens.batch_size, k_seeds, 64, device=device)
+    state = torch.get_rng_state()
+    seed = attention.draw_dropout_seed() if dropout else None
+    torch.set_rng_state(state)
+    _both(lambda: blocks.pma_block(blk, x, tokens, dropout, None),
+          lambda: masked_layers._pma_separate(blk, x, tokens, seed), x, list(blk.parameters()), g, amp)
+
+
+def test_frozen_parameters_and_input(device):
+    tokens, blk = _tokens(device, False), _sab(device, 1, 2)
+    for p in list(blk.sab.mab.fc_k.parameters()) + [blk.norm.ln.bias, blk.mlp.mlp[0].weight]:
+        p.requires_grad_(False)
+    x = torch.randn(tokens.num_tokens, 64, device=device)
+    out = blocks.sab_block(blk, x, tokens, True, 0.0, None)
+    params = [p for p in blk.parameters() if p.requires_grad]
+    got = torch.autograd.grad(out.sum(), params)
+    ref = torch.autograd.grad(masked_layers._sab_separate(blk, x, tokens).sum(), params)
+    assert all(torch.allclose(a, b, rtol=1e-4, atol=1e-4 * float(b.abs().max())) for a, b in zip(got, ref))
+    with torch.no_grad():
+        assert torch.equal(blocks.sab_block(blk, x, tokens, True, 0.0, None), out)
+
+
+def test_differentiated_again_and_not_taken(device):
+    tokens, blk = _tokens(device, False), _sab(device, 0, 2)
+    x = torch.randn(tokens.num_tokens, 64, device=device, requires_grad=True)
+    grads = []
+    for fn in (lambda: masked_layers._sab_forward_packed(blk, x, tokens), lambda: masked_layers._sab_separate(blk, x, tokens)):
+        w = blk.mlp.mlp[2].weight
+        (gw,) = torch.autograd.grad(fn().square().sum(), w, create_graph=True)
+        assert gw.requires_grad
+        grads.append(torch.autograd.grad(gw.square().sum(), w)[0])
+    assert torch.allclose(grads[0], grads[1], rtol=1e-4, atol=1e-4 * float(grads[1].abs().max()))
+    assert blocks.sab_block(blk, x.bfloat16(), tokens, False, 0.0, None) is None
+    with torch.autocast("cuda", torch.float16):
+        assert blocks.sab_block(blk, x, tokens, False, 0.0, None) is None
+    seen = []
+    handle = blk.mlp.register_forward_hook(lambda *a: seen.append(1))
+    masked_layers._sab_forward_packed(blk, x, tokens)
+    handle.remove()
+    assert seen
