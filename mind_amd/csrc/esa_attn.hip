@@ -1329,14 +1329,11 @@ __global__ __launch_bounds__(256) void list_dkdv_kernel(const AttnArgs a0) {
 
 // ======================================================================== fp32 path
 // fp32 q, k, v, outputs and softmax (the reference's fp32 modules, compared
-// at 1e-5 relative).  One thread per (outer token, head) of a group of up to
-// 128 outer tokens of one segment (a per-segment plan, longest partner range
-// first: a block walks only its own segment's partners, so few-query
-// segments such as PMA seeds get one block per segment and head), partner
-// runs of 32 tokens staged in LDS and read by broadcast (the forward holds a
-// partner row across each 16-lane wave row instead and splits a group's key
-// tiles over several thread groups; see attn_fwd_f32_kernel).  Scores,
-// softmax and both products are fp32 FMA chains in a fixed order.  Exponentials and the
+// at 1e-5 relative).  Blocks take groups of up to 128 outer tokens of one
+// segment (a per-segment plan, longest partner range first: a block walks
+// only its own segment's partners, so few-query segments such as PMA seeds
+// get one block per segment and head).  Scores, softmax and all products are
+// fp32, in a fixed order.  Exponentials and the
 // log-sum-exp use the hardware v_exp_f32 / v_log_f32 (about 1 ulp): every
 // exponent is <= 0 (a score minus the running maximum or the row's LSE2) and
 // every log argument >= 1 (the row sum includes the maximum's 1), so the
@@ -1358,8 +1355,6 @@ struct AttnF32Args {
   float* o; float* lse_out; float* dq; float* dk; float* dv;
 };
 
-constexpr int kF32Threads = kGroupTok;
-
 // Rows of HD fp32 values (HD = 16, 24, 32 or 64) as float4 chunks.
 template <int HD>
 DEVI void loadn(const float* p, float x[HD]) {
@@ -1376,39 +1371,6 @@ DEVI void storen(float* p, const float x[HD], float mul) {
     reinterpret_cast<float4*>(p)[i] = make_float4(x[4 * i] * mul, x[4 * i + 1] * mul, x[4 * i + 2] * mul,
                                                   x[4 * i + 3] * mul);
 }
-template <int HD>
-DEVI float dotn(const float x[HD], const float4* y) {
-  float s = 0.f;
-#pragma unroll
-  for (int i = 0; i < HD / 4; ++i) {
-    const float4 v = y[i];
-    s = fmaf(x[4 * i], v.x, s); s = fmaf(x[4 * i + 1], v.y, s);
-    s = fmaf(x[4 * i + 2], v.z, s); s = fmaf(x[4 * i + 3], v.w, s);
-  }
-  return s;
-}
-template <int HD>
-DEVI void axpyn(float a, const float4* y, float x[HD]) {
-#pragma unroll
-  for (int i = 0; i < HD / 4; ++i) {
-    const float4 v = y[i];
-    x[4 * i] = fmaf(a, v.x, x[4 * i]); x[4 * i + 1] = fmaf(a, v.y, x[4 * i + 1]);
-    x[4 * i + 2] = fmaf(a, v.z, x[4 * i + 2]); x[4 * i + 3] = fmaf(a, v.w, x[4 * i + 3]);
-  }
-}
-
-// Stage the 32 tokens from t0 of a [T][H][HD] fp32 tensor into LDS [32][HD / 4]
-// float4 (128 threads, HD / 16 float4 each); tokens at or past `end` read as zeros.
-template <int HD>
-DEVI void stage_rows_f32(float4 (*dst)[HD / 4], const float* src, int end, int H, int head, int t0, int tid) {
-#pragma unroll
-  for (int i = tid; i < kTile * HD / 4; i += kF32Threads) {
-    const int t = t0 + i / (HD / 4), part = i % (HD / 4);
-    dst[i / (HD / 4)][part] = t < end ? reinterpret_cast<const float4*>(src + ((size_t)t * H + head) * HD)[part]
-                                      : make_float4(0.f, 0.f, 0.f, 0.f);
-  }
-}
-
 // Admissible partner p (below the segment's partner end phi) of outer token oi.
 template <bool MASKED>
 DEVI bool admissible_f32(int p, int phi, int oi, int2 pn, int2 own) {
@@ -1417,240 +1379,259 @@ DEVI bool admissible_f32(int p, int phi, int oi, int2 pn, int2 own) {
   return ok;
 }
 
-// This thread's outer token of group g (clamped into the group when past its
-// segment's end).
-struct F32Outer { int oi, oc; bool valid; int plo, phi; };
-DEVI F32Outer f32_outer(const int4& g, int tid) {
-  F32Outer o;
-  o.oi = g.x + tid;
-  o.valid = o.oi < g.y;
-  o.oc = o.valid ? o.oi : g.x;
-  o.plo = g.z;
-  o.phi = g.w;
-  return o;
-}
+// ---- Tiled fp32 kernels on the matrix cores.
+// v_mfma_f32_16x16x4_f32 multiplies exactly and accumulates in fp32.  A block
+// takes a group of up to 128 outer tokens of one segment and one head; a wave
+// owns QB 16-token column blocks of it, and partner tokens are staged 64 at a
+// time into double-buffered LDS, the next stage's rows in flight in registers.
+// Scores of a 16-partner x 16-owned block: A = partner rows, B = owned rows,
+// lane l (column l % 16, group G = l / 16) supplying dims 4 G + j of MFMA j's
+// four, so both operands are 16-byte reads of rows as they are in memory.  The
+// result leaves lane l partners 4 G .. 4 G + 3 of its owned token, which is
+// the B operand of the products over partners (MFMA r takes partner 4 G + r
+// of every group), with A[dim l % 16] = that partner's value, a 4-byte read:
+// P and dS never leave their registers.  Staged rows are 4 floats longer than
+// their dims, which keeps both reads free of bank conflicts.  Dims past HD
+// (HD 24) are staged as zeros.
+//
+// What bounds them: the fp32 matrix rate (32 cycles per MFMA and SIMD; per
+// block of 256 scores at head dim 16: 8 in the forward, 12 in dQ, 16 in
+// dK/dV) and, on small batches, the serial walk of the longest segment.  One
+// thread per (token, head) with vector FMAs, before: forward / dQ / dK/dV of
+// 64 small molecules (21,752 tokens, 8 heads of 16) 135 / 192 / 214 us dense and
+// 143 / 234 / 241 us with the edge mask, now
+// 90 / 103 / 122 and 100 / 119 / 149 us; 8 heads of 64, dense: 445 / 1054 / 2071
+// -> 221 / 296 / 406 us (93-107 of the 154 TFLOP/s of a large fp32 product).
+constexpr int kF32Stage = 64;
 
-// Partner rows across a wave row.  A staged partner row of HD fp32 values is
-// held by the 16 lanes of each wave row: lane l holds dims l % 16,
-// 16 + l % 16, ... (NR = ceil(HD / 16) registers, zeros past HD), and all
-// four rows of the wave hold the same partner.  `v_fmac_f32_dpp` with
-// row_newbcast:i hands dim 16 r + i of that partner to the 16 lanes of each
-// row inside the multiply-add, so a product with a partner row costs one VALU
-// instruction per dim and one 4-byte LDS read per partner and lane.  Read as
-// whole rows per lane, the same partner costs HD / 4 16-byte reads per lane:
-// the broadcast reads move 64 x 16 bytes through the LDS pipe each, and they,
-// not the FMAs, bounded the kernels.  DPP reads the source lane's register,
-// so every lane of the wave is active at these instructions (lanes past
-// their group's end compute on a clamped token and store nothing).  The
-// leading s_nop 1 covers the two wait states a DPP read of a VGPR needs
-// after a VALU write of it.
-#define F32_FM(ACC, SRC, MUL, I) \
-  "v_fmac_f32_dpp %" #ACC ", %" #SRC ", %" #MUL " row_newbcast:" #I " row_mask:0xf bank_mask:0xf\n\t"
-#define F32_DOT4(I, Q) F32_FM(0, 4, Q, I) F32_FM(1, 5, Q, I) F32_FM(2, 6, Q, I) F32_FM(3, 7, Q, I)
-#define F32_AXPY8(V, P)                                                                                 \
-  F32_FM(0, V, P, 0) F32_FM(1, V, P, 1) F32_FM(2, V, P, 2) F32_FM(3, V, P, 3) F32_FM(4, V, P, 4)         \
-  F32_FM(5, V, P, 5) F32_FM(6, V, P, 6) F32_FM(7, V, P, 7)
-#define F32_AXPY16(V, P)                                                                                \
-  F32_AXPY8(V, P) F32_FM(8, V, P, 8) F32_FM(9, V, P, 9) F32_FM(10, V, P, 10) F32_FM(11, V, P, 11)        \
-  F32_FM(12, V, P, 12) F32_FM(13, V, P, 13) F32_FM(14, V, P, 14) F32_FM(15, V, P, 15)
-
-// s[k] += sum over the register's N dims (8 or 16, ascending) of x[i] * dim i
-// of partner k's row register y[k], for four partners.
-template <int N>
-DEVI void dot4_rows(float (&s)[4], const float (&y)[4], const float* x) {
-  if constexpr (N == 16)
-    asm("s_nop 1\n\t"
-        F32_DOT4(0, 8) F32_DOT4(1, 9) F32_DOT4(2, 10) F32_DOT4(3, 11) F32_DOT4(4, 12) F32_DOT4(5, 13)
-        F32_DOT4(6, 14) F32_DOT4(7, 15) F32_DOT4(8, 16) F32_DOT4(9, 17) F32_DOT4(10, 18) F32_DOT4(11, 19)
-        F32_DOT4(12, 20) F32_DOT4(13, 21) F32_DOT4(14, 22) F32_DOT4(15, 23)
-        : "+v"(s[0]), "+v"(s[1]), "+v"(s[2]), "+v"(s[3])
-        : "v"(y[0]), "v"(y[1]), "v"(y[2]), "v"(y[3]), "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(x[4]),
-          "v"(x[5]), "v"(x[6]), "v"(x[7]), "v"(x[8]), "v"(x[9]), "v"(x[10]), "v"(x[11]), "v"(x[12]),
-          "v"(x[13]), "v"(x[14]), "v"(x[15]));
-  else
-    asm("s_nop 1\n\t"
-        F32_DOT4(0, 8) F32_DOT4(1, 9) F32_DOT4(2, 10) F32_DOT4(3, 11) F32_DOT4(4, 12) F32_DOT4(5, 13)
-        F32_DOT4(6, 14) F32_DOT4(7, 15)
-        : "+v"(s[0]), "+v"(s[1]), "+v"(s[2]), "+v"(s[3])
-        : "v"(y[0]), "v"(y[1]), "v"(y[2]), "v"(y[3]), "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(x[4]),
-          "v"(x[5]), "v"(x[6]), "v"(x[7]));
-}
-
-// x[i] += a * dim i of the row register y, over the register's N dims (8 or 16).
-template <int N>
-DEVI void axpy_row(float* x, float y, float a) {
-  if constexpr (N == 16)
-    asm("s_nop 1\n\t" F32_AXPY16(16, 17)
-        : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]), "+v"(x[7]),
-          "+v"(x[8]), "+v"(x[9]), "+v"(x[10]), "+v"(x[11]), "+v"(x[12]), "+v"(x[13]), "+v"(x[14]), "+v"(x[15])
-        : "v"(y), "v"(a));
-  else
-    asm("s_nop 1\n\t" F32_AXPY8(8, 9)
-        : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]), "+v"(x[7])
-        : "v"(y), "v"(a));
-}
-
-// Dims held by register r of an HD-wide row (16, or 8 for the last register of HD 24).
 template <int HD>
-DEVI constexpr int row_dims(int r) { return HD - 16 * r >= 16 ? 16 : HD - 16 * r; }
+struct F32Tile {
+  static constexpr int NR = (HD + 15) / 16;              // 16-dim chunks of a row
+  static constexpr int QB = HD <= 32 ? 2 : 1;            // column blocks per wave
+  static constexpr int kThreads = 64 * (kGroupTok / (16 * QB));
+  static constexpr int kStride = 16 * NR + 4;            // floats per staged row
+  static constexpr int kPer = kF32Stage * 4 * NR / kThreads;   // 16-byte chunks per thread and staged tensor
+  typedef float Rows[kF32Stage][kStride];
+};
 
-// A partner row's registers for lane li: y[r] = dim 16 r + li of the row.
+DEVI f32x4 mfma16x4f(float a, float b, const f32x4& c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
+// The stage's rows of a [T][H][HD] tensor from token t0 on, into registers and from there into LDS; tokens at or
+// past `end` are zeros.
 template <int HD>
-DEVI void row_regs(float (&y)[(HD + 15) / 16], const float* row, int li) {
+DEVI void f32_load(f32x4 (&r)[F32Tile<HD>::kPer], const float* src, int end, int H, int head, int t0) {
+  using T = F32Tile<HD>;
 #pragma unroll
-  for (int r = 0; r < (HD + 15) / 16; ++r) y[r] = row[16 * r + li];
-}
-
-// Four partners' dot products with the lane's row x (HD dims, ascending):
-// s[k] = sum_d x[d] * dim d of partner k, from the partners' row registers.
-template <int HD, int R = 0>
-DEVI void dot4(float (&s)[4], const float* x, const float (&y)[4][(HD + 15) / 16]) {
-  if constexpr (R == 0) s[0] = s[1] = s[2] = s[3] = 0.f;
-  if constexpr (16 * R < HD) {
-    const float yr[4] = {y[0][R], y[1][R], y[2][R], y[3][R]};
-    dot4_rows<row_dims<HD>(R)>(s, yr, x + 16 * R);
-    dot4<HD, R + 1>(s, x, y);
+  for (int i = 0; i < T::kPer; ++i) {
+    const int x = threadIdx.x + i * T::kThreads, t = t0 + x / (4 * T::NR), part = x % (4 * T::NR);
+    r[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (t < end && part < HD / 4) r[i] = *reinterpret_cast<const f32x4*>(src + ((size_t)t * H + head) * HD + 4 * part);
   }
 }
-
-// x[d] += a * dim d of a partner row (HD dims) from its row registers.
-template <int HD, int R = 0>
-DEVI void axpy(float* x, float a, const float (&y)[(HD + 15) / 16]) {
-  if constexpr (16 * R < HD) {
-    axpy_row<row_dims<HD>(R)>(x + 16 * R, y[R], a);
-    axpy<HD, R + 1>(x, a, y);
-  }
-}
-
-// Stage the 32 tokens from t0 of a [T][H][HD] fp32 tensor into LDS rows of
-// 16 NR floats (128 threads): dims past HD and tokens at or past `end` are zeros.
 template <int HD>
-DEVI void stage_rows_lane(float (*dst)[16 * ((HD + 15) / 16)], const float* src, int end, int H, int head, int t0,
-                          int tid) {
-  constexpr int C = 4 * ((HD + 15) / 16);   // float4 chunks per staged row
+DEVI void f32_store(float (*dst)[F32Tile<HD>::kStride], const f32x4 (&r)[F32Tile<HD>::kPer]) {
+  using T = F32Tile<HD>;
 #pragma unroll
-  for (int i = tid; i < kTile * C; i += kF32Threads) {
-    const int t = t0 + i / C, part = i % C;
-    reinterpret_cast<float4*>(dst[i / C])[part] =
-        t < end && part < HD / 4 ? reinterpret_cast<const float4*>(src + ((size_t)t * H + head) * HD)[part]
-                                 : make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int i = 0; i < T::kPer; ++i) {
+    const int x = threadIdx.x + i * T::kThreads;
+    *reinterpret_cast<f32x4*>(&dst[x / (4 * T::NR)][4 * (x % (4 * T::NR))]) = r[i];
   }
 }
 
-// Key splits of the fp32 forward: S groups of 128 threads per block take the
-// group's key tiles in turn (tile i goes to split i mod S), each with its own
-// staging buffers, and merge their (max, sum, output) partials at the end in
-// split order.  One thread per (query, head) gives only a few thousand waves
-// per call (configuration 0: 2,392 for 1,024 SIMDs) with per-block work
-// proportional to the segment length; with the splits the long segments'
-// blocks finish S times sooner and the SIMDs hold S times the waves.
+// An owned row's B operand: dims 16 c + 4 grp .. + 3.
 template <int HD>
-constexpr int f32_splits() { return HD >= 64 ? 2 : 4; }
+DEVI void f32_owned(f32x4 (&x)[F32Tile<HD>::NR], const float* src, int tok, int H, int head, int grp) {
+#pragma unroll
+  for (int c = 0; c < F32Tile<HD>::NR; ++c) {
+    x[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (16 * c + 4 * grp < HD) x[c] = *reinterpret_cast<const f32x4*>(src + ((size_t)tok * H + head) * HD + 16 * c + 4 * grp);
+  }
+}
+template <int HD>
+DEVI void f32_write(float* dst, const f32x4 (&x)[F32Tile<HD>::NR], float mul, int tok, int H, int head, int grp) {
+#pragma unroll
+  for (int c = 0; c < F32Tile<HD>::NR; ++c)
+    if (16 * c + 4 * grp < HD) {
+      f32x4 y = x[c];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[e] *= mul;
+      *reinterpret_cast<f32x4*>(dst + ((size_t)tok * H + head) * HD + 16 * c + 4 * grp) = y;
+    }
+}
+
+// Partner rows p0 + l % 16 (a staged tile's row offset) times the owned rows: 16 x 16 products.
+template <int HD>
+DEVI void f32_rows(f32x4 (&x)[F32Tile<HD>::NR], const float (*rows)[F32Tile<HD>::kStride], int p0, int c16, int grp) {
+#pragma unroll
+  for (int c = 0; c < F32Tile<HD>::NR; ++c) x[c] = *reinterpret_cast<const f32x4*>(&rows[p0 + c16][16 * c + 4 * grp]);
+}
+template <int HD>
+DEVI f32x4 f32_product(const f32x4 (&p)[F32Tile<HD>::NR], const f32x4 (&o)[F32Tile<HD>::NR]) {
+  f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int c = 0; c < F32Tile<HD>::NR; ++c)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) s = mfma16x4f(p[c][j], o[c][j], s);
+  return s;
+}
+// acc[b] += over the 16 partners from p0: partner's row times w[b] (partner 4 grp + r in w[b][r]), for QB owned blocks.
+template <int HD>
+DEVI void f32_gather(f32x4 (&acc)[F32Tile<HD>::QB][F32Tile<HD>::NR], const float (*rows)[F32Tile<HD>::kStride], int p0,
+                     const f32x4 (&w)[F32Tile<HD>::QB], int c16, int grp) {
+#pragma unroll
+  for (int c = 0; c < F32Tile<HD>::NR; ++c)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float x = rows[p0 + 4 * grp + r][16 * c + c16];
+#pragma unroll
+      for (int b = 0; b < F32Tile<HD>::QB; ++b) acc[b][c] = mfma16x4f(x, w[b][r], acc[b][c]);
+    }
+}
+
+// The block's work item, the wave's column blocks and this lane's owned tokens (clamped into the group).
+template <int HD>
+struct F32Own {
+  static constexpr int QB = F32Tile<HD>::QB;
+  int plo, phi, tok[QB];
+  bool live, valid[QB];   // live: the wave owns a token (wave-uniform)
+  DEVI F32Own(const int4& g, int wave, int c16) {
+    plo = g.z;
+    phi = g.w;
+    live = g.x + 16 * QB * wave < g.y;
+#pragma unroll
+    for (int b = 0; b < QB; ++b) {
+      const int t = g.x + 16 * (QB * wave + b) + c16;
+      valid[b] = t < g.y;
+      tok[b] = valid[b] ? t : g.x;
+    }
+  }
+};
+
+// Walks the partner range in stages of 64: `load(t0)` takes a stage's rows into registers, `store(buf)` from there
+// into LDS, `use(buf, t0)` computes (live waves).
+template <class Load, class Store, class Use>
+DEVI void f32_stages(int lo, int hi, bool live, Load load, Store store, Use use) {
+  if (lo >= hi) return;
+  load(lo);
+  store(0);
+  int buf = 0;
+  for (int t0 = lo; t0 < hi; t0 += kF32Stage, buf ^= 1) {
+    const bool more = t0 + kF32Stage < hi;
+    if (more) load(t0 + kF32Stage);
+    __syncthreads();   // the stage is in LDS, and every wave is done with the other buffer
+    if (live) use(buf, t0);
+    if (more) store(buf ^ 1);
+  }
+}
 
 template <bool MASKED, int HD, bool DROP>
-__global__ __launch_bounds__(kF32Threads * f32_splits<HD>()) void attn_fwd_f32_kernel(const AttnF32Args a) {
-  constexpr int NR = (HD + 15) / 16, S = f32_splits<HD>();
-  __shared__ float sK[S][kTile][16 * NR], sV[S][kTile][16 * NR];
-  __shared__ int2 sN[S][kTile];
-  __shared__ uint32_t sKey[S][DROP ? kTile : 1];   // column keys of the staged keys
-  __shared__ float sAcc[kF32Threads][16 * NR + 1];   // a later split's partial: output row, then m and l
-  __shared__ float sML[kF32Threads][2];
-  const int split = threadIdx.x / kF32Threads, tid = threadIdx.x - split * kF32Threads, li = tid & 15;
-  const int H = a.heads;
-  const int item = blockIdx.x / H, head = blockIdx.x - item * H;
+__global__ __launch_bounds__(F32Tile<HD>::kThreads) void attn_fwd_f32_kernel(const AttnF32Args a) {
+  using T = F32Tile<HD>;
+  constexpr int NR = T::NR, QB = T::QB, KB = kF32Stage / 16;
+  __shared__ __align__(16) typename T::Rows sK[2], sV[2];
+  __shared__ int2 sN[2][MASKED ? kF32Stage : 1];
+  __shared__ uint32_t sKey[2][DROP ? kF32Stage : 1];   // column keys of the staged keys
+  const int H = a.heads, item = blockIdx.x / H, head = blockIdx.x - item * H;
   if (item >= *a.count) return;
-  const F32Outer ot = f32_outer(a.plan[item], tid);
-  const int oi = ot.oi, oc = ot.oc, phi = ot.phi;
-  float q[16 * NR], acc[16 * NR];
-  loadn<HD>(a.q + ((size_t)oc * H + head) * HD, q);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c16 = lane & 15, grp = lane >> 4;
+  const F32Own<HD> own(a.plan[item], wave, c16);
+  const int phi = own.phi;
+  f32x4 q[QB][NR], acc[QB][NR];
+  int2 node[QB];
+  uint32_t rk[QB];
+  float m[QB], l[QB];
 #pragma unroll
-  for (int i = 0; i < 16 * NR; ++i) {
-    if (i >= HD) q[i] = 0.f;
-    acc[i] = 0.f;
+  for (int b = 0; b < QB; ++b) {
+    f32_owned<HD>(q[b], a.q, own.tok[b], H, head, grp);
+#pragma unroll
+    for (int c = 0; c < NR; ++c) acc[b][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    node[b] = MASKED ? a.nodes[own.tok[b]] : make_int2(0, 0);
+    rk[b] = DROP ? drop_row(a.drop, own.tok[b], head) : 0u;
+    m[b] = -INFINITY;
+    l[b] = 0.f;
   }
-  const int2 own = MASKED ? a.nodes[oc] : make_int2(0, 0);
-  const uint32_t rk = DROP ? drop_row(a.drop, oc, head) : 0u;
-  float m = -INFINITY, l = 0.f;
-  const int rounds = (phi - ot.plo + S * kTile - 1) / (S * kTile);
-  for (int it = 0; it < rounds; ++it) {
-    const int k0 = ot.plo + (it * S + split) * kTile;   // past phi: nothing to do this round (split-uniform)
-    __syncthreads();
-    if (k0 < phi) {
-      stage_rows_lane<HD>(sK[split], a.k, phi, H, head, k0, tid);
-      stage_rows_lane<HD>(sV[split], a.v, phi, H, head, k0, tid);
-      if (MASKED && tid < kTile) sN[split][tid] = k0 + tid < phi ? a.nodes[k0 + tid] : make_int2(-1, -1);
-      if (DROP && tid < kTile) sKey[split][tid] = drop_col(a.drop, k0 + tid);
-    }
-    __syncthreads();
-    if (k0 >= phi) continue;
-    float s[kTile];
-    float mt = -INFINITY;
-    float ky[kTile][NR];   // the tile's key rows, loaded one group of four ahead of their products
+  f32x4 rK[T::kPer], rV[T::kPer];
+  int2 rN = make_int2(-1, -1);
+  uint32_t rKey = 0;
+  f32_stages(
+      own.plo, phi, own.live,
+      [&](int t0) {
+        f32_load<HD>(rK, a.k, phi, H, head, t0);
+        f32_load<HD>(rV, a.v, phi, H, head, t0);
+        if (MASKED && tid < kF32Stage) rN = t0 + tid < phi ? a.nodes[t0 + tid] : make_int2(-1, -1);
+        if (DROP && tid < kF32Stage) rKey = drop_col(a.drop, t0 + tid);
+      },
+      [&](int buf) {
+        f32_store<HD>(sK[buf], rK);
+        f32_store<HD>(sV[buf], rV);
+        if (MASKED && tid < kF32Stage) sN[buf][tid] = rN;
+        if (DROP && tid < kF32Stage) sKey[buf][tid] = rKey;
+      },
+      [&](int buf, int k0) {
+        f32x4 s[KB][QB];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) row_regs<HD>(ky[u], sK[split][u], li);
+        for (int kb = 0; kb < KB; ++kb) {
+          f32x4 x[NR];
+          f32_rows<HD>(x, sK[buf], 16 * kb, c16, grp);
 #pragma unroll
-    for (int j = 0; j < kTile; j += 4) {
-      if (j + 4 < kTile) {
+          for (int b = 0; b < QB; ++b) s[kb][b] = f32_product<HD>(x, q[b]);
+        }
+        const bool tail = k0 + kF32Stage > phi;
 #pragma unroll
-        for (int u = 4; u < 8; ++u) row_regs<HD>(ky[j + u], sK[split][j + u], li);
-      }
-      __builtin_amdgcn_sched_barrier(0);   // keep the next group's reads ahead of these products
-      float d[4];
-      dot4<HD>(d, q, *reinterpret_cast<const float(*)[4][NR]>(&ky[j]));
+        for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int2 pn = MASKED ? sN[split][j + u] : make_int2(0, 0);
-        s[j + u] = admissible_f32<MASKED>(k0 + j + u, phi, oi, pn, own) ? a.c * d[u] : -INFINITY;
-        mt = fmaxf(mt, s[j + u]);
-      }
-    }
-    if (mt > m) {
-      const float alpha = fast_exp2(m - mt);   // 0 while m = -inf
-      l *= alpha;
+          for (int r = 0; r < 4; ++r) {
+            const int key = 16 * kb + 4 * grp + r;
+            const int2 pn = MASKED ? sN[buf][key] : make_int2(0, 0);
 #pragma unroll
-      for (int i = 0; i < 16 * NR; ++i) acc[i] *= alpha;
-      m = mt;
-    }
-    const float mb = m == -INFINITY ? 0.f : m;   // no admissible key yet: every p is exp2(-inf) = 0
-    float vy[kTile][NR];   // value rows, loaded four keys ahead of their products
+            for (int b = 0; b < QB; ++b) {
+              s[kb][b][r] *= a.c;
+              if (MASKED || tail)
+                s[kb][b][r] = admissible_f32<MASKED>(k0 + key, phi, own.tok[b], pn, node[b]) ? s[kb][b][r] : -INFINITY;
+            }
+          }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) row_regs<HD>(vy[j], sV[split][j], li);
+        for (int b = 0; b < QB; ++b) {
+          float mt = s[0][b][0];
 #pragma unroll
-    for (int j = 0; j < kTile; ++j) {
-      if (j + 4 < kTile) row_regs<HD>(vy[j + 4], sV[split][j + 4], li);
-      __builtin_amdgcn_sched_barrier(0);   // keep the reads four keys ahead of their product
-      const float p = fast_exp2(s[j] - mb);
-      l += p;
-      axpy<HD>(acc, DROP && !drop_keep(a.drop, rk, sKey[split][j], k0 + j) ? 0.f : p, vy[j]);
-    }
+          for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) mt = fmaxf(mt, s[kb][b][r]);
+          if (__ballot(mt > m[b])) {   // a token's keys lie in four lanes: they share its maximum
+            mt = fmaxf(mt, __shfl_xor(mt, 16));
+            mt = fmaxf(fmaxf(mt, __shfl_xor(mt, 32)), m[b]);
+            const float alpha = mt == -INFINITY ? 1.f : fast_exp2(m[b] - mt);   // 0 while m = -inf
+            l[b] *= alpha;
+#pragma unroll
+            for (int c = 0; c < NR; ++c)
+#pragma unroll
+              for (int e = 0; e < 4; ++e) acc[b][c][e] *= alpha;
+            m[b] = mt;
+          }
+          const float mb = m[b] == -INFINITY ? 0.f : m[b];   // no admissible key yet: every p is exp2(-inf) = 0
+#pragma unroll
+          for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const float p = fast_exp2(s[kb][b][r] - mb);
+              l[b] += p;
+              const int key = 16 * kb + 4 * grp + r;
+              s[kb][b][r] = DROP && !drop_keep(a.drop, rk[b], sKey[buf][key], k0 + key) ? 0.f : p;
+            }
+        }
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) f32_gather<HD>(acc, sV[buf], 16 * kb, s[kb], c16, grp);
+      });
+#pragma unroll
+  for (int b = 0; b < QB; ++b) {
+    float sum = l[b] + __shfl_xor(l[b], 16);
+    sum += __shfl_xor(sum, 32);
+    if (!own.valid[b]) continue;
+    f32_write<HD>(a.o, acc[b], sum > 0.f ? (DROP ? a.drop.inv_keep : 1.f) / sum : 0.f, own.tok[b], H, head, grp);
+    if (grp == 0)
+      a.lse_out[(size_t)head * a.total_q + own.tok[b]] = sum > 0.f ? (m[b] + fast_log2(sum)) * kLn2 : -INFINITY;
   }
-  // Merge in split order: split 0 takes over split 1's partial, then split 2's, ...
-  // (m = -inf marks an empty partial; its output and sum are 0).
-#pragma unroll
-  for (int src = 1; src < S; ++src) {
-    __syncthreads();
-    if (split == src) {
-#pragma unroll
-      for (int i = 0; i < HD; ++i) sAcc[tid][i] = acc[i];
-      sML[tid][0] = m;
-      sML[tid][1] = l;
-    }
-    __syncthreads();
-    if (split == 0) {
-      const float m2 = sML[tid][0], l2 = sML[tid][1];
-      const float mn = fmaxf(m, m2);
-      if (mn != -INFINITY) {
-        const float a1 = fast_exp2(m - mn), a2 = fast_exp2(m2 - mn);
-        l = l * a1 + l2 * a2;
-#pragma unroll
-        for (int i = 0; i < HD; ++i) acc[i] = acc[i] * a1 + sAcc[tid][i] * a2;
-        m = mn;
-      }
-    }
-  }
-  if (split != 0 || !ot.valid) return;
-  storen<HD>(a.o + ((size_t)oi * H + head) * HD, acc, l > 0.f ? (DROP ? a.drop.inv_keep : 1.f) / l : 0.f);
-  a.lse_out[(size_t)head * a.total_q + oi] = l > 0.f ? (m + fast_log2(l)) * kLn2 : -INFINITY;
 }
 
 // fp32 calls with segments of a few queries (the PMA's seeds: the expanded
@@ -1853,97 +1834,170 @@ __global__ __launch_bounds__(256) void attn_dkdv_few_kernel(const AttnFewArgs a)
 
 // dQ = scale * sum_j P_ij (dP_ij - D_i) k_j, P recomputed from the saved LSE.
 template <bool MASKED, int HD, bool DROP>
-__global__ __launch_bounds__(kF32Threads) void attn_dq_f32_kernel(const AttnF32Args a) {
-  __shared__ float4 sK[kTile][HD / 4], sV[kTile][HD / 4];
-  __shared__ int2 sN[kTile];
-  __shared__ uint32_t sKey[DROP ? kTile : 1];   // column keys of the staged keys
-  const int tid = threadIdx.x, H = a.heads;
-  const int item = blockIdx.x / H, head = blockIdx.x - item * H;
+__global__ __launch_bounds__(F32Tile<HD>::kThreads) void attn_dq_f32_kernel(const AttnF32Args a) {
+  using T = F32Tile<HD>;
+  constexpr int NR = T::NR, QB = T::QB, KB = kF32Stage / 16;
+  __shared__ __align__(16) typename T::Rows sK[2], sV[2];
+  __shared__ int2 sN[2][MASKED ? kF32Stage : 1];
+  __shared__ uint32_t sKey[2][DROP ? kF32Stage : 1];   // column keys of the staged keys
+  const int H = a.heads, item = blockIdx.x / H, head = blockIdx.x - item * H;
   if (item >= *a.count) return;
-  const F32Outer ot = f32_outer(a.plan[item], tid);
-  const int oi = ot.oi, oc = ot.oc, phi = ot.phi;
-  const bool valid = ot.valid;
-  float q[HD], g[HD], acc[HD];
-  loadn<HD>(a.q + ((size_t)oc * H + head) * HD, q);
-  loadn<HD>(a.dout + ((size_t)oc * H + head) * HD, g);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c16 = lane & 15, grp = lane >> 4;
+  const F32Own<HD> own(a.plan[item], wave, c16);
+  const int phi = own.phi;
+  f32x4 q[QB][NR], g[QB][NR], acc[QB][NR];
+  int2 node[QB];
+  uint32_t rk[QB];
+  float2 rs[QB];
 #pragma unroll
-  for (int i = 0; i < HD; ++i) acc[i] = 0.f;
-  const float2 rs = a.rows[(size_t)head * a.tq_pad + oc];   // (LSE2, D)
-  const int2 own = MASKED ? a.nodes[oc] : make_int2(0, 0);
-  const uint32_t rk = DROP ? drop_row(a.drop, oc, head) : 0u;
-  for (int k0 = ot.plo; k0 < phi; k0 += kTile) {
-    __syncthreads();
-    stage_rows_f32<HD>(sK, a.k, phi, H, head, k0, tid);
-    stage_rows_f32<HD>(sV, a.v, phi, H, head, k0, tid);
-    if (MASKED && tid < kTile) sN[tid] = k0 + tid < phi ? a.nodes[k0 + tid] : make_int2(-1, -1);
-    if (DROP && tid < kTile) sKey[tid] = drop_col(a.drop, k0 + tid);
-    __syncthreads();
-    if (!valid) continue;
+  for (int b = 0; b < QB; ++b) {
+    f32_owned<HD>(q[b], a.q, own.tok[b], H, head, grp);
+    f32_owned<HD>(g[b], a.dout, own.tok[b], H, head, grp);
 #pragma unroll
-    for (int j = 0; j < kTile; ++j) {
-      const int2 pn = MASKED ? sN[j] : make_int2(0, 0);
-      if (!admissible_f32<MASKED>(k0 + j, phi, oi, pn, own)) continue;
-      const float p = fast_exp2(a.c * dotn<HD>(q, sK[j]) - rs.x);
-      float dp = dotn<HD>(g, sV[j]);
-      if (DROP) dp = drop_keep(a.drop, rk, sKey[j], k0 + j) ? dp * a.drop.inv_keep : 0.f;
-      const float ds = p * (dp - rs.y);
-      axpyn<HD>(ds, sK[j], acc);
-    }
+    for (int c = 0; c < NR; ++c) acc[b][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    rs[b] = a.rows[(size_t)head * a.tq_pad + own.tok[b]];   // (LSE2, D)
+    node[b] = MASKED ? a.nodes[own.tok[b]] : make_int2(0, 0);
+    rk[b] = DROP ? drop_row(a.drop, own.tok[b], head) : 0u;
   }
-  if (!valid) return;
-  storen<HD>(a.dq + ((size_t)oi * H + head) * HD, acc, a.scale);
+  f32x4 rK[T::kPer], rV[T::kPer];
+  int2 rN = make_int2(-1, -1);
+  uint32_t rKey = 0;
+  f32_stages(
+      own.plo, phi, own.live,
+      [&](int t0) {
+        f32_load<HD>(rK, a.k, phi, H, head, t0);
+        f32_load<HD>(rV, a.v, phi, H, head, t0);
+        if (MASKED && tid < kF32Stage) rN = t0 + tid < phi ? a.nodes[t0 + tid] : make_int2(-1, -1);
+        if (DROP && tid < kF32Stage) rKey = drop_col(a.drop, t0 + tid);
+      },
+      [&](int buf) {
+        f32_store<HD>(sK[buf], rK);
+        f32_store<HD>(sV[buf], rV);
+        if (MASKED && tid < kF32Stage) sN[buf][tid] = rN;
+        if (DROP && tid < kF32Stage) sKey[buf][tid] = rKey;
+      },
+      [&](int buf, int k0) {
+        const bool tail = k0 + kF32Stage > phi;
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) {
+          f32x4 x[NR], s[QB], ds[QB];
+          f32_rows<HD>(x, sK[buf], 16 * kb, c16, grp);
+#pragma unroll
+          for (int b = 0; b < QB; ++b) s[b] = f32_product<HD>(x, q[b]);
+          f32_rows<HD>(x, sV[buf], 16 * kb, c16, grp);
+#pragma unroll
+          for (int b = 0; b < QB; ++b) ds[b] = f32_product<HD>(x, g[b]);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int key = 16 * kb + 4 * grp + r;
+            const int2 pn = MASKED ? sN[buf][key] : make_int2(0, 0);
+#pragma unroll
+            for (int b = 0; b < QB; ++b) {
+              float p = fast_exp2(a.c * s[b][r] - rs[b].x);
+              if (MASKED || tail) p = admissible_f32<MASKED>(k0 + key, phi, own.tok[b], pn, node[b]) ? p : 0.f;
+              float dp = ds[b][r];
+              if (DROP) dp = drop_keep(a.drop, rk[b], sKey[buf][key], k0 + key) ? dp * a.drop.inv_keep : 0.f;
+              ds[b][r] = p * (dp - rs[b].y);
+            }
+          }
+          f32_gather<HD>(acc, sK[buf], 16 * kb, ds, c16, grp);
+        }
+      });
+#pragma unroll
+  for (int b = 0; b < QB; ++b)
+    if (own.valid[b]) f32_write<HD>(a.dq, acc[b], a.scale, own.tok[b], H, head, grp);
 }
 
-// dV = sum_i P_ij dO_i, dK = scale * sum_i P_ij (dP_ij - D_i) q_i, one thread
-// per key; the partner tiles are query tiles with their (LSE2, D).
+// dV = sum_i P_ij dO_i, dK = scale * sum_i P_ij (dP_ij - D_i) q_i; the partners are queries with their (LSE2, D).
 template <bool MASKED, int HD, bool DROP>
-__global__ __launch_bounds__(kF32Threads) void attn_dkdv_f32_kernel(const AttnF32Args a) {
-  __shared__ float4 sQ[kTile][HD / 4], sG[kTile][HD / 4];
-  __shared__ float2 sR[kTile];
-  __shared__ int2 sN[kTile];
-  __shared__ uint32_t sKey[DROP ? kTile : 1];   // row keys of the staged queries
-  const int tid = threadIdx.x, H = a.heads;
-  const int item = blockIdx.x / H, head = blockIdx.x - item * H;
+__global__ __launch_bounds__(F32Tile<HD>::kThreads) void attn_dkdv_f32_kernel(const AttnF32Args a) {
+  using T = F32Tile<HD>;
+  constexpr int NR = T::NR, QB = T::QB, KB = kF32Stage / 16;
+  __shared__ __align__(16) typename T::Rows sQ[2], sG[2];
+  __shared__ __align__(16) float sL[2][kF32Stage], sD[2][kF32Stage];
+  __shared__ int2 sN[2][MASKED ? kF32Stage : 1];
+  __shared__ uint32_t sKey[2][DROP ? kF32Stage : 1];   // row keys of the staged queries
+  const int H = a.heads, item = blockIdx.x / H, head = blockIdx.x - item * H;
   if (item >= *a.count) return;
-  const F32Outer ot = f32_outer(a.plan[item], tid);
-  const int oi = ot.oi, oc = ot.oc, phi = ot.phi;
-  const bool valid = ot.valid;
-  float kx[HD], vx[HD], dk[HD], dv[HD];
-  loadn<HD>(a.k + ((size_t)oc * H + head) * HD, kx);
-  loadn<HD>(a.v + ((size_t)oc * H + head) * HD, vx);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c16 = lane & 15, grp = lane >> 4;
+  const F32Own<HD> own(a.plan[item], wave, c16);
+  const int phi = own.phi;
+  f32x4 kx[QB][NR], vx[QB][NR], dk[QB][NR], dv[QB][NR];
+  int2 node[QB];
+  uint32_t ck[QB];
 #pragma unroll
-  for (int i = 0; i < HD; ++i) dk[i] = dv[i] = 0.f;
-  const int2 own = MASKED ? a.nodes[oc] : make_int2(0, 0);
-  const uint32_t ck = DROP ? drop_col(a.drop, oc) : 0u;
-  for (int q0 = ot.plo; q0 < phi; q0 += kTile) {
-    __syncthreads();
-    stage_rows_f32<HD>(sQ, a.q, phi, H, head, q0, tid);
-    stage_rows_f32<HD>(sG, a.dout, phi, H, head, q0, tid);
-    if (tid < kTile) {
-      const bool in = q0 + tid < phi;
-      sR[tid] = in ? a.rows[(size_t)head * a.tq_pad + q0 + tid] : make_float2(INFINITY, 0.f);
-      if (MASKED) sN[tid] = in ? a.nodes[q0 + tid] : make_int2(-1, -1);
-      if (DROP) sKey[tid] = drop_row(a.drop, q0 + tid, head);
-    }
-    __syncthreads();
-    if (!valid) continue;
+  for (int b = 0; b < QB; ++b) {
+    f32_owned<HD>(kx[b], a.k, own.tok[b], H, head, grp);
+    f32_owned<HD>(vx[b], a.v, own.tok[b], H, head, grp);
 #pragma unroll
-    for (int i = 0; i < kTile; ++i) {
-      const int2 pn = MASKED ? sN[i] : make_int2(0, 0);
-      if (!admissible_f32<MASKED>(q0 + i, phi, oi, pn, own)) continue;
-      const float2 rs = sR[i];
-      const float p = fast_exp2(a.c * dotn<HD>(kx, sQ[i]) - rs.x);
-      const bool keep = !DROP || drop_keep(a.drop, sKey[i], ck, oc);
-      axpyn<HD>(keep ? p : 0.f, sG[i], dv);
-      float dp = dotn<HD>(vx, sG[i]);
-      if (DROP) dp = keep ? dp * a.drop.inv_keep : 0.f;
-      const float ds = p * (dp - rs.y);
-      axpyn<HD>(ds, sQ[i], dk);
-    }
+    for (int c = 0; c < NR; ++c) dk[b][c] = dv[b][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    node[b] = MASKED ? a.nodes[own.tok[b]] : make_int2(0, 0);
+    ck[b] = DROP ? drop_col(a.drop, own.tok[b]) : 0u;
   }
-  if (!valid) return;
-  storen<HD>(a.dv + ((size_t)oi * H + head) * HD, dv, DROP ? a.drop.inv_keep : 1.f);
-  storen<HD>(a.dk + ((size_t)oi * H + head) * HD, dk, a.scale);
+  f32x4 rQ[T::kPer], rG[T::kPer];
+  float2 rR = make_float2(INFINITY, 0.f);
+  int2 rN = make_int2(-1, -1);
+  uint32_t rKey = 0;
+  f32_stages(
+      own.plo, phi, own.live,
+      [&](int t0) {
+        f32_load<HD>(rQ, a.q, phi, H, head, t0);
+        f32_load<HD>(rG, a.dout, phi, H, head, t0);
+        if (tid < kF32Stage) {
+          const bool in = t0 + tid < phi;
+          rR = in ? a.rows[(size_t)head * a.tq_pad + t0 + tid] : make_float2(INFINITY, 0.f);
+          if (MASKED) rN = in ? a.nodes[t0 + tid] : make_int2(-1, -1);
+          if (DROP) rKey = drop_row(a.drop, t0 + tid, head);
+        }
+      },
+      [&](int buf) {
+        f32_store<HD>(sQ[buf], rQ);
+        f32_store<HD>(sG[buf], rG);
+        if (tid < kF32Stage) {
+          sL[buf][tid] = rR.x;
+          sD[buf][tid] = rR.y;
+          if (MASKED) sN[buf][tid] = rN;
+          if (DROP) sKey[buf][tid] = rKey;
+        }
+      },
+      [&](int buf, int q0) {
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) {
+          f32x4 x[NR], s[QB], ds[QB];
+          f32_rows<HD>(x, sQ[buf], 16 * kb, c16, grp);
+#pragma unroll
+          for (int b = 0; b < QB; ++b) s[b] = f32_product<HD>(x, kx[b]);
+          f32_rows<HD>(x, sG[buf], 16 * kb, c16, grp);
+#pragma unroll
+          for (int b = 0; b < QB; ++b) ds[b] = f32_product<HD>(x, vx[b]);
+          const f32x4 lse2 = ldsf4(&sL[buf][16 * kb + 4 * grp]), d = ldsf4(&sD[buf][16 * kb + 4 * grp]);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int qi = 16 * kb + 4 * grp + r;
+            const int2 pn = MASKED ? sN[buf][qi] : make_int2(0, 0);
+#pragma unroll
+            for (int b = 0; b < QB; ++b) {
+              float p = fast_exp2(a.c * s[b][r] - lse2[r]);   // a query past the range has LSE2 = inf
+              if (MASKED) p = admissible_f32<true>(q0 + qi, phi, own.tok[b], pn, node[b]) ? p : 0.f;
+              const bool keep = !DROP || drop_keep(a.drop, sKey[buf][qi], ck[b], own.tok[b]);
+              float dp = ds[b][r];
+              if (DROP) dp = keep ? dp * a.drop.inv_keep : 0.f;
+              ds[b][r] = p * (dp - d[r]);
+              s[b][r] = keep ? p : 0.f;
+            }
+          }
+          f32_gather<HD>(dv, sG[buf], 16 * kb, s, c16, grp);
+          f32_gather<HD>(dk, sQ[buf], 16 * kb, ds, c16, grp);
+        }
+      });
+#pragma unroll
+  for (int b = 0; b < QB; ++b)
+    if (own.valid[b]) {
+      f32_write<HD>(a.dv, dv[b], DROP ? a.drop.inv_keep : 1.f, own.tok[b], H, head, grp);
+      f32_write<HD>(a.dk, dk[b], a.scale, own.tok[b], H, head, grp);
+    }
 }
 
 // ======================================================================== prep kernel
@@ -2445,24 +2499,14 @@ GraphAttnArgs edge_gather_args(const void* plan, const void* q, const void* k, c
 }
 
 // KERNEL<false, HD, DROP> (the fp32 kernels without a mask) for head dim 16, 24, 32 or 64.
-#define ESA_F32_LAUNCH_HD(KERNEL, D, hd, grid, st, a)                                                \
-  do {                                                                                               \
-    if (hd == 16) hipLaunchKernelGGL((KERNEL<false, 16, D>), grid, dim3(kF32Threads), 0, st, a);      \
-    else if (hd == 24) hipLaunchKernelGGL((KERNEL<false, 24, D>), grid, dim3(kF32Threads), 0, st, a); \
-    else if (hd == 32) hipLaunchKernelGGL((KERNEL<false, 32, D>), grid, dim3(kF32Threads), 0, st, a); \
-    else hipLaunchKernelGGL((KERNEL<false, 64, D>), grid, dim3(kF32Threads), 0, st, a);              \
-  } while (0)
-constexpr unsigned kF32FwdThreads(int hd) { return kF32Threads * (hd >= 64 ? f32_splits<64>() : f32_splits<16>()); }
-#define ESA_F32_FWD_HD(D, hd, grid, st, a)                                                                 \
-  do {                                                                                                     \
-    if (hd == 16)                                                                                          \
-      hipLaunchKernelGGL((attn_fwd_f32_kernel<false, 16, D>), grid, dim3(kF32FwdThreads(16)), 0, st, a);    \
-    else if (hd == 24)                                                                                     \
-      hipLaunchKernelGGL((attn_fwd_f32_kernel<false, 24, D>), grid, dim3(kF32FwdThreads(24)), 0, st, a);    \
-    else if (hd == 32)                                                                                     \
-      hipLaunchKernelGGL((attn_fwd_f32_kernel<false, 32, D>), grid, dim3(kF32FwdThreads(32)), 0, st, a);    \
-    else                                                                                                   \
-      hipLaunchKernelGGL((attn_fwd_f32_kernel<false, 64, D>), grid, dim3(kF32FwdThreads(64)), 0, st, a);    \
+#define ESA_F32_LAUNCH_K(KERNEL, MASKED, HD, D, grid, st, a) \
+  hipLaunchKernelGGL((KERNEL<MASKED, HD, D>), grid, dim3(F32Tile<HD>::kThreads), 0, st, a)
+#define ESA_F32_LAUNCH_HD(KERNEL, D, hd, grid, st, a)                        \
+  do {                                                                       \
+    if (hd == 16) ESA_F32_LAUNCH_K(KERNEL, false, 16, D, grid, st, a);       \
+    else if (hd == 24) ESA_F32_LAUNCH_K(KERNEL, false, 24, D, grid, st, a);  \
+    else if (hd == 32) ESA_F32_LAUNCH_K(KERNEL, false, 32, D, grid, st, a);  \
+    else ESA_F32_LAUNCH_K(KERNEL, false, 64, D, grid, st, a);                \
   } while (0)
 // Unmasked fp32 calls whose max_seqlen_q is 1..kFewQueries take the few-query kernels (the forward at
 // every head dim, the backward at head dims up to kFewBwdMaxHd: a dK/dV thread holds six rows of the head dim).
@@ -2501,11 +2545,6 @@ AttnFewArgs few_args(const void* q, const void* k, const void* v, const int* cu_
   return f;
 }
 
-#define ESA_F32_FWD_LAUNCH(hd, drop, grid, st, a)  \
-  do {                                             \
-    if (drop) ESA_F32_FWD_HD(true, hd, grid, st, a); \
-    else ESA_F32_FWD_HD(false, hd, grid, st, a);     \
-  } while (0)
 #define ESA_F32_LAUNCH(KERNEL, hd, drop, grid, st, a)                                                \
   do {                                                                                               \
     if (drop) ESA_F32_LAUNCH_HD(KERNEL, true, hd, grid, st, a);                                     \
@@ -2697,9 +2736,9 @@ int esa_varlen_attn_fwd(const void* q, const void* k, const void* v, const int* 
     const dim3 fgrid((unsigned)(groups_of(total_q) + batch) * (unsigned)heads);
     if (masked)   // head_dim 16 without dropout (the rest take the gather kernels)
       ESA_TIMED(esa_profile::kAttnFwdMasked, st,
-                hipLaunchKernelGGL((attn_fwd_f32_kernel<true, 16, false>), fgrid, dim3(kF32FwdThreads(16)), 0, st, a));
+                ESA_F32_LAUNCH_K(attn_fwd_f32_kernel, true, 16, false, fgrid, st, a));
     else
-      ESA_TIMED(esa_profile::kAttnFwd, st, ESA_F32_FWD_LAUNCH(head_dim, drop, fgrid, st, a));
+      ESA_TIMED(esa_profile::kAttnFwd, st, ESA_F32_LAUNCH(attn_fwd_f32_kernel, head_dim, drop, fgrid, st, a));
     ESA_LAUNCH_CHECK();
     return ESA_OK;
   }
@@ -2881,14 +2920,14 @@ int esa_varlen_attn_bwd(const void* dout, const void* q, const void* k, const vo
     const dim3 fqgrid((unsigned)(groups_of(total_q) + batch) * (unsigned)heads);
     if (masked)   // head_dim 16 without dropout (the rest take the gather kernels)
       ESA_TIMED(esa_profile::kAttnBwdDkdvMasked, st,
-                hipLaunchKernelGGL((attn_dkdv_f32_kernel<true, 16, false>), fkgrid, dim3(kF32Threads), 0, st, a));
+                ESA_F32_LAUNCH_K(attn_dkdv_f32_kernel, true, 16, false, fkgrid, st, a));
     else
       ESA_TIMED(esa_profile::kAttnBwdDkdv, st, ESA_F32_LAUNCH(attn_dkdv_f32_kernel, head_dim, drop, fkgrid, st, a));
     ESA_LAUNCH_CHECK();
     a.plan = pa.plan_q; a.count = pa.count_q;
     if (masked)
       ESA_TIMED(esa_profile::kAttnBwdDqMasked, st,
-                hipLaunchKernelGGL((attn_dq_f32_kernel<true, 16, false>), fqgrid, dim3(kF32Threads), 0, st, a));
+                ESA_F32_LAUNCH_K(attn_dq_f32_kernel, true, 16, false, fqgrid, st, a));
     else
       ESA_TIMED(esa_profile::kAttnBwdDq, st, ESA_F32_LAUNCH(attn_dq_f32_kernel, head_dim, drop, fqgrid, st, a));
     ESA_LAUNCH_CHECK();
