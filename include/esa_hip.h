@@ -476,6 +476,35 @@ ESA_API int esa_linear_f32(const float* x, int rows, int in_features, int n_out,
                    const float* const* weight, const float* const* bias, float* const* y,
                    const int* out_features, void* stream);
 
+/* The blocks' Linears with what follows them, over x [rows, in] (ESA_F32 or */
+/* ESA_BF16; weights, biases, outputs and `other` of that type, sums fp32):  */
+/*   PLAIN  y_i = x W_i^T + b_i for n (1-3) weights W_i [out_i, in]          */
+/*   MISH   y_0 = z = x W^T + b, result = mish(z)        (mlp_utils.py:18-37) */
+/*   MAB    y_0 = z, result = other + mish(z)            (esa/mha.py:87), or  */
+/*          with residual (fp32): result (fp32) = residual + that, rounded    */
+/*          first                             (esa/masked_layers.py:471-472)  */
+/*   ADD    result (fp32) = residual + y, y rounded first          (:478-483) */
+/* (n = 1 but for PLAIN; y_0 may be null in MISH and MAB: z is not kept.)     */
+/* in and, in PLAIN, every tensor as nn.Linear's; in % 32 == 0, out_i % 8 ==  */
+/* 0 (fp32: 4), all pointers 16-byte aligned; weight, bias, y and             */
+/* out_features are host arrays of n entries, biases may be null.             */
+#define ESA_LINEAR_PLAIN 0
+#define ESA_LINEAR_MISH 1
+#define ESA_LINEAR_MAB 2
+#define ESA_LINEAR_ADD 3
+ESA_API int esa_linear_fwd(const void* x, long long rows, int in_features, int dtype, int n,
+                   const void* const* weight, const void* const* bias, void* const* y,
+                   const int* out_features, int epilogue, const void* other,
+                   const float* residual, void* result, void* stream);
+
+/* Input gradients of those Linears: dx [rows, in] = sum over n (1-3) of     */
+/* g_i W_i (g_i [rows, out_i]), plus base where it is not null, or times      */
+/* mish'(mish_z) where that is not null (not both); summed in fp32 and rounded */
+/* once.  out_i % 32 == 0, in % 8 == 0 (fp32: 4), pointers 16-byte aligned.   */
+ESA_API int esa_linear_dx(const void* const* g, const void* const* weight, int n, long long rows,
+                   const int* out_features, int in_features, int dtype, const void* base,
+                   const void* mish_z, void* dx, void* stream);
+
 /* Weight and bias gradients of n (1-3) of the blocks' Linear layers over    */
 /* one batch of rows (the autograd of nn.Linear, esa/mha.py:12-15,           */
 /* esa/mlp_utils.py:18-37): dW_i = g_i^T x_i [out_i, in_i] and, where db_i   */
@@ -502,7 +531,7 @@ ESA_API int esa_weight_grad(long long rows, int n, const void* const* g, const v
 /* launch count per kernel id (capacity >= ESA_PROFILE_KERNELS) and clears   */
 /* the record.  Not for concurrent use from several threads.                 */
 /* ------------------------------------------------------------------------ */
-#define ESA_PROFILE_KERNELS 24
+#define ESA_PROFILE_KERNELS 25
 ESA_API int esa_profile_enable(int on);
 ESA_API int esa_profile_collect(float* total_ms, int* launches, int capacity);
 ESA_API const char* esa_profile_kernel_name(int kernel);

@@ -103,6 +103,12 @@ _PROTOS = {
     # x rows in n_out | weight[] bias[] y[] out_features[] stream
     "esa_linear_f32": (_c_int, [_vp, _c_int, _c_int, _c_int, ctypes.POINTER(_vp), ctypes.POINTER(_vp),
                                 ctypes.POINTER(_vp), ctypes.POINTER(_c_int), _vp]),
+    # x rows in dtype n | w[] b[] y[] out_features[] | epilogue other residual result stream
+    "esa_linear_fwd": (_c_int, [_vp, _c_i64, _c_int, _c_int, _c_int, ctypes.POINTER(_vp), ctypes.POINTER(_vp),
+                                ctypes.POINTER(_vp), ctypes.POINTER(_c_int), _c_int, _vp, _vp, _vp, _vp]),
+    # g[] w[] n rows | out_features[] in dtype | base mish_z dx stream
+    "esa_linear_dx": (_c_int, [ctypes.POINTER(_vp), ctypes.POINTER(_vp), _c_int, _c_i64, ctypes.POINTER(_c_int), _c_int,
+                               _c_int, _vp, _vp, _vp, _vp]),
     "esa_weight_grad_workspace_size": (_c_int, [_c_i64, _c_int, ctypes.POINTER(_c_int), ctypes.POINTER(_c_int), _c_int,
                                                 ctypes.POINTER(_c_sz)]),
     # rows n | g[] x[] out_features[] in_features[] dtype | dw[] db[] ws bytes stream
@@ -116,7 +122,7 @@ _PROTOS = {
     "esa_profile_kernel_name": (ctypes.c_char_p, [_c_int]),
 }
 
-PROFILE_KERNELS = 24
+PROFILE_KERNELS = 25
 
 _lock = threading.Lock()
 _lib = None

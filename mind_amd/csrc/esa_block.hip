@@ -26,6 +26,7 @@
 // fp32 residual and the bf16 GEMM input); the backward takes the gradients of
 // both outputs and sums them, so no cast or add kernel runs beside it.
 #include "esa_common.h"
+#include "esa_mish.h"
 #include "esa_profile.h"
 #include "../../include/esa_hip.h"
 
@@ -33,24 +34,6 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kUnroll = 4;
-constexpr float kMishLinear = 20.f;   // above: tanh(softplus(x)) == 1 in fp32
-
-DEVI float mish_f(float x) {
-  if (x > kMishLinear) return x;
-  const float w = fast_exp2(x * kLog2e);
-  const float n = w * (w + 2.f);
-  return x * n * __builtin_amdgcn_rcpf(n + 2.f);
-}
-
-// At x = +inf the slope is NaN, as torch's mish backward gives (inf * 0);
-// x is multiplied last so that a huge negative x meets w = 0 (slope 0).
-DEVI float mish_grad_f(float x) {
-  if (x > kMishLinear) return x < INFINITY ? 1.f : NAN;
-  const float w = fast_exp2(x * kLog2e);
-  const float n = w * (w + 2.f);
-  const float r = __builtin_amdgcn_rcpf(n + 2.f);
-  return n * r + x * (4.f * w * (1.f + w) * (r * r));
-}
 
 template <typename T> struct Chunk;
 template <> struct Chunk<float> {

@@ -30,6 +30,7 @@ enum Kernel : int {
   kAttnEdgeOverflow,  // edge-mask walk kernels over the overflow groups
   kSegmentMinMax,     // segmented minimum / maximum with argument
   kLinearF32,         // fp32 Linear layers of the blocks
+  kLinearGemm,        // the blocks' Linears with their epilogues, and their input gradients
   kWeightGrad,        // weight and bias gradients of the blocks' Linear layers
   kNumKernels
 };

@@ -36,7 +36,7 @@
 #include <algorithm>
 #include <type_traits>
 
-#include "esa_attn_tiles.h"
+#include "esa_stage.h"
 #include "esa_profile.h"
 #include "../../include/esa_hip.h"
 
@@ -60,59 +60,6 @@ struct WgradArgs {
 
 struct ReducePart { const float* src; float* dst; int64_t n; int block0; };
 struct ReduceArgs { int splits, n; ReducePart p[2 * kMaxPairs]; };
-
-DEVI f32x16 mfma32x2(float a, float b, const f32x16& c) {
-  return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
-}
-
-// Staging and operand reads of one operand's stage, [tokens][COLS].
-template <typename T, int COLS>
-struct Rows;
-template <int COLS>
-struct Rows<bf16, COLS> {
-  static constexpr int kTok = 32, kSteps = 2;   // tokens per stage, MFMA k steps of it
-  static constexpr int kBytes = kTok * COLS * 2, kLoads = kBytes / 4096;   // 1 KB LDS-direct loads per wave
-  typedef bf16x8 Op;
-  // lane's byte offset (in the stage's 1 KB load j) from the stage's first row
-  static DEVI uint32_t offset(int j, int lane, int col0, int cols) {
-    constexpr int kChunks = COLS / 8;   // 16-byte chunks per row
-    const int tok = (64 * j + lane) / kChunks, slot = (64 * j + lane) % kChunks, c = col0 + 8 * (slot ^ (2 * (tok & 3)));
-    return c < cols ? (uint32_t)(tok * cols + c) * 2u : 0xfffffff0u;
-  }
-  // features c0 .. c0 + 31 over the 16 tokens of step k
-  static DEVI Op operand(const char* lds, int c0, int k, int lane) {
-    const int i = lane & 15, grp = lane >> 4;
-    const int tok = 16 * k + 8 * (grp >> 1) + (i >> 2), c = c0 + 16 * (grp & 1) + 4 * (i & 3);
-    const int slot = (c >> 3) ^ (2 * (tok & 3));
-    const bf16* p = reinterpret_cast<const bf16*>(lds) + tok * COLS + slot * 8 + (c & 4);
-    const bf16x4 lo = lds_tr4(p), hi = lds_tr4(p + 4 * COLS);   // tokens + 4: the same slot
-    return bf16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-  }
-  static DEVI f32x16 product(const Op& a, const Op& b, const f32x16& c) { return mfma32(a, b, c); }
-  static DEVI float add_tokens(const Op& a, float s) {
-    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-    const bf16x2 one = {(bf16)1.f, (bf16)1.f};
-#pragma unroll
-    for (int e = 0; e < 8; e += 2) s = __builtin_amdgcn_fdot2_f32_bf16(bf16x2{a[e], a[e + 1]}, one, s, false);
-    return s;
-  }
-};
-template <int COLS>
-struct Rows<float, COLS> {
-  static constexpr int kTok = 16, kSteps = 8;
-  static constexpr int kBytes = kTok * COLS * 4, kLoads = kBytes / 4096;
-  typedef float Op;
-  static DEVI uint32_t offset(int j, int lane, int col0, int cols) {
-    constexpr int kChunks = COLS / 4;
-    const int tok = (64 * j + lane) / kChunks, c = col0 + 4 * ((64 * j + lane) % kChunks);
-    return c < cols ? (uint32_t)(tok * cols + c) * 4u : 0xfffffff0u;
-  }
-  static DEVI Op operand(const char* lds, int c0, int k, int lane) {
-    return reinterpret_cast<const float*>(lds)[(2 * k + (lane >> 5)) * COLS + c0 + (lane & 31)];
-  }
-  static DEVI f32x16 product(const Op& a, const Op& b, const f32x16& c) { return mfma32x2(a, b, c); }
-  static DEVI float add_tokens(const Op& a, float s) { return s + a; }
-};
 
 template <typename T, int NV>
 __global__ __launch_bounds__(256, 2) void wgrad_kernel(const WgradArgs a) {

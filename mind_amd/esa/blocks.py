@@ -25,11 +25,12 @@ import torch
 from torch import nn
 
 from . import attention
-from .activations import Mish, mab_residual_backward, mab_residual_forward, mish_backward, mish_forward
+from .activations import Mish, mab_residual_backward, mish_backward
 from .attention import HEAD_DIMS, attn_bwd, attn_fwd, pma_backward, pma_forward
-from .eager import call, plain
+from .eager import Unrecorded, call, plain
 from .layer_norm import f32_values, ln_backward, ln_forward, supported
-from .linear import cast_param, hookless, linear_fwd, weight_bias_grads
+from .linear import (cast_param, hookless, input_grad, linear_outputs, linear_then_add, linear_then_mab,
+                     linear_then_mish, weight_bias_grads)
 from .mlp_utils import SmallMLP
 
 
@@ -84,6 +85,12 @@ class _Setup:
         self.dropout = (dropout_p, attention.draw_dropout_seed() if dropout_p > 0.0 else 0)
         self.again = again   # (x, seed) -> the block's output through the separate functions
         self.mask = {}
+        # whole stages of the fused products both ways, for the parameters themselves or (amp) their contiguous casts
+        layers = (mab.fc_q, mab.fc_k, mab.fc_v, mab.fc_o, *mlp)
+        self.fused = all(fc.weight.dim() == 2 and fc.weight.is_contiguous() and max(fc.weight.shape) <= 16384
+                         and fc.weight.shape[0] % 32 == 0 and fc.weight.shape[1] % 32 == 0
+                         and (self.amp or all(t is None or (t.is_contiguous() and t.data_ptr() % 16 == 0)
+                                              for t in (fc.weight, fc.bias))) for fc in layers)
 
 
 def _rebuilt(setup, inputs, g, needs):
@@ -103,30 +110,30 @@ def _norm(setup, x, w, b, eps, full):
     return y, y, stats
 
 
-def _mlp_forward(x, params):
-    """Linear (-> Mish -> Linear)*: (output, [the tensors _mlp_backward takes: input, weight and, before a Mish, z])."""
+def _mlp_forward(x, params, residual, keep, fused):
+    """Linear (-> Mish -> Linear)* plus the residual: (output, [the tensors _mlp_backward takes: a layer's input and
+    weight and, before a Mish, z])."""
     saved = []
     for i in range(0, len(params), 2):
         w, b = cast_param(params[i], x.dtype), cast_param(params[i + 1], x.dtype)
-        (z,) = linear_fwd(x, [(w, b)])
         saved += (x, w)
         if i + 2 < len(params):
+            z, x = linear_then_mish(x, w, b, keep, fused)
             saved.append(z)
-            x = mish_forward(z)
-    return z, saved
+    if residual.dtype == torch.float32:
+        return linear_then_add(x, w, b, residual, fused), saved
+    return linear_outputs(x, [(w, b)], fused)[0] + residual, saved
 
 
-def _mlp_backward(g, saved, needs):
+def _mlp_backward(g, saved, needs, fused):
     """(dx, the parameters' gradients) for the output gradient g in the compute dtype."""
     grads = [None] * len(needs)
     layers = [saved[i:i + 3] for i in range(0, len(saved), 3)]
     for i in range(len(layers) - 1, -1, -1):
         x, w = layers[i][:2]
-        if len(layers[i]) == 3:
-            g = mish_backward(layers[i][2], g)
         ((grads[2 * i], grads[2 * i + 1]),) = weight_bias_grads([(g, x)], needs[2 * i:2 * i + 1],
                                                                 needs[2 * i + 1:2 * i + 2])
-        g = g.mm(w)
+        g = input_grad([(g, w)], fused, mish_z=layers[i - 1][2] if i else None)
     return g, grads
 
 
@@ -134,22 +141,20 @@ class _SabBlock(torch.autograd.Function):
     @staticmethod
     def forward(ctx, setup, x, *params):
         ln_w, ln_b, wq, bq, wk, bk, wv, bv, wo, bo = params[:10]
-        t, d, h = x.shape[0], x.shape[1], setup.heads
+        t, d, h, keeps = x.shape[0], x.shape[1], setup.heads, not isinstance(ctx, Unrecorded)
         x1, xm, stats = _norm(setup, x, ln_w, ln_b, setup.eps[0], True)
         weights = [cast_param(p, setup.dt) for p in (wq, wk, wv, wo)]
         biases = [cast_param(p, setup.dt) for p in (bq, bk, bv, bo)]
-        q, k, v = (y.view(t, h, d // h) for y in linear_fwd(xm, list(zip(weights[:3], biases[:3]))))
+        q, k, v = (y.view(t, h, d // h) for y in linear_outputs(xm, list(zip(weights[:3], biases[:3])), setup.fused))
         cu, n, (p, seed) = setup.cu, setup.max_items, setup.dropout
         o, lse = attn_fwd(q, k, v, cu, cu, n, n, 1.0 / math.sqrt(d // h), dropout_p=p, dropout_seed=seed, **setup.mask)
-        (z,) = linear_fwd(o.view(t, d), [(weights[3], biases[3])])
-        x2 = mab_residual_forward(z, o, x1)
+        z, x2 = linear_then_mab(o.view(t, d), weights[3], biases[3], x1, keeps, setup.fused)
         keep = [x, f32_values(ln_w), stats, xm, q, k, v, o, lse, z] + weights
         out = x2
         if setup.n_mlp:
             ln_w2, ln_b2 = params[10:12]
             _, ym, stats2 = _norm(setup, x2, ln_w2, ln_b2, setup.eps[1], False)
-            y, saved = _mlp_forward(ym, params[12:])
-            out = y + x2
+            out, saved = _mlp_forward(ym, params[12:], x2, keeps, setup.fused)
             keep += [x2, f32_values(ln_w2), stats2] + saved
         ctx.setup, ctx.n_keep, ctx.mask_keys = setup, len(keep), list(setup.mask)
         ctx.save_for_backward(*keep, cu, *setup.mask.values(), *params)
@@ -168,20 +173,18 @@ class _SabBlock(torch.autograd.Function):
         mlp_grads = ()
         if setup.n_mlp:
             x2, ln_w2, stats2 = tensors[14:17]
-            dy, mlp_grads = _mlp_backward(g.to(setup.dt), tensors[17:ctx.n_keep], needs[13:])
+            dy, mlp_grads = _mlp_backward(g.to(setup.dt), tensors[17:ctx.n_keep], needs[13:], setup.fused)
             g, dw, db = ln_backward(x2, ln_w2, stats2, None if setup.amp else dy, dy if setup.amp else None, g,
                                     needs[11], needs[12])
             mlp_grads = (dw, db, *mlp_grads)
         dz, g_o = mab_residual_backward(z, g)
-        do = torch.addmm(g_o, dz, wo).view_as(o)
+        do = input_grad([(dz, wo)], setup.fused, g_o).view_as(o)
         grads_o = weight_bias_grads([(dz, o.view(t, d))], needs[9:10], needs[10:11])
         n, (p, seed) = setup.max_items, setup.dropout
         gq, gk, gv = (y.view(t, d) for y in attn_bwd(do, q, k, v, o, lse, cu, cu, n, n, 1.0 / math.sqrt(d // setup.heads),
                                                      dropout_p=p, dropout_seed=seed, **mask))
         # fp32: the norm's one output feeds the projections and the residual, whose gradient g starts the sum
-        dxm = gq.mm(wq) if setup.amp else torch.addmm(g, gq, wq)
-        dxm.addmm_(gk, wk)
-        dxm.addmm_(gv, wv)
+        dxm = input_grad([(gq, wq), (gk, wk), (gv, wv)], setup.fused, None if setup.amp else g)
         grads = weight_bias_grads([(gq, xm), (gk, xm), (gv, xm)], needs[3:9:2], needs[4:9:2])
         dx, dw, db = ln_backward(x, ln_w, stats, g if setup.amp else dxm, dxm if setup.amp else None, None, needs[1],
                                  needs[2])
@@ -211,24 +214,22 @@ class _PmaBlock(torch.autograd.Function):
     @staticmethod
     def forward(ctx, setup, x, seeds, *params):
         ln_w, ln_b, wq, bq, wk, bk, wv, bv, wo, bo = params[:10]
-        (k_seeds, d), h = seeds.shape[1:], setup.heads
+        (k_seeds, d), h, keeps = seeds.shape[1:], setup.heads, not isinstance(ctx, Unrecorded)
         _, xm, stats = _norm(setup, x, ln_w, ln_b, setup.eps[0], False)
         s = cast_param(seeds, setup.dt).reshape(k_seeds, d)
         weights = [cast_param(p, setup.dt) for p in (wq, wk, wv, wo)]
         biases = [cast_param(p, setup.dt) for p in (bq, bk, bv, bo)]
-        (q,) = linear_fwd(s, [(weights[0], biases[0])])
-        k, v = linear_fwd(xm, list(zip(weights[1:3], biases[1:3])))
+        (q,) = linear_outputs(s, [(weights[0], biases[0])], setup.fused)
+        k, v = linear_outputs(xm, list(zip(weights[1:3], biases[1:3])), setup.fused)
         q, k, v = (y.view(-1, h, d // h) for y in (q, k, v))
         o, lse = pma_forward(q, k, v, setup.cu, setup.max_items, 1.0 / math.sqrt(d // h), *setup.dropout)
-        (z,) = linear_fwd(o.view(-1, d), [(weights[3], biases[3])])
-        x2 = mish_forward(z, o.view(-1, d))
+        z, x2 = linear_then_mab(o.view(-1, d), weights[3], biases[3], None, keeps, setup.fused)
         keep = [x, f32_values(ln_w), stats, xm, s, q, k, v, o, lse, z] + weights
         out = x2
         if setup.n_mlp:
             ln_w2, ln_b2 = params[10:12]
             _, ym, stats2 = _norm(setup, x2, ln_w2, ln_b2, setup.eps[1], False)
-            y, saved = _mlp_forward(ym, params[12:])
-            out = y + x2
+            out, saved = _mlp_forward(ym, params[12:], x2, keeps, setup.fused)
             keep += [x2, f32_values(ln_w2), stats2] + saved
         ctx.setup, ctx.n_keep = setup, len(keep)
         ctx.save_for_backward(*keep, setup.cu, seeds, *params)
@@ -246,18 +247,17 @@ class _PmaBlock(torch.autograd.Function):
         mlp_grads = ()
         if setup.n_mlp:
             x2, ln_w2, stats2 = tensors[15:18]
-            dy, mlp_grads = _mlp_backward(g, tensors[18:ctx.n_keep], needs[14:])
+            dy, mlp_grads = _mlp_backward(g, tensors[18:ctx.n_keep], needs[14:], setup.fused)
             g, dw, db = ln_backward(x2, ln_w2, stats2, None if setup.amp else dy, dy if setup.amp else None, g,
                                     needs[12], needs[13])
             mlp_grads = (dw, db, *mlp_grads)
         dz = mish_backward(z, g)
-        do = torch.addmm(g, dz, wo).view_as(o)
+        do = input_grad([(dz, wo)], setup.fused, g).view_as(o)
         grads_o = weight_bias_grads([(dz, o.view(-1, d))], needs[10:11], needs[11:12])
         gq, gk, gv = (y.view(-1, d) for y in pma_backward(do, q, k, v, o, lse, cu, setup.max_items,
                                                           1.0 / math.sqrt(d // setup.heads), *setup.dropout))
-        dseeds = gq.mm(wq).view(seeds.shape).to(seeds.dtype) if needs[1] else None
-        dxm = gk.mm(wk)
-        dxm.addmm_(gv, wv)
+        dseeds = input_grad([(gq, wq)], setup.fused).view(seeds.shape).to(seeds.dtype) if needs[1] else None
+        dxm = input_grad([(gk, wk), (gv, wv)], setup.fused)
         grads = (weight_bias_grads([(gq, s)], needs[4:5], needs[5:6])
                  + weight_bias_grads([(gk, xm), (gv, xm)], needs[6:10:2], needs[7:10:2]))
         dx, dw, db = ln_backward(x, ln_w, stats, None if setup.amp else dxm, dxm if setup.amp else None, None, needs[2],

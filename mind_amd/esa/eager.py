@@ -33,7 +33,7 @@ def records(*args) -> bool:
     return torch.is_grad_enabled() and any(isinstance(a, torch.Tensor) and a.requires_grad for a in args)
 
 
-class _Unrecorded:
+class Unrecorded:
     """The context of a forward that autograd does not record: nothing is kept."""
 
     needs_input_grad = ()
@@ -51,5 +51,5 @@ class _Unrecorded:
 def call(function, *args):
     """``function.apply(*args)`` of an autograd function; its forward alone where nothing records or traces it."""
     if not records(*args) and plain(*args):
-        return function.forward(_Unrecorded(), *args)
+        return function.forward(Unrecorded(), *args)
     return function.apply(*args)

@@ -86,6 +86,8 @@ def column_sum(g: torch.Tensor) -> torch.Tensor:
 
 
 _MAX_LINEAR_OUT = 3
+_VP = [ctypes.c_void_p * n for n in range(_MAX_LINEAR_OUT + 1)]   # host arrays of the C ABI
+_CI = [ctypes.c_int * n for n in range(_MAX_LINEAR_OUT + 1)]
 _MAX_FEATURES = 16384
 
 
@@ -111,7 +113,7 @@ def esa_weight_grad(pairs, bias) -> list[tuple[torch.Tensor, torch.Tensor | None
     through esa_weight_grad; ``bias`` says per pair whether the column sums are wanted."""
     n, (rows, dev) = len(pairs), (pairs[0][0].shape[0], pairs[0][0].device)
     code = _CODES[pairs[0][0].dtype]
-    vp, ci = ctypes.c_void_p * n, ctypes.c_int * n
+    vp, ci = _VP[n], _CI[n]
     o, i = ci(*[g.shape[1] for g, _ in pairs]), ci(*[x.shape[1] for _, x in pairs])
     lib = _lib.load()
     nbytes = ctypes.c_size_t(0)
@@ -180,6 +182,113 @@ def esa_linear(x: torch.Tensor, pairs) -> list[torch.Tensor]:
     _lib.check(_lib.load().esa_linear_f32(x.data_ptr(), x.shape[0], x.shape[1], n, w_arr, b_arr, y_arr, n_arr,
                                           _lib.stream_of(x)), "esa_linear_f32")
     return ys
+
+
+PLAIN, MISH, MAB, ADD = range(4)   # esa_linear_fwd's epilogues
+
+
+def _gemm_k(k: int) -> bool:
+    return 32 <= k <= _MAX_FEATURES and k % 32 == 0
+
+
+def _gemm_cols(c: int, dtype) -> bool:
+    return 8 <= c <= _MAX_FEATURES and c % (8 if dtype == torch.bfloat16 else 4) == 0
+
+
+def fused_fwd(x, pairs, epilogue=PLAIN, other=None, residual=None, keep=True):
+    """esa_linear_fwd: the outputs y_i for PLAIN, else (z or None, result); see the C ABI for the epilogues.
+    x [rows, in] and (W, b) of one dtype, contiguous and 16-byte aligned, sizes as ``fused_ok`` accepts."""
+    n, rows, dt = len(pairs), x.shape[0], x.dtype
+    keep = keep and epilogue != ADD
+    ys = [torch.empty(rows, w.shape[0], dtype=dt, device=x.device) if keep else None for w, _ in pairs]
+    result = None
+    if epilogue != PLAIN:
+        result = torch.empty(rows, pairs[0][0].shape[0], dtype=dt if residual is None else torch.float32, device=x.device)
+    vp = _VP[n]
+    _lib.check(_lib.load().esa_linear_fwd(
+        x.data_ptr(), rows, x.shape[1], _CODES[dt], n, vp(*[w.data_ptr() for w, _ in pairs]),
+        vp(*[_lib.ptr(b) for _, b in pairs]), vp(*[_lib.ptr(y) for y in ys]),
+        _CI[n](*[w.shape[0] for w, _ in pairs]), epilogue, _lib.ptr(other), _lib.ptr(residual),
+        _lib.ptr(result), _lib.stream_of(x)), "esa_linear_fwd")
+    return ys if epilogue == PLAIN else (ys[0], result)
+
+
+def fused_dx(pairs, base=None, mish_z=None):
+    """esa_linear_dx: [base +] sum of g W over the (g, W) pairs, or (g W) mish'(mish_z)."""
+    (g, w), n = pairs[0], len(pairs)
+    dx = torch.empty(g.shape[0], w.shape[1], dtype=g.dtype, device=g.device)
+    vp = _VP[n]
+    _lib.check(_lib.load().esa_linear_dx(
+        vp(*[t.data_ptr() for t, _ in pairs]), vp(*[t.data_ptr() for _, t in pairs]), n, g.shape[0],
+        _CI[n](*[t.shape[1] for t, _ in pairs]), w.shape[1], _CODES[g.dtype], _lib.ptr(base),
+        _lib.ptr(mish_z), dx.data_ptr(), _lib.stream_of(g)), "esa_linear_dx")
+    return dx
+
+
+def fused_ok(x, weights, along: bool) -> bool:
+    """Whether esa_linear_fwd (``along``: the contraction runs along the weights' rows) or esa_linear_dx takes
+    these sizes and layouts."""
+    if not (x.is_cuda and x.dtype in _CODES and x.dim() == 2 and x.shape[0] < 2 ** 31):
+        return False
+    return all(w.dtype == x.dtype and w.is_contiguous() and _aligned(w)
+               and _gemm_k(w.shape[1 if along else 0]) and _gemm_cols(w.shape[0 if along else 1], w.dtype)
+               for w in weights)
+
+
+def _library_rate(x, w, fused_passes: bool) -> bool:
+    """bf16 products of this size run at a higher rate in the library GEMM, and its call's host time is hidden:
+    from 4e10 operations, where the epilogue saves no pass or the contraction is long (129,850 rows: 512 -> 512
+    82 vs 101 us, 512 -> 2048 with Mish 513 vs 546, 2048 -> 512 with the residual 363 vs 382; but 512 -> 512 with
+    the MAB's residual 235 vs 228, with the block's residual 240 vs 189)."""
+    return (x.dtype == torch.bfloat16 and 2 * x.shape[0] * w.numel() >= 4e10
+            and (not fused_passes or x.shape[1] >= 1024))
+
+
+# The Linears of the packed blocks.  ``fused``: the caller's word that esa_linear_fwd / esa_linear_dx take the sizes
+# and layouts (``fused_ok`` of both directions).
+
+def linear_outputs(x, pairs, fused: bool) -> list[torch.Tensor]:
+    """[x W^T + b for (W, b) in pairs]: one launch of esa_linear_fwd, or ``linear_fwd``."""
+    if fused and not _library_rate(x, pairs[0][0], False):
+        return fused_fwd(x, pairs)
+    return linear_fwd(x, pairs)
+
+
+def linear_then_mish(x, w, b, keep: bool, fused: bool):
+    """(z = x W^T + b or None, mish(z))."""
+    from .activations import mish_forward   # deferred: activations.py takes this module's functions
+    if fused and not _library_rate(x, w, False):
+        return fused_fwd(x, [(w, b)], MISH, keep=keep)
+    (z,) = linear_fwd(x, [(w, b)])
+    return z, mish_forward(z)
+
+
+def linear_then_mab(o, w, b, residual, keep: bool, fused: bool):
+    """(z = o W^T + b or None, o + mish(z), in fp32 on top of ``residual`` where that is given)."""
+    from .activations import mab_residual_forward, mish_forward
+    if fused and not _library_rate(o, w, True):
+        return fused_fwd(o, [(w, b)], MAB, o, residual, keep)
+    (z,) = linear_fwd(o, [(w, b)])
+    return z, mish_forward(z, o) if residual is None else mab_residual_forward(z, o, residual)
+
+
+def linear_then_add(x, w, b, residual, fused: bool):
+    """x W^T + b, rounded, plus the fp32 ``residual``."""
+    if fused and not _library_rate(x, w, True):
+        return fused_fwd(x, [(w, b)], ADD, residual=residual)[1]
+    return linear_fwd(x, [(w, b)])[0] + residual
+
+
+def input_grad(pairs, fused: bool, base=None, mish_z=None) -> torch.Tensor:
+    """[base +] sum of g W over the (g, W) pairs, or (g W) mish'(mish_z); all of one dtype."""
+    from .activations import mish_backward
+    (g, w) = pairs[0]
+    if fused and not _library_rate(g, w, len(pairs) > 1 or base is not None or mish_z is not None):
+        return fused_dx(pairs, base, mish_z)
+    dx = g.mm(w) if base is None else torch.addmm(base, g, w)
+    for g, w in pairs[1:]:
+        dx.addmm_(g, w)
+    return dx if mish_z is None else mish_backward(mish_z, dx)
 
 
 def linear_fwd(x: torch.Tensor, pairs) -> list[torch.Tensor]:

@@ -1,9 +1,10 @@
-"""The packed blocks recorded as one autograd node (mind_amd.esa.blocks) against the separate functions on the same
-kernels: outputs bit for bit, gradients of every input.
+"""The packed blocks recorded as one autograd node (mind_amd.esa.blocks) against the separate functions: outputs
+and gradients of every input.
 
-Bar of the gradients, norm-wise per tensor: the two differ in where partial gradients are added and rounded.  fp32:
-one more or less rounding of 2^-24 per addition, far below 1e-5.  bf16 autocast: a gradient rounded to bf16 once
-more or once less, 2^-9 of its magnitude per rounding, at most four of them on any path: 2^-7."""
+Bar, norm-wise per tensor: the two differ in the order of the Linears' sums and in where partial gradients are added
+and rounded.  fp32: roundings of 2^-24 per addition, far below 1e-5.  bf16 autocast: a value rounded to bf16 the
+other way, or a gradient rounded once more or once less, 2^-9 of its magnitude per rounding, at most four of them on
+any path: 2^-7."""
 import numpy as np
 import pytest
 import torch
@@ -37,14 +38,15 @@ def _both(one, separate, x, params, g, amp):
         assert out is not None
         res.append((out, torch.autograd.grad(out, [x] + params, g.to(out.dtype))))
     (o1, g1), (o2, g2) = res
-    assert torch.equal(o1, o2)
+    bar = 2.0 ** -7 if amp else 1e-5
+    assert o1.dtype == o2.dtype and float((o1.double() - o2.double()).norm()) <= bar * float(o2.double().norm())
     size = 0.0
     for a, b in zip(g1, g2):
         assert a.dtype == b.dtype and a.shape == b.shape
         # a bias sums the rows that its weight (the tensor before it) sums against inputs of about 1; fc_k's is zero
         # but for rounding, the softmax being unchanged by it
         size = max(float(b.double().norm()), size if b.dim() == 1 else 0.0)
-        assert float((a.double() - b.double()).norm()) <= (2.0 ** -7 if amp else 1e-5) * size
+        assert float((a.double() - b.double()).norm()) <= bar * size
 
 
 @pytest.mark.parametrize("amp", [False, True])
@@ -117,3 +119,20 @@ def test_differentiated_again_and_not_taken(device):
     masked_layers._sab_forward_packed(blk, x, tokens)
     handle.remove()
     assert seen
+
+
+@pytest.mark.parametrize("amp", [False, True])
+def test_strided_and_misaligned_parameters(device, amp):
+    """Parameters that the fused products do not take: a transposed weight, a bias off a 16-byte boundary."""
+    tokens = _tokens(device, False)
+    for which in ("weight", "bias"):
+        blk = _sab(device, 0, 2)
+        fc = blk.mlp.mlp[0]
+        if which == "weight":
+            fc.weight = torch.nn.Parameter(fc.weight.detach().t().contiguous().t())
+        else:
+            fc.bias = torch.nn.Parameter(torch.randn(fc.bias.numel() + 1, device=device)[1:])
+        x = torch.randn(tokens.num_tokens, 64, device=device, requires_grad=True)
+        g = torch.randn(tokens.num_tokens, 64, device=device)
+        _both(lambda: blocks.sab_block(blk, x, tokens, False, 0.0, None),
+              lambda: masked_layers._sab_separate(blk, x, tokens), x, [blk.mlp.mlp[2].weight, blk.norm.ln.weight], g, amp)
