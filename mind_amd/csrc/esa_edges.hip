@@ -310,7 +310,8 @@ constexpr int kSortItems = 16;
 constexpr int kSortTile = kSortThreads * kSortItems;
 constexpr int kRadixBits = 8;
 constexpr int kRadixBins = 1 << kRadixBits;
-static_assert(kRadixBins == kSortThreads, "one digit per thread in the per-digit steps");
+constexpr int kWideBits = 9;   // digit width where it saves a pass (see csr_build_impl)
+template <int BITS> constexpr int kDigits = (1 << BITS) / kSortThreads;   // digits per thread in the per-digit steps
 
 DEVI int clamp_key(int k, int num_nodes) { return (unsigned)k < (unsigned)num_nodes ? k : num_nodes; }
 
@@ -332,38 +333,61 @@ DEVI bool skipped(const int* skip) { return skip && *skip; }
 // pairs; else the caller's keys (clamped).  Digit order inside the tile is
 // irrelevant here, so full tiles read 16-byte vectors.
 // fill / fill_n: also set fill[0, fill_n) to -1 (indptr before its run pass),
-// so that no launch of its own is spent on it.
-template <bool PAIRS>
+// so that no launch of its own is spent on it.  descends: also set
+// descends[tile] to whether a key of the tile is followed by a smaller one.
+template <int BITS, bool PAIRS>
 __global__ __launch_bounds__(kSortThreads) void radix_hist_kernel(const int* __restrict__ in, long n, int num_nodes,
                                                                  int shift, bool vec, int* __restrict__ hist,
                                                                  int* __restrict__ fill, long fill_n,
-                                                                 const int* __restrict__ skip) {
-  if (skipped(skip)) return;
-  __shared__ int h[kRadixBins];
+                                                                 int* __restrict__ descends,
+                                                                 const int* __restrict__ skip,
+                                                                 const int* __restrict__ sorted) {
+  if (skipped(skip) || skipped(sorted)) return;
+  constexpr int kBins = 1 << BITS;
+  __shared__ int h[kBins];
   const int tid = threadIdx.x;
-  h[tid] = 0;
+#pragma unroll
+  for (int i = 0; i < kDigits<BITS>; ++i) h[i * kSortThreads + tid] = 0;
   if (fill)
     for (long i = (long)blockIdx.x * kSortThreads + tid; i < fill_n; i += (long)gridDim.x * kSortThreads) fill[i] = -1;
   const long tile = (long)blockIdx.x * kSortTile;
   int d[kSortItems];
+  bool down = false;
   if (vec && tile + kSortTile <= n) {
     if (PAIRS) {
       const int4* p = reinterpret_cast<const int4*>(in + 2 * tile);
 #pragma unroll
       for (int r = 0; r < kSortItems / 2; ++r) {
         const int4 x = p[r * kSortThreads + tid];
-        d[2 * r] = (x.x >> shift) & (kRadixBins - 1);
-        d[2 * r + 1] = (x.z >> shift) & (kRadixBins - 1);
+        d[2 * r] = (x.x >> shift) & (kBins - 1);
+        d[2 * r + 1] = (x.z >> shift) & (kBins - 1);
       }
     } else {
       const int4* p = reinterpret_cast<const int4*>(in + tile);
+      int4 x[kSortItems / 4];
+      int after[kSortItems / 4];
 #pragma unroll
       for (int r = 0; r < kSortItems / 4; ++r) {
-        const int4 x = p[r * kSortThreads + tid];
-        d[4 * r] = (clamp_key(x.x, num_nodes) >> shift) & (kRadixBins - 1);
-        d[4 * r + 1] = (clamp_key(x.y, num_nodes) >> shift) & (kRadixBins - 1);
-        d[4 * r + 2] = (clamp_key(x.z, num_nodes) >> shift) & (kRadixBins - 1);
-        d[4 * r + 3] = (clamp_key(x.w, num_nodes) >> shift) & (kRadixBins - 1);
+        x[r] = p[r * kSortThreads + tid];
+        // the key after this lane's four: the next lane's first, from memory only at the wave's end
+        const long next = tile + 4 * (r * kSortThreads + tid) + 4;
+        after[r] = -1;   // past the end: clamped to the largest key
+        if (descends && (tid & 63) == 63 && next < n) after[r] = in[next];
+      }
+#pragma unroll
+      for (int r = 0; r < kSortItems / 4; ++r) {
+        const int y = __shfl_down(x[r].x, 1);
+        if ((tid & 63) != 63) after[r] = y;
+      }
+#pragma unroll
+      for (int r = 0; r < kSortItems / 4; ++r) {
+        const int k0 = clamp_key(x[r].x, num_nodes), k1 = clamp_key(x[r].y, num_nodes);
+        const int k2 = clamp_key(x[r].z, num_nodes), k3 = clamp_key(x[r].w, num_nodes);
+        down |= k0 > k1 || k1 > k2 || k2 > k3 || k3 > clamp_key(after[r], num_nodes);
+        d[4 * r] = (k0 >> shift) & (kBins - 1);
+        d[4 * r + 1] = (k1 >> shift) & (kBins - 1);
+        d[4 * r + 2] = (k2 >> shift) & (kBins - 1);
+        d[4 * r + 3] = (k3 >> shift) & (kBins - 1);
       }
     }
   } else {
@@ -371,29 +395,87 @@ __global__ __launch_bounds__(kSortThreads) void radix_hist_kernel(const int* __r
     for (int j = 0; j < kSortItems; ++j) {
       const long i = tile + (long)j * kSortThreads + tid;
       const int k = i < n ? (PAIRS ? in[2 * i] : clamp_key(in[i], num_nodes)) : -1;
-      d[j] = k >= 0 ? (k >> shift) & (kRadixBins - 1) : -1;
+      if (!PAIRS && descends && i + 1 < n) down |= k > clamp_key(in[i + 1], num_nodes);
+      d[j] = k >= 0 ? (k >> shift) & (kBins - 1) : -1;
     }
   }
-  __syncthreads();
+  if (descends) {   // grid-uniform
+    const int any = __syncthreads_or(down);
+    if (tid == 0) descends[blockIdx.x] = any;
+  } else {
+    __syncthreads();
+  }
 #pragma unroll
   for (int j = 0; j < kSortItems; ++j)
     if (d[j] >= 0) atomicAdd(&h[d[j]], 1);
   __syncthreads();
-  hist[(long)blockIdx.x * kRadixBins + tid] = h[tid];
+#pragma unroll
+  for (int i = 0; i < kDigits<BITS>; ++i)
+    hist[(long)blockIdx.x * kBins + i * kSortThreads + tid] = h[i * kSortThreads + tid];
 }
 
-// The (digit, tile)-order exclusive scan of hist, in place, over its
-// [tile][digit] rows: per chunk of kHistChunk tiles the column sums (part);
-// one block scans part down each digit's column and adds the digit's base
-// (the exclusive scan of the digit totals); per chunk, each digit's column
-// is then walked down its kHistChunk rows.
-constexpr int kHistChunk = 64;
+// Sets *sorted to whether no tile descends, by one block.
+DEVI void store_sorted(const int* __restrict__ descends, int ntiles, int* __restrict__ sorted) {
+  int any = 0;
+  for (int t = threadIdx.x; t < ntiles; t += blockDim.x) any |= descends[t];
+  any = __syncthreads_or(any);
+  if (threadIdx.x == 0) *sorted = !any;
+}
+
+// The scan of hist, in place over its [tile][digit] rows: each digit's column
+// becomes its exclusive prefix over the tiles, and totals[digit] its sum (the
+// scatter adds the exclusive scan of the totals).  Up to kColumnScanTiles
+// tiles one launch does it, a block per 64 digits, its 16 waves taking equal
+// runs of rows (256 bytes per row and wave, summed, then walked again from L2):
+// 260 tiles of 512 digits 4 us, where a chunked scan took three launches and
+// 14 us.  Beyond, per chunk of kHistChunk tiles the column sums (part), one
+// block scans part down each digit's column and adds the digit's base (the
+// scatter then takes no totals), and per chunk each digit's column is walked
+// down its kHistChunk rows.
+// descends / sorted: see store_sorted (first pass).
+constexpr int kHistChunk = 64, kColumnScanTiles = 1024;
+
+template <int BITS>
+__global__ __launch_bounds__(1024) void hist_columns_kernel(int* __restrict__ hist, int ntiles, int* __restrict__ totals,
+                                                           const int* __restrict__ descends, int* __restrict__ sorted,
+                                                           const int* __restrict__ skip) {
+  if (skipped(skip) || (!descends && skipped(sorted))) return;
+  constexpr int kBins = 1 << BITS;
+  __shared__ int wsum[16][64];
+  if (descends && blockIdx.x == 0) store_sorted(descends, ntiles, sorted);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, digit = blockIdx.x * 64 + lane;
+  const int per = (ntiles + 15) / 16, t0 = min(ntiles, wave * per), t1 = min(ntiles, t0 + per);
+  int s = 0;
+#pragma unroll 8
+  for (int t = t0; t < t1; ++t) s += hist[(long)t * kBins + digit];
+  wsum[wave][lane] = s;
+  __syncthreads();
+  int run = 0, total = 0;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) {
+    const int x = wsum[w][lane];
+    run += w < wave ? x : 0;
+    total += x;
+  }
+  if (wave == 0) totals[digit] = total;
+  for (int u0 = t0; u0 < t1; u0 += 8) {
+    int x[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) x[u] = u0 + u < t1 ? hist[(long)(u0 + u) * kBins + digit] : 0;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      if (u0 + u < t1) hist[(long)(u0 + u) * kBins + digit] = run;
+      run += x[u];
+    }
+  }
+}
 
 int hist_chunks(int ntiles) { return (ntiles + kHistChunk - 1) / kHistChunk; }
 
 __global__ __launch_bounds__(kRadixBins) void hist_chunk_sum_kernel(const int* __restrict__ hist, int ntiles,
-                                                                   int* __restrict__ part, const int* __restrict__ skip) {
-  if (skipped(skip)) return;
+                                                                   int* __restrict__ part, const int* __restrict__ skip,
+                                                                   const int* __restrict__ sorted) {
+  if (skipped(skip) || skipped(sorted)) return;
   const int b0 = blockIdx.x * kHistChunk, tid = threadIdx.x;
   int x[kHistChunk];
 #pragma unroll
@@ -405,11 +487,15 @@ __global__ __launch_bounds__(kRadixBins) void hist_chunk_sum_kernel(const int* _
 }
 
 __global__ __launch_bounds__(4 * kRadixBins) void hist_chunk_scan_kernel(int* __restrict__ part, int nchunks,
+                                                                        int ntiles,
+                                                                        const int* __restrict__ descends,
+                                                                        int* __restrict__ sorted,
                                                                         const int* __restrict__ skip) {
-  if (skipped(skip)) return;
+  if (skipped(skip) || (!descends && skipped(sorted))) return;
   // thread: digit d, quarter q of the chunks
   __shared__ int qsum[4][kRadixBins];
   __shared__ int wtot[4][kRadixBins / 64];
+  if (descends) store_sorted(descends, ntiles, sorted);
   const int d = threadIdx.x & (kRadixBins - 1), q = threadIdx.x / kRadixBins;
   const int lane = threadIdx.x & 63, wv = d >> 6;
   const int per = (nchunks + 3) / 4, c0 = min(nchunks, q * per), c1 = min(nchunks, c0 + per);
@@ -446,8 +532,9 @@ __global__ __launch_bounds__(4 * kRadixBins) void hist_chunk_scan_kernel(int* __
 
 __global__ __launch_bounds__(kRadixBins) void hist_chunk_apply_kernel(int* __restrict__ hist, int ntiles,
                                                                      const int* __restrict__ part,
-                                                                     const int* __restrict__ skip) {
-  if (skipped(skip)) return;
+                                                                     const int* __restrict__ skip,
+                                                                     const int* __restrict__ sorted) {
+  if (skipped(skip) || skipped(sorted)) return;
   const int b0 = blockIdx.x * kHistChunk, tid = threadIdx.x;
   int x[kHistChunk];
 #pragma unroll
@@ -456,53 +543,6 @@ __global__ __launch_bounds__(kRadixBins) void hist_chunk_apply_kernel(int* __res
 #pragma unroll
   for (int r = 0; r < kHistChunk; ++r) {
     if (b0 + r < ntiles) hist[(long)(b0 + r) * kRadixBins + tid] = run;
-    run += x[r];
-  }
-}
-
-// The same scan in one block of 4 x 256 threads when ntiles <= 4 kHistChunk:
-// thread (q, d) holds rows [64 q, 64 q + 64) of digit d's column in registers;
-// the quarters' sums and the digit totals' exclusive scan go through LDS.
-constexpr int kSmallScanTiles = 4 * kHistChunk;
-
-__global__ __launch_bounds__(4 * kRadixBins) void hist_scan_small_kernel(int* __restrict__ hist, int ntiles,
-                                                                        const int* __restrict__ skip) {
-  if (skipped(skip)) return;
-  __shared__ int qsum[4][kRadixBins];
-  __shared__ int wtot[kRadixBins / 64];
-  const int d = threadIdx.x & (kRadixBins - 1), q = threadIdx.x / kRadixBins;
-  const int lane = threadIdx.x & 63, wv = d >> 6, r0 = q * kHistChunk;
-  int x[kHistChunk];
-  int s = 0;
-#pragma unroll
-  for (int r = 0; r < kHistChunk; ++r) {
-    x[r] = r0 + r < ntiles ? hist[(long)(r0 + r) * kRadixBins + d] : 0;
-    s += x[r];
-  }
-  qsum[q][d] = s;
-  __syncthreads();
-  int tot = 0, run = 0;
-#pragma unroll
-  for (int w = 0; w < 4; ++w) {
-    const int y = qsum[w][d];
-    run += w < q ? y : 0;
-    tot += y;
-  }
-  // exclusive scan of the digit totals, by the first quarter's waves
-  int incl = tot;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int y = __shfl_up(incl, o);
-    if (lane >= o) incl += y;
-  }
-  if (q == 0 && lane == 63) wtot[wv] = incl;
-  __syncthreads();
-#pragma unroll
-  for (int w = 0; w < kRadixBins / 64; ++w) run += w < wv ? wtot[w] : 0;
-  run += incl - tot;
-#pragma unroll
-  for (int r = 0; r < kHistChunk; ++r) {
-    if (r0 + r < ntiles) hist[(long)(r0 + r) * kRadixBins + d] = run;
     run += x[r];
   }
 }
@@ -525,9 +565,11 @@ DEVI int block_exclusive_scan256(int v, int* sh) {
   return before + x - v;
 }
 
-// offsets: the exclusive scan of hist in (digit, tile) order, in hist's
-// [tile][digit] rows: offsets[t * kRadixBins + d] is the first output slot of
-// tile t's digit-d elements.  IN_PAIRS: the input is (key, id) pairs, else the
+// offsets / totals: the scanned hist; the first output slot of tile t's digit-d
+// elements is offsets[t][d] plus, with totals, those of the digits below d.  sorted /
+// keys: where the caller's keys are in order already (*sorted), every pass but
+// the last returns at once and the last copies the keys and writes the
+// positions as ids.  IN_PAIRS: the input is (key, id) pairs, else the
 // caller's keys (clamped) with the positions as ids.  OUT_PAIRS: the output is
 // pairs, else keys_out and vals_out.  Each wave ranks its 1024 edges on its
 // own (a running count per digit in its own LDS row, peers of a round found
@@ -537,18 +579,30 @@ DEVI int block_exclusive_scan256(int v, int* sh) {
 // order, so consecutive threads write consecutive slots of one digit's run
 // instead of one slot per digit.  vec: the input may be read as 16-byte
 // vectors (full waves read theirs through their LDS slice).
-template <bool IN_PAIRS, bool OUT_PAIRS>
+template <int BITS, bool IN_PAIRS, bool OUT_PAIRS>
 __global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(const int* __restrict__ in, long n,
                                                                     int num_nodes, int shift, bool vec,
                                                                     const int* __restrict__ offsets,
+                                                                    const int* __restrict__ totals,
                                                                     int* __restrict__ out,
                                                                     int* __restrict__ vals_out,
+                                                                    const int* __restrict__ keys,
+                                                                    const int* __restrict__ sorted,
                                                                     const int* __restrict__ skip) {
   if (skipped(skip)) return;
-  constexpr int kWaves = kSortThreads / 64;
+  if (skipped(sorted)) {
+    if (!OUT_PAIRS)
+      for (long i = (long)blockIdx.x * kSortTile + threadIdx.x; i < min(n, ((long)blockIdx.x + 1) * kSortTile);
+           i += kSortThreads) {
+        out[i] = clamp_key(keys[i], num_nodes);
+        vals_out[i] = (int)i;
+      }
+    return;
+  }
+  constexpr int kWaves = kSortThreads / 64, kBins = 1 << BITS, kD = kDigits<BITS>;
   constexpr int kWaveItems = kSortItems * 64;
-  __shared__ int gbase[kRadixBins];         // output slot of the tile's local slot 0, per digit
-  __shared__ int wrun[kWaves][kRadixBins];  // per wave: running count, then first tile-local slot, per digit
+  __shared__ int gbase[kBins];         // output slot of the tile's local slot 0, per digit
+  __shared__ int wrun[kWaves][kBins];  // per wave: running count, then first tile-local slot, per digit
   __shared__ int2 skv[kSortTile];           // the wave's inputs in edge order, then the tile in output order
   __shared__ int sh[kWaves];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -603,9 +657,24 @@ __global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(const int* 
       }
     }
   }
-  const int g0 = offsets[(long)t_idx * kRadixBins + tid];
+  int g0[kD], below_digits = 0;   // this thread's digits kD tid .., and the totals of the digits below them
 #pragma unroll
-  for (int w = 0; w < kWaves; ++w) wrun[w][tid] = 0;
+  for (int i = 0; i < kD; ++i) g0[i] = offsets[(long)t_idx * kBins + kD * tid + i];
+  if (totals) {   // grid-uniform
+    int t[kD], sum = 0;
+#pragma unroll
+    for (int i = 0; i < kD; ++i) t[i] = totals[kD * tid + i];
+#pragma unroll
+    for (int i = 0; i < kD; ++i) {
+      g0[i] += sum;
+      sum += t[i];
+    }
+    below_digits = block_exclusive_scan256(sum, sh);
+  }
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w)
+#pragma unroll
+    for (int i = 0; i < kD; ++i) wrun[w][kD * tid + i] = 0;
   __syncthreads();
   // rank inside the wave: slot among the wave's earlier edges of the same digit
   const uint64_t below_mask = (1ull << lane) - 1;
@@ -614,10 +683,10 @@ __global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(const int* 
 #pragma unroll
   for (int j = 0; j < kSortItems; ++j) {
     const bool valid = k[j] >= 0;
-    const int d = valid ? (k[j] >> shift) & (kRadixBins - 1) : 0;
+    const int d = valid ? (k[j] >> shift) & (kBins - 1) : 0;
     uint64_t peers = __ballot(valid);
 #pragma unroll
-    for (int b = 0; b < kRadixBits; ++b) {
+    for (int b = 0; b < BITS; ++b) {
       const bool bit = (d >> b) & 1;
       const uint64_t m = __ballot(bit);
       peers &= bit ? m : ~m;
@@ -630,25 +699,30 @@ __global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(const int* 
     r[j] = before + below;
   }
   __syncthreads();
-  // digit tid: tile-local start, and each wave's first slot in it
+  // this thread's digits: tile-local start, and each wave's first slot in it
   {
-    int c[kWaves], tot = 0;
+    int c[kD][kWaves], tot = 0;
 #pragma unroll
-    for (int w = 0; w < kWaves; ++w) { c[w] = wrun[w][tid]; tot += c[w]; }
+    for (int i = 0; i < kD; ++i)
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) { c[i][w] = wrun[w][kD * tid + i]; tot += c[i][w]; }
     int acc = block_exclusive_scan256(tot, sh);
-    gbase[tid] = g0 - acc;
 #pragma unroll
-    for (int w = 0; w < kWaves; ++w) { wrun[w][tid] = acc; acc += c[w]; }
+    for (int i = 0; i < kD; ++i) {
+      gbase[kD * tid + i] = below_digits + g0[i] - acc;
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) { wrun[w][kD * tid + i] = acc; acc += c[i][w]; }
+    }
   }
   __syncthreads();
 #pragma unroll
   for (int j = 0; j < kSortItems; ++j)
-    if (k[j] >= 0) skv[run[(k[j] >> shift) & (kRadixBins - 1)] + r[j]] = int2{k[j], v[j]};
+    if (k[j] >= 0) skv[run[(k[j] >> shift) & (kBins - 1)] + r[j]] = int2{k[j], v[j]};
   __syncthreads();
   const int m = (int)min((long)kSortTile, n - tile);
   for (int t = tid; t < m; t += kSortThreads) {
     const int2 x = skv[t];
-    const int g = gbase[(x.x >> shift) & (kRadixBins - 1)] + t;
+    const int g = gbase[(x.x >> shift) & (kBins - 1)] + t;
     if (OUT_PAIRS) {
       reinterpret_cast<int2*>(out)[g] = x;
     } else {
@@ -891,7 +965,7 @@ __global__ __launch_bounds__(256) void segment_sum_rows_kernel(const T* __restri
 #define ESA_STREAM_BYTES 128  // bytes in flight per lane per step
 #endif
 #ifndef ESA_STREAM_NODES
-#define ESA_STREAM_NODES 32   // nodes per wave (at most 63)
+#define ESA_STREAM_NODES 32   // nodes per wave at most (at most 63)
 #endif
 #ifndef ESA_NODE_MODE
 #define ESA_NODE_MODE 1       // canonical-order CSRs of 512 / 1024-byte rows: the node-per-wave kernel
@@ -922,16 +996,16 @@ template <typename T, int VB>
 __global__ __launch_bounds__(256) void segment_sum_stream_kernel(const T* __restrict__ y,
                                                                  const int* __restrict__ perm,
                                                                  const int* __restrict__ indptr, int num_nodes,
-                                                                 T* __restrict__ out) {
+                                                                 int npw, T* __restrict__ out) {
   typedef typename RowVec<T, VB>::type V;
   constexpr int N = RowVec<T, VB>::N;
   constexpr int F = 64 * N;
   constexpr int kStreamU = StreamU<VB>::value;
   const int lane = threadIdx.x & 63;
   const int wave = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int n0 = wave * kStreamNodes;
+  const int n0 = wave * npw;
   if (n0 >= num_nodes) return;
-  const int nn = min(kStreamNodes, num_nodes - n0);
+  const int nn = min(npw, num_nodes - n0);
   const int ip = indptr[n0 + min(lane, nn)];   // lanes 0..nn: indptr[n0 .. n0 + nn]
   const int col = lane * N;
   int k = 0;                                    // current node n0 + k
@@ -1116,28 +1190,83 @@ size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
 int radix_blocks(int64_t num_edges) { return (int)((num_edges + kSortTile - 1) / kSortTile); }
 
-// Passes of kRadixBits over the keys 0 .. num_nodes (num_nodes: the slot of invalid keys).
-int radix_passes(int num_nodes) {
+// Digit width and passes over the keys 0 .. num_nodes (num_nodes: the slot of
+// invalid keys): 8 bits, or 9 where they save a pass and the column scan takes
+// the tiles (1,060,921 edges over 2^17 nodes, keys in no order: three passes of
+// 8 bits 95 us, two of 9 bits 56 us).
+struct RadixPlan { int bits, passes; };
+RadixPlan radix_plan(int num_nodes, int ntiles) {
   const int bits = 32 - __builtin_clz((unsigned)num_nodes | 1u);
-  return (bits + kRadixBits - 1) / kRadixBits;
+  const int narrow = (bits + kRadixBits - 1) / kRadixBits, wide = (bits + kWideBits - 1) / kWideBits;
+  return wide < narrow && ntiles <= kColumnScanTiles ? RadixPlan{kWideBits, wide} : RadixPlan{kRadixBits, narrow};
 }
 
-// Workspace: hist and its chunk sums, and two buffers of E (key, id) pairs
-// (pass p writes pair buffer p & 1; the last pass writes the sorted keys into
-// the buffer it does not read).
-struct CsrWs { size_t hist, part, pairs_a, pairs_b, total; };
+// Workspace: hist and its chunk sums, the digits' totals, the tiles' descends
+// flags with the sorted flag, and two buffers of E (key, id) pairs (pass p
+// writes pair buffer p & 1; the last pass writes the sorted keys into the
+// buffer it does not read).
+struct CsrWs { size_t hist, part, totals, descends, pairs_a, pairs_b, total; };
 CsrWs csr_ws(int64_t num_edges, int num_nodes) {
-  (void)num_nodes;
   CsrWs w;
-  const long nhist = (long)kRadixBins * radix_blocks(num_edges);
-  const long npart = (long)kRadixBins * hist_chunks(radix_blocks(num_edges));
+  const int ntiles = radix_blocks(num_edges);
+  const long nhist = (1L << radix_plan(num_nodes, ntiles).bits) * ntiles;
+  const long npart = (long)kRadixBins * hist_chunks(ntiles);
   size_t off = 0;
   w.hist = off; off += align256((size_t)(nhist > 0 ? nhist : 1) * 4);
   w.part = off; off += align256((size_t)(npart > 0 ? npart : 1) * 4);
+  w.totals = off; off += align256((size_t)4 << kWideBits);
+  w.descends = off; off += align256(((size_t)ntiles + 1) * 4);
   w.pairs_a = off; off += align256((size_t)num_edges * 8);
   w.pairs_b = off; off += align256((size_t)num_edges * 8);
   w.total = off;
   return w;
+}
+
+// The stable sort: perm and, into the returned buffer, the sorted keys.  The first pass's histogram finds whether the
+// keys are in order (edges listed by target, as radius graphs are): the passes then return at once and the last
+// copies: 1,060,921 edges over 2^17 nodes 95 -> 32 us, 2^25 over 2^21 528 -> 220 us; the check costs keys in no order
+// 2 % at 2^25 edges, where all passes stay).
+template <int BITS>
+const int* radix_sort(const int* keys, long num_edges, int num_nodes, int passes, int* indptr, int* perm, char* ws,
+                      const CsrWs& w, hipStream_t st, const int* skip) {
+  const int ntiles = radix_blocks(num_edges), nchunks = hist_chunks(ntiles);
+  int* hist = reinterpret_cast<int*>(ws + w.hist);
+  int* part = reinterpret_cast<int*>(ws + w.part);
+  int* totals = reinterpret_cast<int*>(ws + w.totals);
+  int* descends = reinterpret_cast<int*>(ws + w.descends);
+  int* sorted = descends + ntiles;
+  int* pairs[2] = {reinterpret_cast<int*>(ws + w.pairs_a), reinterpret_cast<int*>(ws + w.pairs_b)};
+  int* skeys = pairs[(passes - 1) & 1];
+  const bool vec_keys = !misaligned16(keys);
+  for (int p = 0; p < passes; ++p) {
+    const int shift = p * BITS;
+    const bool first = p == 0, last = p == passes - 1;
+    const int* in = first ? keys : pairs[(p - 1) & 1];
+    int* out = last ? skeys : pairs[p & 1];
+    int* flags = first ? descends : nullptr;
+    if (first)
+      hipLaunchKernelGGL((radix_hist_kernel<BITS, false>), dim3(ntiles), dim3(kSortThreads), 0, st, in, num_edges,
+                         num_nodes, shift, vec_keys, hist, indptr, (long)num_nodes + 1, flags, skip, nullptr);
+    else
+      hipLaunchKernelGGL((radix_hist_kernel<BITS, true>), dim3(ntiles), dim3(kSortThreads), 0, st, in, num_edges,
+                         num_nodes, shift, true, hist, nullptr, 0L, flags, skip, sorted);
+    if (ntiles <= kColumnScanTiles) {
+      hipLaunchKernelGGL(hist_columns_kernel<BITS>, dim3((1 << BITS) / 64), dim3(1024), 0, st, hist, ntiles, totals,
+                         flags, sorted, skip);
+    } else {   // BITS is kRadixBits here (radix_plan)
+      const int* done = first ? nullptr : sorted;
+      hipLaunchKernelGGL(hist_chunk_sum_kernel, dim3(nchunks), dim3(kRadixBins), 0, st, hist, ntiles, part, skip, done);
+      hipLaunchKernelGGL(hist_chunk_scan_kernel, dim3(1), dim3(4 * kRadixBins), 0, st, part, nchunks, ntiles, flags,
+                         sorted, skip);
+      hipLaunchKernelGGL(hist_chunk_apply_kernel, dim3(nchunks), dim3(kRadixBins), 0, st, hist, ntiles, part, skip,
+                         sorted);
+    }
+    auto scatter = first ? (last ? radix_scatter_kernel<BITS, false, false> : radix_scatter_kernel<BITS, false, true>)
+                         : (last ? radix_scatter_kernel<BITS, true, false> : radix_scatter_kernel<BITS, true, true>);
+    hipLaunchKernelGGL(scatter, dim3(ntiles), dim3(kSortThreads), 0, st, in, num_edges, num_nodes, shift,
+                       !first || vec_keys, hist, ntiles <= kColumnScanTiles ? totals : nullptr, out, perm, keys, sorted, skip);
+  }
+  return skeys;
 }
 
 template <typename T>
@@ -1165,16 +1294,19 @@ int launch_segsum(const T* y, long ld, const int* perm1, const int* indptr1, int
     }
   } else if (rows_ok && !perm2 && !indptr2 && off1 == 0 && ld == features &&
              (row_bytes == 64 * 16 || row_bytes == 64 * 8)) {
-    const long waves = ((long)num_nodes + kStreamNodes - 1) / kStreamNodes;
+    // nodes per wave: 32 where that leaves four waves per SIMD, fewer below (28,274 nodes of 4.6 rows of 1 KB:
+    // 45 -> 31 us)
+    const int npw = std::min(kStreamNodes, std::max(4, (num_nodes + 4095) / 4096));
+    const long waves = ((long)num_nodes + npw - 1) / npw;
     const unsigned blocks = (unsigned)((waves + 3) / 4);
     if (row_bytes == 64 * 16)
       ESA_TIMED(esa_profile::kSegmentSum, st,
                 hipLaunchKernelGGL((segment_sum_stream_kernel<T, 16>), dim3(blocks), dim3(256), 0, st, y, perm1,
-                                   indptr1, num_nodes, out));
+                                   indptr1, num_nodes, npw, out));
     else
       ESA_TIMED(esa_profile::kSegmentSum, st,
                 hipLaunchKernelGGL((segment_sum_stream_kernel<T, 8>), dim3(blocks), dim3(256), 0, st, y, perm1,
-                                   indptr1, num_nodes, out));
+                                   indptr1, num_nodes, npw, out));
   } else if (rows_ok && row_bytes % (64 * 16) == 0) {
     const unsigned blocks = grid_for((long)num_nodes, 4, 1L << 18);
     ESA_TIMED(esa_profile::kSegmentSum, st,
@@ -1357,40 +1489,10 @@ int csr_build_impl(const int* keys, int64_t num_edges, int num_nodes, int* indpt
   char* ws = static_cast<char*>(workspace);
   ESA_TIMED(esa_profile::kCsrBuild, st, {
     const int* sorted = nullptr;
-    if (num_edges > 0) {
-      // perm: stable radix sort of the edge ids by key
-      const int ntiles = radix_blocks(num_edges), passes = radix_passes(num_nodes);
-      const int nchunks = hist_chunks(ntiles);
-      int* hist = reinterpret_cast<int*>(ws + w.hist);
-      int* part = reinterpret_cast<int*>(ws + w.part);
-      int* pairs[2] = {reinterpret_cast<int*>(ws + w.pairs_a), reinterpret_cast<int*>(ws + w.pairs_b)};
-      int* skeys = pairs[(passes - 1) & 1];
-      const bool vec_keys = !misaligned16(keys);
-      for (int p = 0; p < passes; ++p) {
-        const int shift = p * kRadixBits;
-        const bool first = p == 0, last = p == passes - 1;
-        const int* in = first ? keys : pairs[(p - 1) & 1];
-        int* out = last ? skeys : pairs[p & 1];
-        if (first)
-          hipLaunchKernelGGL(radix_hist_kernel<false>, dim3(ntiles), dim3(kSortThreads), 0, st, in,
-                             (long)num_edges, num_nodes, shift, vec_keys, hist, indptr, (long)num_nodes + 1, skip);
-        else
-          hipLaunchKernelGGL(radix_hist_kernel<true>, dim3(ntiles), dim3(kSortThreads), 0, st, in,
-                             (long)num_edges, num_nodes, shift, true, hist, nullptr, 0L, skip);
-        if (ntiles <= kSmallScanTiles) {
-          hipLaunchKernelGGL(hist_scan_small_kernel, dim3(1), dim3(4 * kRadixBins), 0, st, hist, ntiles, skip);
-        } else {
-          hipLaunchKernelGGL(hist_chunk_sum_kernel, dim3(nchunks), dim3(kRadixBins), 0, st, hist, ntiles, part, skip);
-          hipLaunchKernelGGL(hist_chunk_scan_kernel, dim3(1), dim3(4 * kRadixBins), 0, st, part, nchunks, skip);
-          hipLaunchKernelGGL(hist_chunk_apply_kernel, dim3(nchunks), dim3(kRadixBins), 0, st, hist, ntiles,
-                             part, skip);
-        }
-        auto scatter = first ? (last ? radix_scatter_kernel<false, false> : radix_scatter_kernel<false, true>)
-                             : (last ? radix_scatter_kernel<true, false> : radix_scatter_kernel<true, true>);
-        hipLaunchKernelGGL(scatter, dim3(ntiles), dim3(kSortThreads), 0, st, in, (long)num_edges, num_nodes,
-                           shift, !first || vec_keys, hist, out, perm, skip);
-      }
-      sorted = skeys;
+    if (num_edges > 0) {   // perm: stable radix sort of the edge ids by key
+      const RadixPlan plan = radix_plan(num_nodes, radix_blocks(num_edges));
+      sorted = (plan.bits == kWideBits ? radix_sort<kWideBits> : radix_sort<kRadixBits>)(
+          keys, (long)num_edges, num_nodes, plan.passes, indptr, perm, ws, w, st, skip);
     }
     // indptr: the boundaries of the sorted keys' runs (set to -1 by the first histogram pass)
     if (num_edges == 0)

@@ -357,7 +357,7 @@ class _EdgeTokenLinear(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, g):
-        from .esa.linear import column_sum, weight_bias_grads
+        from .esa.linear import column_sum, fused_ok, input_grad, weight_bias_grads
         x, w2, src, dst, edge_attr, w_e = ctx.saved_tensors
         src_csr, dst_csr = ctx.csrs
         n, f = x.shape
@@ -368,16 +368,18 @@ class _EdgeTokenLinear(torch.autograd.Function):
         if dst_csr is None:
             dst_csr = CSR.build(dst, n)
         # d(a[src] + b[dst]) / d(a, b): per-node sums of the edge gradients, in ascending edge order
-        dpq = torch.cat((segment_sum_csr(g, src_csr.indptr, src_csr.perm),
-                         segment_sum_csr(g, dst_csr.indptr, dst_csr.perm)), 1)   # [N, 2D]
-        dx = dpq @ w2 if ctx.needs_input_grad[0] else None
+        gs = segment_sum_csr(g, src_csr.indptr, src_csr.perm)   # [N, D]
+        gd = segment_sum_csr(g, dst_csr.indptr, dst_csr.perm)
+        dx = None
+        if ctx.needs_input_grad[0]:
+            terms = [(gs, w2[:d]), (gd, w2[d:])]
+            dx = input_grad(terms, fused_ok(gs, [w for _, w in terms], False))
         dweight = None
         if ctx.needs_input_grad[1]:
-            dw2 = weight_bias_grads([(dpq, x)], [True], [False])[0][0].to(w2.dtype)   # [2D, F]
-            parts = [dw2[:d], dw2[d:]]
+            parts = [dw for dw, _ in weight_bias_grads([(gs, x), (gd, x)], [True, True], [False, False])]   # [D, F] each
             if edge_attr is not None:
-                parts.append(weight_bias_grads([(g, edge_attr)], [True], [False])[0][0].to(w2.dtype))   # [D, F_e]
-            dweight = torch.cat(parts, 1)                          # [D, 2F (+ F_e)]
+                parts.append(weight_bias_grads([(g, edge_attr)], [True], [False])[0][0])   # [D, F_e]
+            dweight = torch.cat(parts, 1).to(w2.dtype)              # [D, 2F (+ F_e)]
         dbias = column_sum(g).to(g.dtype) if ctx.has_bias and ctx.needs_input_grad[2] else None
         dattr = g @ w_e if edge_attr is not None and ctx.needs_input_grad[7] else None
         return dx, dweight, dbias, None, None, None, None, dattr
