@@ -269,10 +269,14 @@ DEVI void wait_vmcnt() {
 // `gtok` tokens (one block each), segments ordered by partner tiles (longest first, counting sort in
 // one block; segments with equal counts in any order, which changes no
 // result).  groups[i] = (outer begin, outer segment end, inner begin, inner end).
+// With `pairs` the cuts lie at even tokens: a segment that begins at an odd
+// one is cut as if it began one token earlier, and outer begin / 2 * 2 is the
+// first token of a group's tiles.  At most floor(n / gtok) + 1 groups of a
+// segment of n tokens either way.
 constexpr int kPlanBuckets = 1024;
 
 DEVI void seg_plan_block(const int* __restrict__ cu_outer, const int* __restrict__ cu_inner, int nseg, int gtok,
-                         int4* __restrict__ groups, int* __restrict__ count, int tid) {
+                         int4* __restrict__ groups, int* __restrict__ count, int tid, bool pairs = false) {
   constexpr int PER = kPlanBuckets / 256;
   __shared__ int hist[kPlanBuckets];
   __shared__ int part[256];
@@ -283,8 +287,8 @@ DEVI void seg_plan_block(const int* __restrict__ cu_outer, const int* __restrict
     return kPlanBuckets - 1 - min(max(tiles, 0), kPlanBuckets - 1);
   };
   for (int s = tid; s < nseg; s += 256) {
-    const int n = cu_outer[s + 1] - cu_outer[s];
-    if (n > 0) atomicAdd(&hist[bucket(s)], (n + gtok - 1) / gtok);
+    const int ob = cu_outer[s], n = cu_outer[s + 1] - ob;
+    if (n > 0) atomicAdd(&hist[bucket(s)], (n + (pairs ? ob & 1 : 0) + gtok - 1) / gtok);
   }
   __syncthreads();
   int loc[PER], sum = 0;
@@ -309,10 +313,11 @@ DEVI void seg_plan_block(const int* __restrict__ cu_outer, const int* __restrict
   for (int s = tid; s < nseg; s += 256) {
     const int ob = cu_outer[s], oe = cu_outer[s + 1];
     if (oe <= ob) continue;
-    const int ng = (oe - ob + gtok - 1) / gtok;
+    const int base = pairs ? ob & ~1 : ob;
+    const int ng = (oe - base + gtok - 1) / gtok;
     const int pos = atomicAdd(&hist[bucket(s)], ng);
     const int ib = cu_inner[s], ie = cu_inner[s + 1];
-    for (int j = 0; j < ng; ++j) groups[pos + j] = make_int4(ob + j * gtok, oe, ib, max(ie, ib));
+    for (int j = 0; j < ng; ++j) groups[pos + j] = make_int4(max(ob, base + j * gtok), oe, ib, max(ie, ib));
   }
 }
 

@@ -43,6 +43,8 @@
 // the bf16 probabilities the P V products take (v_dot2c_f32_bf16), so the
 // normalisation matches the products exactly (a one-key row gives out = v).  Every sum has a fixed order: the
 // backward is deterministic (dQ pass, then dK/dV pass; no atomics).
+#include <climits>
+
 #include "esa_attn_tiles.h"
 #include "esa_attn_dense.h"
 #include "esa_profile.h"
@@ -180,7 +182,8 @@ struct WStage {
 };
 
 template <int HD>
-DEVI WStage<HD> wide_gload(const bf16* a, const bf16* b, int g0, int total, int H, int head, int tid) {
+DEVI WStage<HD> wide_gload(const bf16* a, const bf16* b, int g0, int total, int H, int head, int tid,
+                           int lo = INT_MIN) {
   constexpr int NR = HD / 8;
   WStage<HD> s;
 #pragma unroll
@@ -189,7 +192,7 @@ DEVI WStage<HD> wide_gload(const bf16* a, const bf16* b, int g0, int total, int 
     if (WStage<HD>::NCH % 256 != 0 && c >= WStage<HD>::NCH) { s.r[i] = i32x4{}; continue; }
     const int tensor = c / (kWStage * NR), rem = c - tensor * (kWStage * NR);
     const int tok = rem / NR, o = rem - tok * NR;
-    const int t = min(g0 + tok, total - 1);
+    const int t = min(max(g0 + tok, lo), total - 1);
     s.r[i] = *reinterpret_cast<const i32x4*>((tensor ? b : a) + ((size_t)t * H + head) * HD + 8 * o);
   }
   return s;
@@ -232,47 +235,50 @@ struct WStageK {
 // Zeroes x[r] for the partners the keep mask drops: register r of lane half
 // h holds partner row_local(r, h) of the tile whose 32 partner keys start at
 // `keys` (LDS), the lane's own key is `own`.  Forward and dQ: the partners
-// are the keys, register 8 b + e holding key base + 16 b + 8 h + e, so the
-// global key pair {2i, 2i + 1} sits in two neighbouring registers of a run of
-// 8 and shares one hash: with the tile base `bp` = base mod 2 even the pairs
-// are registers (0, 1) .. (6, 7), 4 hashes per run; odd, (1, 2) .. (5, 6)
-// with registers 0 and 7 alone (their pairs lie in other runs), 5.
-DEVI void drop_tile(const DropoutCfg& d, uint32_t own, const uint32_t* keys, int h, int bp, float (&x)[16]) {
+// are the keys, register 8 b + e holding key base + 16 b + 8 h + e of an even
+// tile base, so the registers (0, 1) .. (6, 7) of a run of 8 are the global
+// key pairs {2i, 2i + 1} and share one hash.  A segment that begins at an odd
+// key is walked from the key before it, which the tile masks.
+DEVI void drop_tile(const DropoutCfg& d, uint32_t own, const uint32_t* keys, int h, float (&x)[16]) {
 #pragma unroll
   for (int b = 0; b < 2; ++b) {
     const uint4 k0 = *reinterpret_cast<const uint4*>(keys + 16 * b + 8 * h);
     const uint4 k1 = *reinterpret_cast<const uint4*>(keys + 16 * b + 8 * h + 4);
-    const uint32_t kk[8] = {k0.x, k0.y, k0.z, k0.w, k1.x, k1.y, k1.z, k1.w};
+    const uint32_t kk[4] = {k0.x, k0.z, k1.x, k1.z};
     float* y = x + 8 * b;
-    if (bp == 0) {
 #pragma unroll
-      for (int e = 0; e < 8; e += 2) {
-        const uint32_t bits = drop_bits(own, kk[e]);
-        y[e] = drop_half(d, bits, 0) ? y[e] : 0.f;
-        y[e + 1] = drop_half(d, bits, 1) ? y[e + 1] : 0.f;
-      }
-    } else {
-      y[0] = drop_half(d, drop_bits(own, kk[0]), 1) ? y[0] : 0.f;
-#pragma unroll
-      for (int e = 1; e < 7; e += 2) {
-        const uint32_t bits = drop_bits(own, kk[e]);
-        y[e] = drop_half(d, bits, 0) ? y[e] : 0.f;
-        y[e + 1] = drop_half(d, bits, 1) ? y[e + 1] : 0.f;
-      }
-      y[7] = drop_half(d, drop_bits(own, kk[7]), 0) ? y[7] : 0.f;
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t bits = drop_bits(own, kk[e]);
+      y[2 * e] = (bits << 16) >= d.thr_hi ? y[2 * e] : 0.f;
+      y[2 * e + 1] = bits >= d.thr_hi ? y[2 * e + 1] : 0.f;
     }
   }
 }
-// dK / dV (the partners are queries, the lane's own token the key, of parity
-// kpar): each score takes its key's half of its own hash.
-DEVI void drop_tile_key(const DropoutCfg& d, uint32_t own, const uint32_t* keys, int h, int kpar, float (&x)[16]) {
+// A value of the even (ctrl 0xA0: quad lanes 0, 0, 2, 2) or odd (0xF5: 1, 1,
+// 3, 3) lane of a pair, on both.
+template <int CTRL>
+DEVI uint32_t pair_lane(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xf, 0xf, true);
+}
+// dK / dV: the partners are queries, the lane's own token the key, and the
+// lanes of a pair (even tile base) own the two keys that share a hash per
+// query.  Each hashes four of a run's eight queries, the even lane the first
+// ones, and takes the others from its neighbour: half[r] = the key's 16 bits
+// for query row_local(r, h), in place (`mask`).  The hash is what bounds the
+// dropout passes (VALU issue, two 32-bit multiplies each); with one hash per
+// score this pass took 353 us at 43,670 tokens in 32 segments, 8 heads of 24,
+// with half of them 316 us.
+DEVI void drop_tile_key(uint32_t own, const uint32_t* keys, int h, int par, uint32_t mask, uint32_t (&half)[16]) {
 #pragma unroll
   for (int b = 0; b < 2; ++b) {
-    const uint4 k0 = *reinterpret_cast<const uint4*>(keys + 16 * b + 8 * h);
-    const uint4 k1 = *reinterpret_cast<const uint4*>(keys + 16 * b + 8 * h + 4);
-    const uint32_t kk[8] = {k0.x, k0.y, k0.z, k0.w, k1.x, k1.y, k1.z, k1.w};
+    const uint4 k = *reinterpret_cast<const uint4*>(keys + 16 * b + 8 * h + 4 * par);
+    const uint32_t kk[4] = {k.x, k.y, k.z, k.w};
 #pragma unroll
-    for (int e = 0; e < 8; ++e) x[8 * b + e] = drop_half(d, drop_bits(kk[e], own), kpar) ? x[8 * b + e] : 0.f;
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t bits = drop_bits(kk[e], own);
+      half[8 * b + e] = pair_lane<0xA0>(bits) & mask;
+      half[8 * b + 4 + e] = pair_lane<0xF5>(bits) & mask;
+    }
   }
 }
 
@@ -340,7 +346,9 @@ __global__ __launch_bounds__(256) void wide_fwd_kernel(const WideArgs a) {
 #pragma unroll
   for (int m = 0; m < NM; ++m) acc[m] = f32x16{};
   float m_run = fixed_ref ? 0.f : -INFINITY, l_run = 0.f;
-  const int n_tiles = (g.w - g.z + kTile - 1) >> 5;
+  // the first staged key: with dropout an even one (drop_tile); a key before the segment is masked
+  const int z0 = DROP && g.w > g.z ? g.z & ~1 : g.z;
+  const int n_tiles = (g.w - z0 + kTile - 1) >> 5;
   const int n_stages = (n_tiles + 1) >> 1;
   const f32x16 zero = {};
   auto run = [&](auto online_tag) {
@@ -349,8 +357,8 @@ __global__ __launch_bounds__(256) void wide_fwd_kernel(const WideArgs a) {
       n_stages,
       [&](int st) {
         WStageK<HD> s;
-        s.rows = wide_gload<HD>(a.k, a.v, g.z + st * kWStage, a.total_k, H, head, tid);
-        s.key = DROP && tid < kWStage ? drop_col(a.drop, g.z + st * kWStage + tid) : 0u;
+        s.rows = wide_gload<HD>(a.k, a.v, z0 + st * kWStage, a.total_k, H, head, tid, DROP ? g.z : INT_MIN);
+        s.key = DROP && tid < kWStage ? drop_col(a.drop, z0 + st * kWStage + tid) : 0u;
         return s;
       },
       [&](int buf, const WStageK<HD>& s) {
@@ -362,13 +370,14 @@ __global__ __launch_bounds__(256) void wide_fwd_kernel(const WideArgs a) {
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
           if (2 * st + u >= n_tiles) break;
-          const int k0 = g.z + st * kWStage + u * kTile;
+          const int k0 = z0 + st * kWStage + u * kTile;
           f32x16 s = zero;
 #pragma unroll
           for (int c = 0; c < NC; ++c) s = mfma32(row_octet<NO>(sK[buf], u * kTile + kperm(col), 2 * c + h), qop[c], s);
-          if (k0 + kTile > g.w) {
+          if (k0 + kTile > g.w || (DROP && k0 < g.z)) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) s[r] = k0 + row_local(r, h) < g.w ? s[r] : -INFINITY;
+            for (int r = 0; r < 16; ++r)
+              s[r] = (unsigned)(k0 + row_local(r, h) - g.z) < (unsigned)(g.w - g.z) ? s[r] : -INFINITY;
           }
           float p[16];
           if (ONLINE) {
@@ -397,7 +406,7 @@ __global__ __launch_bounds__(256) void wide_fwd_kernel(const WideArgs a) {
           bf16x8 pb[2] = {cvt8(p), cvt8(p + 8)};
           l_run = bf16_sum8(pb[0], bf16_sum8(pb[1], l_run));
           if (DROP) {
-            drop_tile(a.drop, rk, &sKey[buf][u * kTile], h, g.z & 1, p);
+            drop_tile(a.drop, rk, &sKey[buf][u * kTile], h, p);
             pb[0] = cvt8(p);
             pb[1] = cvt8(p + 8);
           }
@@ -459,15 +468,17 @@ void wide_dq_kernel(const WideArgs a) {
   f32x16 acc[NM];
 #pragma unroll
   for (int m = 0; m < NM; ++m) acc[m] = f32x16{};
-  const int n_tiles = (g.w - g.z + kTile - 1) >> 5;
+  // the first staged key: with dropout an even one (drop_tile); a key before the segment is masked
+  const int z0 = DROP && g.w > g.z ? g.z & ~1 : g.z;
+  const int n_tiles = (g.w - z0 + kTile - 1) >> 5;
   const int n_stages = (n_tiles + 1) >> 1;
   const f32x16 zero = {};
   wide_walk(
       n_stages,
       [&](int st) {
         WStageK<HD> s;
-        s.rows = wide_gload<HD>(a.k, a.v, g.z + st * kWStage, a.total_k, H, head, tid);
-        s.key = DROP && tid < kWStage ? drop_col(a.drop, g.z + st * kWStage + tid) : 0u;
+        s.rows = wide_gload<HD>(a.k, a.v, z0 + st * kWStage, a.total_k, H, head, tid, DROP ? g.z : INT_MIN);
+        s.key = DROP && tid < kWStage ? drop_col(a.drop, z0 + st * kWStage + tid) : 0u;
         return s;
       },
       [&](int buf, const WStageK<HD>& s) {
@@ -479,23 +490,24 @@ void wide_dq_kernel(const WideArgs a) {
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
           if (2 * st + u >= n_tiles) break;
-          const int k0 = g.z + st * kWStage + u * kTile;
+          const int k0 = z0 + st * kWStage + u * kTile;
           f32x16 s = zero, dp = zero;
 #pragma unroll
           for (int c = 0; c < NC; ++c) {
             s = mfma32(row_octet<NO>(sK[buf], u * kTile + kperm(col), 2 * c + h), qop[c], s);
             dp = mfma32(row_octet<NO>(sV[buf], u * kTile + kperm(col), 2 * c + h), gop[c], dp);
           }
-          if (k0 + kTile > g.w) {
+          if (k0 + kTile > g.w || (DROP && k0 < g.z)) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) s[r] = k0 + row_local(r, h) < g.w ? s[r] : -INFINITY;
+            for (int r = 0; r < 16; ++r)
+              s[r] = (unsigned)(k0 + row_local(r, h) - g.z) < (unsigned)(g.w - g.z) ? s[r] : -INFINITY;
           }
           float ds[16];
           if (DROP) {
             float dpk[16];
 #pragma unroll
             for (int r = 0; r < 16; ++r) dpk[r] = dp[r] * a.drop.inv_keep;
-            drop_tile(a.drop, rk, &sKey[buf][u * kTile], h, g.z & 1, dpk);
+            drop_tile(a.drop, rk, &sKey[buf][u * kTile], h, dpk);
 #pragma unroll
             for (int r = 0; r < 16; ++r) ds[r] = fast_exp2(fmaf(s[r], a.c, -lse2)) * (dpk[r] - dsum);
           } else {
@@ -532,8 +544,9 @@ void wide_dkdv_kernel(const WideArgs a) {
   wide_item_head<HD>(H, item, head);
   if (item >= *a.count) return;
   const int4 g = a.groups[item];   // outer = keys, inner = queries
-  const int t = g.x + wave * kTile + col;
-  const bool valid = t < g.y, active = g.x + wave * kTile < g.y;
+  const int x0 = DROP ? g.x & ~1 : g.x;   // even with dropout: drop_tile_key
+  const int t = x0 + wave * kTile + col;
+  const bool valid = t >= g.x && t < g.y, active = x0 + wave * kTile < g.y;
   const size_t row = ((size_t)(valid ? t : g.x) * H + head) * HD;
   bf16x8 kop[NC], vop[NC];
 #pragma unroll
@@ -542,7 +555,9 @@ void wide_dkdv_kernel(const WideArgs a) {
     vop[c] = row_op<HD>(a.v + row, 2 * c + h);
   }
   wide_zero_pad<HD>(sQ[0], sQ[1], sG[0], sG[1], tid);
-  const uint32_t ck = DROP ? drop_col(a.drop, valid ? t : g.x) : 0u;
+  const uint32_t ck = DROP ? drop_col(a.drop, t) : 0u;   // of every lane: its neighbour may be valid
+  const uint32_t half_mask = col & 1 ? 0xffff0000u : 0xffffu;
+  const uint32_t half_thr = col & 1 ? a.drop.thr_hi : a.drop.thr_hi >> 16;
   f32x16 dva[NM], dka[NM];
 #pragma unroll
   for (int m = 0; m < NM; ++m) dva[m] = dka[m] = f32x16{};
@@ -584,7 +599,7 @@ void wide_dkdv_kernel(const WideArgs a) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
               s[8 * b + e] = l0[e]; s[8 * b + 4 + e] = l1[e];
-              dp[8 * b + e] = d0[e]; dp[8 * b + 4 + e] = d1[e];
+              dp[8 * b + e] = DROP ? 0.f : d0[e]; dp[8 * b + 4 + e] = DROP ? 0.f : d1[e];
             }
           }
 #pragma unroll
@@ -599,27 +614,24 @@ void wide_dkdv_kernel(const WideArgs a) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) p[r] = q0 + row_local(r, h) < g.w ? p[r] : 0.f;
           }
-#pragma unroll
-          for (int r = 0; r < 16; ++r) ds[r] = p[r] * dp[r];
           if (DROP) {
-            // dp holds dO v - D: a kept partner's dS is P ((dO v) / (1 - p) - D), a dropped one's -P D
-            float nd[16], pk[16];
+            // a kept partner's dS is P ((dO v) / (1 - p) - D), a dropped one's -P D
+            uint32_t half[16];
+            drop_tile_key(ck, &sKey[buf][u * kTile], h, col & 1, half_mask, half);
 #pragma unroll
-            for (int b = 0; b < 2; ++b) {
-              const f32x4 d0 = ldsf4(&sDel[buf][u * kTile + 16 * b + 8 * h]);
-              const f32x4 d1 = ldsf4(&sDel[buf][u * kTile + 16 * b + 8 * h + 4]);
+            for (int q = 0; q < 4; ++q) {
+              const f32x4 nd = ldsf4(&sDel[buf][u * kTile + 16 * (q >> 1) + 8 * h + 4 * (q & 1)]);
 #pragma unroll
-              for (int e = 0; e < 4; ++e) { nd[8 * b + e] = d0[e]; nd[8 * b + 4 + e] = d1[e]; }
+              for (int e = 0; e < 4; ++e) {
+                const int r = 4 * q + e;
+                const bool keep = half[r] >= half_thr;
+                ds[r] = p[r] * (keep ? fmaf(a.drop.inv_keep, dp[r], nd[e]) : nd[e]);
+                p[r] = keep ? p[r] : 0.f;
+              }
             }
+          } else {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) pk[r] = 1.f;
-            drop_tile_key(a.drop, ck, &sKey[buf][u * kTile], h, t & 1, pk);
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-              const bool keep = pk[r] != 0.f;
-              ds[r] = p[r] * (keep ? fmaf(a.drop.inv_keep, dp[r] - nd[r], nd[r]) : nd[r]);
-              p[r] = keep ? p[r] : 0.f;
-            }
+            for (int r = 0; r < 16; ++r) ds[r] = p[r] * dp[r];
           }
 #pragma unroll
           for (int m = 0; m < NM; ++m)
@@ -647,6 +659,7 @@ struct WidePrep {
   float2* aux;
   const bf16* k; float* knorm;   // forward: max |k| per (head, 32-key tile)
   int nb_plan_k, nb_knorm, nb_rows;
+  bool key_pairs;   // the dK/dV plan's groups begin at even keys (drop_tile_key)
 };
 
 // max |k_t| over key tile `tile` per head: knorm[h * n_tiles + tile].  Lanes
@@ -703,7 +716,10 @@ __global__ __launch_bounds__(256) void wide_prep_kernel(const WidePrep p) {
   int b = blockIdx.x;
   if (b == 0) { seg_plan_block(p.cu_q, p.cu_k, p.nseg, kWGroup, p.plan_q, p.count_q, tid); return; }
   b -= 1;
-  if (b < p.nb_plan_k) { seg_plan_block(p.cu_k, p.cu_q, p.nseg, kWGroup, p.plan_k, p.count_k, tid); return; }
+  if (b < p.nb_plan_k) {
+    seg_plan_block(p.cu_k, p.cu_q, p.nseg, kWGroup, p.plan_k, p.count_k, tid, p.key_pairs);
+    return;
+  }
   b -= p.nb_plan_k;
   if (b < p.nb_knorm) { wide_knorm_block<HD>(p, b, tid); return; }
   b -= p.nb_knorm;
@@ -814,6 +830,7 @@ int wide_attn_bwd(const DenseAttnCall& c, void* workspace, size_t workspace_byte
   p.plan_k = reinterpret_cast<int4*>(ws + w.plan_k);
   p.aux = reinterpret_cast<float2*>(ws + w.aux);
   p.nb_plan_k = 1;
+  p.key_pairs = c.dropout;
   p.nb_rows = (int)std::max(1L, ((long)c.heads * (p.tq_pad - c.total_q) + 255) / 256);
   ESA_TIMED(esa_profile::kAttnPrep, st, ESA_WIDE_PREP(c.head_dim, dim3(2 + p.nb_rows), st, p));
   ESA_LAUNCH_CHECK();

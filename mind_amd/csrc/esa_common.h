@@ -102,20 +102,25 @@ inline DropoutCfg make_dropout(float p, unsigned long long seed, int heads) {
   return d;
 }
 
-DEVI uint32_t fmix32(uint32_t h) {
-  h ^= h >> 16;
+// fmix32(h) = drop_fold(drop_core(drop_fold(h))).  The fold is linear over xor
+// and its own inverse, so it is applied to the keys instead of to their xor:
+// a row or column key is kept before its last fold, which the first fold of
+// the pair's hash would only undo.  The pair's bits are those of
+// fmix32(fmix32(row) ^ fmix32(col)), one fold less per pair.
+DEVI uint32_t drop_fold(uint32_t h) { return h ^ (h >> 16); }
+DEVI uint32_t drop_core(uint32_t h) {
   h *= 0x85EBCA6Bu;
   h ^= h >> 13;
-  h *= 0xC2B2AE35u;
-  h ^= h >> 16;
-  return h;
+  return h * 0xC2B2AE35u;
 }
 DEVI uint32_t drop_row(const DropoutCfg& d, int q, int head) {
-  return fmix32(d.s0 ^ fmix32((uint32_t)q * (uint32_t)d.heads + (uint32_t)head));
+  return drop_core(drop_fold(d.s0) ^ drop_core(drop_fold((uint32_t)q * (uint32_t)d.heads + (uint32_t)head)));
 }
-DEVI uint32_t drop_col(const DropoutCfg& d, int k) { return fmix32(d.s1 ^ fmix32((uint32_t)k >> 1)); }
+DEVI uint32_t drop_col(const DropoutCfg& d, int k) {
+  return drop_core(drop_fold(d.s1) ^ drop_core(drop_fold((uint32_t)k >> 1)));
+}
 // The hash of a (row, col) pair; drop_half takes key k's 16 bits of it.
-DEVI uint32_t drop_bits(uint32_t row, uint32_t col) { return fmix32(row ^ col); }
+DEVI uint32_t drop_bits(uint32_t row, uint32_t col) { return drop_fold(drop_core(row ^ col)); }
 DEVI bool drop_half(const DropoutCfg& d, uint32_t bits, int k) { return (bits << (((k & 1) ^ 1) << 4)) >= d.thr_hi; }
 DEVI bool drop_keep(const DropoutCfg& d, uint32_t row, uint32_t col, int k) {
   return drop_half(d, drop_bits(row, col), k);
