@@ -505,7 +505,7 @@ ESA_API int esa_linear_dx(const void* const* g, const void* const* weight, int n
                    const int* out_features, int in_features, int dtype, const void* base,
                    const void* mish_z, void* dx, void* stream);
 
-/* Weight and bias gradients of n (1-3) of the blocks' Linear layers over    */
+/* Weight and bias gradients of n (1-8) of the blocks' Linear layers over    */
 /* one batch of rows (the autograd of nn.Linear, esa/mha.py:12-15,           */
 /* esa/mlp_utils.py:18-37): dW_i = g_i^T x_i [out_i, in_i] and, where db_i   */
 /* is not null, db_i [out_i] = the column sums of g_i, for g_i [rows, out_i] */

@@ -1,7 +1,7 @@
 // Weight and bias gradients of the packed blocks' Linear layers on gfx950:
-// dW_i = g_i^T x_i and db_i = column sums of g_i, for up to three (g_i, x_i)
-// over the same rows (the MAB's fc_q / fc_k / fc_v, esa/mha.py:54-56; any
-// one nn.Linear of esa/mha.py:12-15, esa/mlp_utils.py:18-37), g_i [rows, out]
+// dW_i = g_i^T x_i and db_i = column sums of g_i, for up to eight (g_i, x_i)
+// over the same rows (a block's nn.Linears, esa/mha.py:12-15, 54-56,
+// esa/mlp_utils.py:18-37, in one launch or one by one), g_i [rows, out]
 // and x_i [rows, in] both bf16 or both fp32, results fp32.
 //
 // The contraction runs over the tokens (up to hundreds of thousands) into a
@@ -30,7 +30,8 @@
 // 768 x 192 29 vs 94; 129,850 x 512 x 512 94 vs 139 (724 TFLOP/s); 129,850 x
 // 2048 x 512 284 vs 381 (958 TFLOP/s); fp32 21,752 x 128 x 128 23 vs 54,
 // three 34 vs 162; 33,000 x 1024 x 256 141 vs 160 (123 of the 154 TFLOP/s that
-// a large fp32 product reaches).  The stage loop holds no spill and no copy of
+// a large fp32 product reaches).  The six weights of a SAB block with its MLP
+// in one launch: fp32 21,752 x 128 63 vs 105 in four, bf16 33,000 x 256 56 vs 99.  The stage loop holds no spill and no copy of
 // the accumulators: scratch loads share the counter that the staging waits on,
 // and a spilling first version ran at a third of the rate.
 #include <algorithm>
@@ -42,7 +43,7 @@
 
 namespace {
 
-constexpr int kMaxPairs = 3;
+constexpr int kMaxPairs = 8;
 constexpr int kWTileO = 128;                 // block tile along `out` (two waves of 64); along `in`: 64 NV (two of 32 NV)
 constexpr int kStages = 3;
 constexpr int kCus = 256, kMinRows = 128;

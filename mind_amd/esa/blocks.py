@@ -125,16 +125,47 @@ def _mlp_forward(x, params, residual, keep, fused):
     return linear_outputs(x, [(w, b)], fused)[0] + residual, saved
 
 
-def _mlp_backward(g, saved, needs, fused):
-    """(dx, the parameters' gradients) for the output gradient g in the compute dtype."""
-    grads = [None] * len(needs)
+# Token counts up to which a block's weight gradients wait for the end of its backward and run in one launch: the
+# launches of single weights leave the chip partly idle at their ends and each costs the host.  Six weights of a SAB
+# block with an MLP, apart and together, us: fp32 21,752 x 128 105 / 63; bf16 33,000 x 256 99 / 56, 65,536 x 512
+# (MLP 2048) 478 / 448; 129,850 x 512 864 / 934, where a weight alone fills the chip and takes longer row ranges.
+# Above the line the operands are freed early, too.
+_TOGETHER = 65536
+
+
+class _Grads:
+    """The gradients of a block's inputs by position, those of its Linears from their (output gradient, input)."""
+
+    def __init__(self, setup, needs, rows):
+        self.needs, self.out, self.pairs = needs, [None] * len(needs), []
+        self.together = setup.fused and rows <= _TOGETHER
+
+    def add(self, *pairs):
+        """(position of the weight, g, x), the bias one further; computed now unless they can wait."""
+        self.pairs += pairs
+        if not self.together:
+            self.compute()
+
+    def compute(self):
+        by_rows = {}
+        for pair in self.pairs:
+            by_rows.setdefault(pair[1].shape[0], []).append(pair)
+        for pairs in by_rows.values():
+            got = weight_bias_grads([p[1:] for p in pairs], [self.needs[p[0]] for p in pairs],
+                                    [self.needs[p[0] + 1] for p in pairs])
+            for (i, _, _), pair in zip(pairs, got):
+                self.out[i:i + 2] = pair
+        self.pairs = []
+
+
+def _mlp_backward(g, saved, grads, first, fused):
+    """dx for the output gradient g in the compute dtype; the parameters from position ``first`` on go to ``grads``."""
     layers = [saved[i:i + 3] for i in range(0, len(saved), 3)]
     for i in range(len(layers) - 1, -1, -1):
         x, w = layers[i][:2]
-        ((grads[2 * i], grads[2 * i + 1]),) = weight_bias_grads([(g, x)], needs[2 * i:2 * i + 1],
-                                                                needs[2 * i + 1:2 * i + 2])
+        grads.add((first + 2 * i, g, x))
         g = input_grad([(g, w)], fused, mish_z=layers[i - 1][2] if i else None)
-    return g, grads
+    return g
 
 
 class _SabBlock(torch.autograd.Function):
@@ -169,26 +200,25 @@ class _SabBlock(torch.autograd.Function):
         x, ln_w, stats, xm, q, k, v, o, lse, z, wq, wk, wv, wo = tensors[:14]
         cu, mask = tensors[ctx.n_keep], dict(zip(ctx.mask_keys, tensors[ctx.n_keep + 1:]))
         t, d = x.shape
-        g = g.contiguous()
-        mlp_grads = ()
+        g, grads = g.contiguous(), _Grads(setup, needs, t)
         if setup.n_mlp:
             x2, ln_w2, stats2 = tensors[14:17]
-            dy, mlp_grads = _mlp_backward(g.to(setup.dt), tensors[17:ctx.n_keep], needs[13:], setup.fused)
-            g, dw, db = ln_backward(x2, ln_w2, stats2, None if setup.amp else dy, dy if setup.amp else None, g,
-                                    needs[11], needs[12])
-            mlp_grads = (dw, db, *mlp_grads)
+            dy = _mlp_backward(g.to(setup.dt), tensors[17:ctx.n_keep], grads, 13, setup.fused)
+            g, *grads.out[11:13] = ln_backward(x2, ln_w2, stats2, None if setup.amp else dy, dy if setup.amp else None,
+                                               g, needs[11], needs[12])
         dz, g_o = mab_residual_backward(z, g)
         do = input_grad([(dz, wo)], setup.fused, g_o).view_as(o)
-        grads_o = weight_bias_grads([(dz, o.view(t, d))], needs[9:10], needs[10:11])
+        grads.add((9, dz, o.view(t, d)))
         n, (p, seed) = setup.max_items, setup.dropout
         gq, gk, gv = (y.view(t, d) for y in attn_bwd(do, q, k, v, o, lse, cu, cu, n, n, 1.0 / math.sqrt(d // setup.heads),
                                                      dropout_p=p, dropout_seed=seed, **mask))
         # fp32: the norm's one output feeds the projections and the residual, whose gradient g starts the sum
         dxm = input_grad([(gq, wq), (gk, wk), (gv, wv)], setup.fused, None if setup.amp else g)
-        grads = weight_bias_grads([(gq, xm), (gk, xm), (gv, xm)], needs[3:9:2], needs[4:9:2])
-        dx, dw, db = ln_backward(x, ln_w, stats, g if setup.amp else dxm, dxm if setup.amp else None, None, needs[1],
-                                 needs[2])
-        return (None, dx, dw, db, *(y for pair in grads + grads_o for y in pair), *mlp_grads)
+        grads.add((3, gq, xm), (5, gk, xm), (7, gv, xm))
+        grads.compute()
+        grads.out[:3] = ln_backward(x, ln_w, stats, g if setup.amp else dxm, dxm if setup.amp else None, None,
+                                    needs[1], needs[2])
+        return (None, *grads.out)
 
 
 def sab_block(blk, x: torch.Tensor, tokens, masked: bool, attn_p: float, again) -> torch.Tensor | None:
@@ -243,26 +273,25 @@ class _PmaBlock(torch.autograd.Function):
         x, ln_w, stats, xm, s, q, k, v, o, lse, z, wq, wk, wv, wo = tensors[:15]
         cu, seeds = tensors[ctx.n_keep:ctx.n_keep + 2]
         d = x.shape[1]
-        g = g.contiguous().view(-1, d)
-        mlp_grads = ()
+        g, grads = g.contiguous().view(-1, d), _Grads(setup, needs, x.shape[0])
         if setup.n_mlp:
             x2, ln_w2, stats2 = tensors[15:18]
-            dy, mlp_grads = _mlp_backward(g, tensors[18:ctx.n_keep], needs[14:], setup.fused)
-            g, dw, db = ln_backward(x2, ln_w2, stats2, None if setup.amp else dy, dy if setup.amp else None, g,
-                                    needs[12], needs[13])
-            mlp_grads = (dw, db, *mlp_grads)
+            dy = _mlp_backward(g, tensors[18:ctx.n_keep], grads, 14, setup.fused)
+            g, *grads.out[12:14] = ln_backward(x2, ln_w2, stats2, None if setup.amp else dy, dy if setup.amp else None,
+                                               g, needs[12], needs[13])
         dz = mish_backward(z, g)
         do = input_grad([(dz, wo)], setup.fused, g).view_as(o)
-        grads_o = weight_bias_grads([(dz, o.view(-1, d))], needs[10:11], needs[11:12])
+        grads.add((10, dz, o.view(-1, d)))
         gq, gk, gv = (y.view(-1, d) for y in pma_backward(do, q, k, v, o, lse, cu, setup.max_items,
                                                           1.0 / math.sqrt(d // setup.heads), *setup.dropout))
-        dseeds = input_grad([(gq, wq)], setup.fused).view(seeds.shape).to(seeds.dtype) if needs[1] else None
+        if needs[1]:
+            grads.out[1] = input_grad([(gq, wq)], setup.fused).view(seeds.shape).to(seeds.dtype)
         dxm = input_grad([(gk, wk), (gv, wv)], setup.fused)
-        grads = (weight_bias_grads([(gq, s)], needs[4:5], needs[5:6])
-                 + weight_bias_grads([(gk, xm), (gv, xm)], needs[6:10:2], needs[7:10:2]))
-        dx, dw, db = ln_backward(x, ln_w, stats, None if setup.amp else dxm, dxm if setup.amp else None, None, needs[2],
-                                 needs[3])
-        return (None, dx, dseeds, dw, db, *(y for pair in grads + grads_o for y in pair), *mlp_grads)
+        grads.add((4, gq, s), (6, gk, xm), (8, gv, xm))
+        grads.compute()
+        grads.out[0], *grads.out[2:4] = ln_backward(x, ln_w, stats, None if setup.amp else dxm,
+                                                    dxm if setup.amp else None, None, needs[2], needs[3])
+        return (None, *grads.out)
 
 
 def pma_block(blk, x: torch.Tensor, tokens, attn_p: float, again) -> torch.Tensor | None:

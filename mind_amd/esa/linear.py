@@ -86,8 +86,9 @@ def column_sum(g: torch.Tensor) -> torch.Tensor:
 
 
 _MAX_LINEAR_OUT = 3
-_VP = [ctypes.c_void_p * n for n in range(_MAX_LINEAR_OUT + 1)]   # host arrays of the C ABI
-_CI = [ctypes.c_int * n for n in range(_MAX_LINEAR_OUT + 1)]
+_MAX_GRADS = 8
+_VP = [ctypes.c_void_p * n for n in range(_MAX_GRADS + 1)]   # host arrays of the C ABI
+_CI = [ctypes.c_int * n for n in range(_MAX_GRADS + 1)]
 _MAX_FEATURES = 16384
 
 
@@ -109,7 +110,7 @@ def _wgrad_ok(pairs) -> bool:
 
 
 def esa_weight_grad(pairs, bias) -> list[tuple[torch.Tensor, torch.Tensor | None]]:
-    """[(g^T x, g.sum(0) or None)] in fp32 for 1-3 (g, x) over the same rows (the shapes ``_wgrad_ok`` accepts)
+    """[(g^T x, g.sum(0) or None)] in fp32 for 1-8 (g, x) over the same rows (the shapes ``_wgrad_ok`` accepts)
     through esa_weight_grad; ``bias`` says per pair whether the column sums are wanted."""
     n, (rows, dev) = len(pairs), (pairs[0][0].shape[0], pairs[0][0].device)
     code = _CODES[pairs[0][0].dtype]
@@ -133,16 +134,23 @@ def _aligned(t: torch.Tensor) -> bool:
 
 
 def weight_bias_grads(pairs, need_w, need_b) -> list[tuple[torch.Tensor | None, torch.Tensor | None]]:
-    """[(g^T x, g.sum(0))] in fp32 for 1-3 (g, x) over the same rows, None where ``need_w`` / ``need_b`` says a
-    gradient is not wanted: one call of esa_weight_grad where it takes them, else ``weight_grad`` and
+    """[(g^T x, g.sum(0))] in fp32 for any (g, x) over the same rows, None where ``need_w`` / ``need_b`` says a
+    gradient is not wanted: calls of esa_weight_grad for up to eight where it takes them, else ``weight_grad`` and
     ``column_sum`` one by one (also where the gradients are to be differentiated again: ``weight_grad`` is made
     of torch operations)."""
-    wanted = [p for p, w in zip(pairs, need_w) if w]
-    again = torch.is_grad_enabled() and any(t.requires_grad for p in wanted for t in p)
-    if wanted and not again and _wgrad_ok(wanted):
-        got = iter(esa_weight_grad(wanted, [b for w, b in zip(need_w, need_b) if w]))
-        return [next(got) if w else (None, column_sum(g) if b else None)
-                for (g, _), w, b in zip(pairs, need_w, need_b)]
+    wanted = [(p, b) for p, w, b in zip(pairs, need_w, need_b) if w]
+    again = torch.is_grad_enabled() and any(t.requires_grad for p, _ in wanted for t in p)
+    if wanted and not again:
+        if _wgrad_ok([p for p, _ in wanted]):
+            got = []
+            for i in range(0, len(wanted), _MAX_GRADS):
+                part = wanted[i:i + _MAX_GRADS]
+                got += esa_weight_grad([p for p, _ in part], [b for _, b in part])
+            got = iter(got)
+            return [next(got) if w else (None, column_sum(g) if b else None)
+                    for (g, _), w, b in zip(pairs, need_w, need_b)]
+        if len(pairs) > 1:
+            return [weight_bias_grads([p], [w], [b])[0] for p, w, b in zip(pairs, need_w, need_b)]
     return [(weight_grad(g, x) if w else None, column_sum(g) if b else None)
             for (g, x), w, b in zip(pairs, need_w, need_b)]
 

@@ -54,6 +54,25 @@ def test_three_pairs_share_rows(device, dtype):
     assert all(torch.equal(a[0], b[0]) for a, b in zip(got, again))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows", [33, 5003])
+def test_many_pairs_of_different_shapes(device, dtype, rows):
+    """A block's Linears together: eight in a call, two more in a second one, an unwanted weight between them, and
+    one the kernel does not take (a bias-only result and a misaligned gradient), which leaves the others to it."""
+    shapes = [(64, 128), (200, 136), (128, 40), (8, 8), (256, 64), (64, 256), (136, 128), (128, 128), (40, 72), (72, 8)]
+    pairs = _pairs(device, rows, shapes, dtype)
+    bias = [i % 3 != 1 for i in range(len(pairs))]
+    _check(pairs, L.weight_bias_grads(pairs, [True] * len(pairs), bias), bias)
+    (dw, db), *rest = L.weight_bias_grads(pairs[:4], [False] + [True] * 3, [True] * 4)
+    assert dw is None and torch.allclose(db, pairs[0][0].float().sum(0), atol=1e-2)
+    _check(pairs[1:4], rest, [True] * 3)
+    flat = torch.randn(rows * 64 + 1, device=device).to(dtype)
+    off = flat[1:].view(rows, 64)
+    got = L.weight_bias_grads([(off, pairs[0][1])] + pairs[1:3], [True] * 3, [False] * 3)
+    assert torch.allclose(got[0][0].double(), off.double().t() @ pairs[0][1].double(), rtol=2e-2, atol=1.0)
+    _check(pairs[1:3], got[1:], [False] * 2)
+
+
 @pytest.mark.parametrize("shapes", [[(512, 512)] * 3, [(2040, 504)]])
 def test_wide_tiles(device, shapes):
     """Enough 128 x 256 tiles and rows for the wide tile, whole and with remainders in rows and features."""
