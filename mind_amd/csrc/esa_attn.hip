@@ -1488,6 +1488,40 @@ DEVI void f32_gather(f32x4 (&acc)[F32Tile<HD>::QB][F32Tile<HD>::NR], const float
     }
 }
 
+// The same over the admissible pairs alone, by vector FMAs: with the edge mask, where a partner's row holds an infinity
+// or a NaN, which times the zero weight of a pair that the mask leaves out would reach tokens that do not attend it.
+template <int HD>
+DEVI void f32_gather_admissible(f32x4 (&acc)[F32Tile<HD>::QB][F32Tile<HD>::NR],
+                                const float (*rows)[F32Tile<HD>::kStride], int p0, const f32x4 (&w)[F32Tile<HD>::QB],
+                                int c16, int grp, const int2* nodes, int t0, int end, const int (&tok)[F32Tile<HD>::QB],
+                                const int2 (&node)[F32Tile<HD>::QB]) {
+#pragma unroll 1
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int p = p0 + 4 * j + r;
+#pragma unroll
+      for (int b = 0; b < F32Tile<HD>::QB; ++b) {
+        const float x = __shfl(w[b][r], 16 * j + c16);
+        if (!admissible_f32<true>(t0 + p, end, tok[b], nodes[p], node[b])) continue;
+#pragma unroll
+        for (int c = 0; c < F32Tile<HD>::NR; ++c)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[b][c][e] = fmaf(x, rows[p][16 * c + 4 * grp + e], acc[b][c][e]);
+      }
+    }
+}
+// Whether a value of the stage's rows is an infinity or a NaN.
+template <int N>
+DEVI bool nonfinite(const f32x4 (&r)[N]) {
+  bool any = false;
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) any |= (__float_as_uint(r[i][e]) & 0x7f800000u) == 0x7f800000u;
+  return any;
+}
+
 // The block's work item, the wave's column blocks and this lane's owned tokens (clamped into the group).
 template <int HD>
 struct F32Own {
@@ -1840,6 +1874,7 @@ __global__ __launch_bounds__(F32Tile<HD>::kThreads) void attn_dq_f32_kernel(cons
   __shared__ __align__(16) typename T::Rows sK[2], sV[2];
   __shared__ int2 sN[2][MASKED ? kF32Stage : 1];
   __shared__ uint32_t sKey[2][DROP ? kF32Stage : 1];   // column keys of the staged keys
+  __shared__ int sOdd[2];   // edge mask: the first token of a stage with a nonfinite key row
   const int H = a.heads, item = blockIdx.x / H, head = blockIdx.x - item * H;
   if (item >= *a.count) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1862,10 +1897,16 @@ __global__ __launch_bounds__(F32Tile<HD>::kThreads) void attn_dq_f32_kernel(cons
   }
   f32x4 rK[T::kPer], rV[T::kPer];
   int2 rN = make_int2(-1, -1);
+  int rT = 0;
+  if (MASKED) {
+    if (tid < 2) sOdd[tid] = -1;
+    __syncthreads();
+  }
   uint32_t rKey = 0;
   f32_stages(
       own.plo, phi, own.live,
       [&](int t0) {
+        rT = t0;
         f32_load<HD>(rK, a.k, phi, H, head, t0);
         f32_load<HD>(rV, a.v, phi, H, head, t0);
         if (MASKED && tid < kF32Stage) rN = t0 + tid < phi ? a.nodes[t0 + tid] : make_int2(-1, -1);
@@ -1874,11 +1915,12 @@ __global__ __launch_bounds__(F32Tile<HD>::kThreads) void attn_dq_f32_kernel(cons
       [&](int buf) {
         f32_store<HD>(sK[buf], rK);
         f32_store<HD>(sV[buf], rV);
+        if (MASKED && nonfinite(rK)) sOdd[buf] = rT;   // the same value from every thread
         if (MASKED && tid < kF32Stage) sN[buf][tid] = rN;
         if (DROP && tid < kF32Stage) sKey[buf][tid] = rKey;
       },
       [&](int buf, int k0) {
-        const bool tail = k0 + kF32Stage > phi;
+        const bool tail = k0 + kF32Stage > phi, odd = MASKED && sOdd[buf] == k0;
 #pragma unroll
         for (int kb = 0; kb < KB; ++kb) {
           f32x4 x[NR], s[QB], ds[QB];
@@ -1894,14 +1936,18 @@ __global__ __launch_bounds__(F32Tile<HD>::kThreads) void attn_dq_f32_kernel(cons
             const int2 pn = MASKED ? sN[buf][key] : make_int2(0, 0);
 #pragma unroll
             for (int b = 0; b < QB; ++b) {
-              float p = fast_exp2(a.c * s[b][r] - rs[b].x);
-              if (MASKED || tail) p = admissible_f32<MASKED>(k0 + key, phi, own.tok[b], pn, node[b]) ? p : 0.f;
+              const float p = fast_exp2(a.c * s[b][r] - rs[b].x);
               float dp = ds[b][r];
               if (DROP) dp = drop_keep(a.drop, rk[b], sKey[buf][key], k0 + key) ? dp * a.drop.inv_keep : 0.f;
               ds[b][r] = p * (dp - rs[b].y);
+              if (MASKED || tail)
+                ds[b][r] = admissible_f32<MASKED>(k0 + key, phi, own.tok[b], pn, node[b]) ? ds[b][r] : 0.f;
             }
           }
-          f32_gather<HD>(acc, sK[buf], 16 * kb, ds, c16, grp);
+          if (MASKED && odd)
+            f32_gather_admissible<HD>(acc, sK[buf], 16 * kb, ds, c16, grp, sN[buf], k0, phi, own.tok, node);
+          else
+            f32_gather<HD>(acc, sK[buf], 16 * kb, ds, c16, grp);
         }
       });
 #pragma unroll
@@ -1918,6 +1964,7 @@ __global__ __launch_bounds__(F32Tile<HD>::kThreads) void attn_dkdv_f32_kernel(co
   __shared__ __align__(16) float sL[2][kF32Stage], sD[2][kF32Stage];
   __shared__ int2 sN[2][MASKED ? kF32Stage : 1];
   __shared__ uint32_t sKey[2][DROP ? kF32Stage : 1];   // row keys of the staged queries
+  __shared__ int sOdd[2];   // edge mask: the first token of a stage with a nonfinite q or dO row
   const int H = a.heads, item = blockIdx.x / H, head = blockIdx.x - item * H;
   if (item >= *a.count) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1939,10 +1986,16 @@ __global__ __launch_bounds__(F32Tile<HD>::kThreads) void attn_dkdv_f32_kernel(co
   f32x4 rQ[T::kPer], rG[T::kPer];
   float2 rR = make_float2(INFINITY, 0.f);
   int2 rN = make_int2(-1, -1);
+  int rT = 0;
+  if (MASKED) {
+    if (tid < 2) sOdd[tid] = -1;
+    __syncthreads();
+  }
   uint32_t rKey = 0;
   f32_stages(
       own.plo, phi, own.live,
       [&](int t0) {
+        rT = t0;
         f32_load<HD>(rQ, a.q, phi, H, head, t0);
         f32_load<HD>(rG, a.dout, phi, H, head, t0);
         if (tid < kF32Stage) {
@@ -1955,6 +2008,7 @@ __global__ __launch_bounds__(F32Tile<HD>::kThreads) void attn_dkdv_f32_kernel(co
       [&](int buf) {
         f32_store<HD>(sQ[buf], rQ);
         f32_store<HD>(sG[buf], rG);
+        if (MASKED && (nonfinite(rQ) || nonfinite(rG))) sOdd[buf] = rT;   // the same value from every thread
         if (tid < kF32Stage) {
           sL[buf][tid] = rR.x;
           sD[buf][tid] = rR.y;
@@ -1963,6 +2017,7 @@ __global__ __launch_bounds__(F32Tile<HD>::kThreads) void attn_dkdv_f32_kernel(co
         }
       },
       [&](int buf, int q0) {
+        const bool odd = MASKED && sOdd[buf] == q0;
 #pragma unroll
         for (int kb = 0; kb < KB; ++kb) {
           f32x4 x[NR], s[QB], ds[QB];
@@ -1979,17 +2034,22 @@ __global__ __launch_bounds__(F32Tile<HD>::kThreads) void attn_dkdv_f32_kernel(co
             const int2 pn = MASKED ? sN[buf][qi] : make_int2(0, 0);
 #pragma unroll
             for (int b = 0; b < QB; ++b) {
-              float p = fast_exp2(a.c * s[b][r] - lse2[r]);   // a query past the range has LSE2 = inf
-              if (MASKED) p = admissible_f32<true>(q0 + qi, phi, own.tok[b], pn, node[b]) ? p : 0.f;
+              const float p = fast_exp2(a.c * s[b][r] - lse2[r]);   // a query past the range has LSE2 = inf
+              const bool in = !MASKED || admissible_f32<true>(q0 + qi, phi, own.tok[b], pn, node[b]);
               const bool keep = !DROP || drop_keep(a.drop, sKey[buf][qi], ck[b], own.tok[b]);
               float dp = ds[b][r];
               if (DROP) dp = keep ? dp * a.drop.inv_keep : 0.f;
-              ds[b][r] = p * (dp - d[r]);
-              s[b][r] = keep ? p : 0.f;
+              ds[b][r] = in ? p * (dp - d[r]) : 0.f;
+              s[b][r] = in && keep ? p : 0.f;
             }
           }
-          f32_gather<HD>(dv, sG[buf], 16 * kb, s, c16, grp);
-          f32_gather<HD>(dk, sQ[buf], 16 * kb, ds, c16, grp);
+          if (MASKED && odd) {
+            f32_gather_admissible<HD>(dv, sG[buf], 16 * kb, s, c16, grp, sN[buf], q0, phi, own.tok, node);
+            f32_gather_admissible<HD>(dk, sQ[buf], 16 * kb, ds, c16, grp, sN[buf], q0, phi, own.tok, node);
+          } else {
+            f32_gather<HD>(dv, sG[buf], 16 * kb, s, c16, grp);
+            f32_gather<HD>(dk, sQ[buf], 16 * kb, ds, c16, grp);
+          }
         }
       });
 #pragma unroll

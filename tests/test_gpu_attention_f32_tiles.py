@@ -47,3 +47,37 @@ def test_dropout_lengths(device, hd):
     _close(out.detach().cpu(), ref, "out")
     for got, want, name in zip(grads, OA.varlen_attention_bwd(g, q, k, v, cu, cu, scale, dropout=(p, seed)), "qkv"):
         _close(got.cpu(), want, "d" + name)
+
+
+@pytest.mark.parametrize("hd,p", [(16, 0.0), (24, 0.2), (64, 0.0)])
+@pytest.mark.parametrize("what", ["k", "q", "g"])
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+def test_edge_mask_nonfinite_row_stays_with_its_neighbours(device, hd, p, what, value):
+    """An infinity or a NaN in one token's key, query or output gradient reaches no gradient of a token whose mask
+    leaves that token out: those equal the gradients with a finite row there (1e-5 of the largest value: they are
+    then added by another instruction)."""
+    rng = np.random.default_rng(1)
+    length, heads, odd = 200, 2, 77
+    src, dst = (rng.integers(0, 40, length) for _ in range(2))
+    shares = (src == src[odd]) | (src == dst[odd]) | (dst == src[odd]) | (dst == dst[odd])
+    cu = torch.as_tensor(cu_from_lengths([length])).to(device)
+    sd, dd = (torch.as_tensor(x.astype(np.int32)).to(device) for x in (src, dst))
+    grads = []
+    for fill in (0.5, value):
+        q, k, v, g = _inputs(length, length, 7, heads, hd)
+        {"q": q, "k": k, "g": g}[what][odd, :, 3] = fill
+        qd, kd, vd = (x.to(device).requires_grad_(True) for x in (q, k, v))
+        out = A.varlen_attention(qd, kd, vd, cu, cu, length, length, edge_src=sd, edge_dst=dd, dropout_p=p,
+                                 dropout_seed=11)
+        grads.append([x.cpu() for x in torch.autograd.grad(out, (qd, kd, vd), g.to(device))])
+    # a token's gradients take in what its neighbours' rows and statistics are: where the odd row spoils those (its
+    # neighbours' for a key), the tokens two steps away see it, too
+    near = shares
+    if what == "k":
+        near = np.array([bool((((src == src[i]) | (src == dst[i]) | (dst == src[i]) | (dst == dst[i])) & shares).any())
+                         for i in range(length)])
+    far, far_q = torch.as_tensor(~near), torch.as_tensor(~shares)
+    assert int(far_q.sum()) > 100 and int(far.sum()) > 30
+    for name, want, got in zip(("dq", "dk", "dv"), *grads):
+        keep = far_q if name == "dq" else far   # dq: the token's own statistics and its keys
+        _close(got[keep], want[keep].double(), name)
