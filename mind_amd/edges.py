@@ -357,7 +357,7 @@ class _EdgeTokenLinear(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, g):
-        from .esa.linear import column_sum, fused_ok, input_grad, weight_bias_grads
+        from .esa.linear import _library_rate, column_sum, fused_dx, fused_ok, weight_bias_grads
         x, w2, src, dst, edge_attr, w_e = ctx.saved_tensors
         src_csr, dst_csr = ctx.csrs
         n, f = x.shape
@@ -373,7 +373,10 @@ class _EdgeTokenLinear(torch.autograd.Function):
         dx = None
         if ctx.needs_input_grad[0]:
             terms = [(gs, w2[:d]), (gd, w2[d:])]
-            dx = input_grad(terms, fused_ok(gs, [w for _, w in terms], False))
+            if fused_ok(gs, [w for _, w in terms], False) and not _library_rate(gs, w2, True):
+                dx = fused_dx(terms)
+            else:   # one product over both halves, so that their sum is rounded once
+                dx = torch.cat((gs, gd), 1) @ w2
         dweight = None
         if ctx.needs_input_grad[1]:
             parts = [dw for dw, _ in weight_bias_grads([(gs, x), (gd, x)], [True, True], [False, False])]   # [D, F] each

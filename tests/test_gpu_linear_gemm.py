@@ -10,6 +10,7 @@ import pytest
 import torch
 from torch.nn import functional as F
 
+from mind_amd import edges
 from mind_amd.esa import linear as L
 
 pytestmark = pytest.mark.gpu
@@ -126,3 +127,23 @@ def test_other_sizes_use_the_library(device):
     empty = torch.empty(0, 64, device=device)
     (y,) = L.linear_outputs(empty, [(_randn(device, 64, 64), None)], True)
     assert y.shape == (0, 64)
+
+
+@pytest.mark.parametrize("out_features", [40, 64])   # 40: the library's product, 64: esa_linear_dx
+def test_edge_linear_input_gradient_is_rounded_once(device, out_features):
+    """dx = [gs | gd] [W_s; W_d] over the per-node sums of the edge gradients: one rounding of the sum of both halves.
+    The halves nearly cancel here (W_d = -W_s but for a tenth), so a rounding of the first alone would show."""
+    n, e, f = 300, 3000, 64
+    x = _randn(device, n, f, dtype=torch.bfloat16).requires_grad_(True)
+    ws = _randn(device, out_features, f, seed=1)
+    w = torch.cat((ws, -ws + 0.1 * _randn(device, out_features, f, seed=2)), 1).bfloat16().requires_grad_(True)
+    gen = torch.Generator().manual_seed(7)
+    src = torch.randint(n, (e,), generator=gen).int().to(device)
+    g = _randn(device, e, out_features, dtype=torch.bfloat16, seed=3)
+    out = edges.edge_token_linear(x, src, src, w, None)
+    (dx,) = torch.autograd.grad(out, x, g)
+    csr = edges.CSR.build(src, n)
+    gs = edges.segment_sum_csr(g, csr.indptr, csr.perm)
+    wd = w.detach()
+    ref, err = _product(torch.cat((gs, gs), 1), torch.cat((wd[:, :f], wd[:, f:]), 0).t())
+    _near(dx, ref, err + U[torch.bfloat16] * ref.abs())
