@@ -56,8 +56,8 @@ def _compute_dtype(x: torch.Tensor, params):
     block is not taken."""
     if not x.is_cuda or x.dtype != torch.float32 or x.shape[0] == 0:
         return None
-    if any(p is not None and p.dtype != torch.float32 for p in params):
-        return None
+    if any(p is not None and (p.dtype != torch.float32 or p.device != x.device) for p in params):
+        return None   # torch's own operations say what is wrong with a mixture
     if not torch.is_autocast_enabled("cuda"):
         return torch.float32
     return torch.bfloat16 if torch.get_autocast_dtype("cuda") == torch.bfloat16 else None
@@ -86,11 +86,22 @@ class _Setup:
         self.again = again   # (x, seed) -> the block's output through the separate functions
         self.mask = {}
         # whole stages of the fused products both ways, for the parameters themselves or (amp) their contiguous casts
-        layers = (mab.fc_q, mab.fc_k, mab.fc_v, mab.fc_o, *mlp)
         self.fused = all(fc.weight.dim() == 2 and fc.weight.is_contiguous() and max(fc.weight.shape) <= 16384
                          and fc.weight.shape[0] % 32 == 0 and fc.weight.shape[1] % 32 == 0
                          and (self.amp or all(t is None or (t.is_contiguous() and t.data_ptr() % 16 == 0)
-                                              for t in (fc.weight, fc.bias))) for fc in layers)
+                                              for t in (fc.weight, fc.bias)))
+                         for fc in (mab.fc_q, mab.fc_k, mab.fc_v, mab.fc_o, *mlp))
+
+
+def _fitting(d: int, mab, mlp) -> bool:
+    """Whether the Linears' parameters have the shapes that the block's kernels read: D to D around the attention, a
+    chain from D to D in the MLP (replaced or pruned parameters may not; F.linear checks them)."""
+    sizes, last = [(fc, d, d) for fc in (mab.fc_q, mab.fc_k, mab.fc_v, mab.fc_o)], d
+    for i, fc in enumerate(mlp):
+        out = d if i + 1 == len(mlp) else fc.weight.shape[0]
+        sizes.append((fc, out, last))
+        last = out
+    return all(fc.weight.shape == (o, i) and (fc.bias is None or fc.bias.shape == (o,)) for fc, o, i in sizes)
 
 
 def _rebuilt(setup, inputs, g, needs):
@@ -232,7 +243,7 @@ def sab_block(blk, x: torch.Tensor, tokens, masked: bool, attn_p: float, again) 
     params = _block_args(blk, mab, mlp)
     dt = _compute_dtype(x, params)
     if (dt is None or d % h or d // h not in HEAD_DIMS or not supported(x, ln) or not supported(x, blk.norm_mlp.ln)
-            or not plain(x, *params)):
+            or not _fitting(d, mab, mlp) or not plain(x, *params)):
         return None
     setup = _Setup(blk, tokens, mab, mlp, dt, attn_p, again)
     if masked:
@@ -246,7 +257,7 @@ class _PmaBlock(torch.autograd.Function):
         ln_w, ln_b, wq, bq, wk, bk, wv, bv, wo, bo = params[:10]
         (k_seeds, d), h, keeps = seeds.shape[1:], setup.heads, not isinstance(ctx, Unrecorded)
         _, xm, stats = _norm(setup, x, ln_w, ln_b, setup.eps[0], False)
-        s = cast_param(seeds, setup.dt).reshape(k_seeds, d)
+        s = cast_param(seeds, setup.dt).reshape(k_seeds, d).contiguous()
         weights = [cast_param(p, setup.dt) for p in (wq, wk, wv, wo)]
         biases = [cast_param(p, setup.dt) for p in (bq, bk, bv, bo)]
         (q,) = linear_outputs(s, [(weights[0], biases[0])], setup.fused)
@@ -307,6 +318,6 @@ def pma_block(blk, x: torch.Tensor, tokens, attn_p: float, again) -> torch.Tenso
     params = _block_args(blk, mab, mlp)
     dt = _compute_dtype(x, [seeds] + params)
     if (dt is None or d % h or d // h not in HEAD_DIMS or not supported(x, ln) or not supported(x, blk.norm_mlp.ln)
-            or not plain(x, seeds, *params)):
+            or not _fitting(d, mab, mlp) or not plain(x, seeds, *params)):
         return None
     return call(_PmaBlock, _Setup(blk, tokens, mab, mlp, dt, attn_p, again), x.contiguous(), seeds, *params)

@@ -5,10 +5,12 @@ T tokens of the batch (T = 131,072 in the encoder-stack benchmark) into a
 small [out, in] matrix: one GEMM with K = T has only a few dozen output tiles
 for 256 CUs.  ``weight_bias_grads`` cuts it over the tokens in one kernel that
 also sums the bias gradient's columns (esa_weight_grad: two launches for up to
-three Linears that share their rows), in fp32 and rounded to the weight's
+eight Linears that share their rows), in fp32 and rounded to the weight's
 dtype once, as the single GEMM's fp32 accumulator is.  Shapes and dtypes
 outside the kernel's run as S batched GEMMs over token chunks (``weight_grad``)
-and a column sum.  Forward (F.linear) and dx = g W are unchanged.
+and a column sum.  The packed blocks' forwards and input gradients run with
+what follows them in esa_linear_fwd / esa_linear_dx where those are faster;
+the autograd functions here keep F.linear and dx = g W.
 Under autocast the inputs are cast as autocast casts F.linear's (x, weight
 and bias to the autocast dtype); the autograd functions take the parameters
 in their own dtype and cast them inside, so the fp32 weight and bias
@@ -238,7 +240,7 @@ def fused_ok(x, weights, along: bool) -> bool:
     these sizes and layouts."""
     if not (x.is_cuda and x.dtype in _CODES and x.dim() == 2 and x.shape[0] < 2 ** 31):
         return False
-    return all(w.dtype == x.dtype and w.is_contiguous() and _aligned(w)
+    return all(w.dtype == x.dtype and w.device == x.device and w.is_contiguous() and _aligned(w)
                and _gemm_k(w.shape[1 if along else 0]) and _gemm_cols(w.shape[0 if along else 1], w.dtype)
                for w in weights)
 
@@ -253,11 +255,12 @@ def _library_rate(x, w, fused_passes: bool) -> bool:
 
 
 # The Linears of the packed blocks.  ``fused``: the caller's word that esa_linear_fwd / esa_linear_dx take the sizes
-# and layouts (``fused_ok`` of both directions).
+# and the weights (``fused_ok`` of both directions).  Rows that come from the caller of the block (the pooling's seeds,
+# the output's gradient) may start anywhere, so the alignment of the rows is looked at here.
 
 def linear_outputs(x, pairs, fused: bool) -> list[torch.Tensor]:
     """[x W^T + b for (W, b) in pairs]: one launch of esa_linear_fwd, or ``linear_fwd``."""
-    if fused and not _library_rate(x, pairs[0][0], False):
+    if fused and _aligned(x) and not _library_rate(x, pairs[0][0], False):
         return fused_fwd(x, pairs)
     return linear_fwd(x, pairs)
 
@@ -291,7 +294,8 @@ def input_grad(pairs, fused: bool, base=None, mish_z=None) -> torch.Tensor:
     """[base +] sum of g W over the (g, W) pairs, or (g W) mish'(mish_z); all of one dtype."""
     from .activations import mish_backward
     (g, w) = pairs[0]
-    if fused and not _library_rate(g, w, len(pairs) > 1 or base is not None or mish_z is not None):
+    if fused and _aligned(g) and (base is None or _aligned(base)) and not _library_rate(
+            g, w, len(pairs) > 1 or base is not None or mish_z is not None):
         return fused_dx(pairs, base, mish_z)
     dx = g.mm(w) if base is None else torch.addmm(base, g, w)
     for g, w in pairs[1:]:

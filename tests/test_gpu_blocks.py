@@ -136,3 +136,40 @@ def test_strided_and_misaligned_parameters(device, amp):
         g = torch.randn(tokens.num_tokens, 64, device=device)
         _both(lambda: blocks.sab_block(blk, x, tokens, False, 0.0, None),
               lambda: masked_layers._sab_separate(blk, x, tokens), x, [blk.mlp.mlp[2].weight, blk.norm.ln.weight], g, amp)
+
+
+def _off_boundary(t):
+    """t's values in memory that starts 4 bytes past a 16-byte boundary."""
+    flat = torch.empty(t.numel() + 1, device=t.device)
+    return flat[1:].view(t.shape).copy_(t)
+
+
+@pytest.mark.parametrize("amp", [False, True])
+def test_rows_off_a_boundary(device, amp):
+    """Seeds and output gradients that are views into a larger buffer, as flat parameter and gradient buffers hold
+    them: the products over them go where no alignment is asked for."""
+    tokens = _tokens(device, False)
+    torch.manual_seed(5)
+    blk = masked_layers.PMAComplete(64, 4, 2, "LN", use_mlp=False, xformers_or_torch_attn="hip").to(device).train()
+    blk.pma.S = torch.nn.Parameter(_off_boundary(blk.pma.S.detach()))
+    x = torch.randn(tokens.num_tokens, 64, device=device, requires_grad=True)
+    g = _off_boundary(torch.randn(tokens.batch_size, 2, 64, device=device))
+    params = [p for n, p in blk.named_parameters() if "norm_mlp" not in n]
+    _both(lambda: blocks.pma_block(blk, x, tokens, 0.0, None), lambda: masked_layers._pma_separate(blk, x, tokens), x,
+          params, g, amp)
+
+
+@pytest.mark.parametrize("amp", [False, True])
+def test_parameters_that_do_not_fit(device, amp):
+    """Parameters left on the host or of other shapes raise torch's errors; no kernel takes their addresses."""
+    tokens = _tokens(device, False)
+    x = torch.randn(tokens.num_tokens, 64, device=device)
+    for change in (lambda fc: fc.cpu(), lambda fc: setattr(fc, "weight", torch.nn.Parameter(fc.weight.detach()[:, :32])),
+                   lambda fc: setattr(fc, "bias", torch.nn.Parameter(fc.bias.detach()[:32]))):
+        for pick in (lambda b: b.sab.mab.fc_o, lambda b: b.mlp.mlp[2]):
+            blk = _sab(device, 0, 2)
+            change(pick(blk))
+            with torch.autocast("cuda", torch.bfloat16, enabled=amp):
+                assert blocks.sab_block(blk, x, tokens, False, 0.0, None) is None
+                with pytest.raises(RuntimeError):
+                    masked_layers._sab_forward_packed(blk, x, tokens)
