@@ -1400,7 +1400,7 @@ DEVI bool admissible_f32(int p, int phi, int oi, int2 pn, int2 own) {
 // thread per (token, head) with vector FMAs, before: forward / dQ / dK/dV of
 // 64 small molecules (21,752 tokens, 8 heads of 16) 135 / 192 / 214 us dense and
 // 143 / 234 / 241 us with the edge mask, now
-// 90 / 103 / 122 and 100 / 119 / 149 us; 8 heads of 64, dense: 445 / 1054 / 2071
+// 90 / 103 / 122 and 103 / 123 / 156 us; 8 heads of 64, dense: 445 / 1054 / 2071
 // -> 221 / 296 / 406 us (93-107 of the 154 TFLOP/s of a large fp32 product).
 constexpr int kF32Stage = 64;
 
@@ -1490,6 +1490,9 @@ DEVI void f32_gather(f32x4 (&acc)[F32Tile<HD>::QB][F32Tile<HD>::NR], const float
 
 // The same over the admissible pairs alone, by vector FMAs: with the edge mask, where a partner's row holds an infinity
 // or a NaN, which times the zero weight of a pair that the mask leaves out would reach tokens that do not attend it.
+// A block that has staged one walks its partners again with it: as a branch inside the one walk it took the registers
+// of two of four waves per SIMD (64 small molecules: dK/dV 174 us, 156 with the second walk and 149 without any check;
+// dQ 127, 123 and 119).  The masked backward kernels are held to the four waves for it; neither spills.
 template <int HD>
 DEVI void f32_gather_admissible(f32x4 (&acc)[F32Tile<HD>::QB][F32Tile<HD>::NR],
                                 const float (*rows)[F32Tile<HD>::kStride], int p0, const f32x4 (&w)[F32Tile<HD>::QB],
@@ -1868,13 +1871,13 @@ __global__ __launch_bounds__(256) void attn_dkdv_few_kernel(const AttnFewArgs a)
 
 // dQ = scale * sum_j P_ij (dP_ij - D_i) k_j, P recomputed from the saved LSE.
 template <bool MASKED, int HD, bool DROP>
-__global__ __launch_bounds__(F32Tile<HD>::kThreads) void attn_dq_f32_kernel(const AttnF32Args a) {
+__global__ __launch_bounds__(F32Tile<HD>::kThreads) __attribute__((amdgpu_waves_per_eu(
+    MASKED ? 4 : 1))) void attn_dq_f32_kernel(const AttnF32Args a) {
   using T = F32Tile<HD>;
   constexpr int NR = T::NR, QB = T::QB, KB = kF32Stage / 16;
   __shared__ __align__(16) typename T::Rows sK[2], sV[2];
   __shared__ int2 sN[2][MASKED ? kF32Stage : 1];
   __shared__ uint32_t sKey[2][DROP ? kF32Stage : 1];   // column keys of the staged keys
-  __shared__ int sOdd[2];   // edge mask: the first token of a stage with a nonfinite key row
   const int H = a.heads, item = blockIdx.x / H, head = blockIdx.x - item * H;
   if (item >= *a.count) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1897,59 +1900,70 @@ __global__ __launch_bounds__(F32Tile<HD>::kThreads) void attn_dq_f32_kernel(cons
   }
   f32x4 rK[T::kPer], rV[T::kPer];
   int2 rN = make_int2(-1, -1);
-  int rT = 0;
-  if (MASKED) {
-    if (tid < 2) sOdd[tid] = -1;
-    __syncthreads();
-  }
   uint32_t rKey = 0;
-  f32_stages(
-      own.plo, phi, own.live,
-      [&](int t0) {
-        rT = t0;
-        f32_load<HD>(rK, a.k, phi, H, head, t0);
-        f32_load<HD>(rV, a.v, phi, H, head, t0);
-        if (MASKED && tid < kF32Stage) rN = t0 + tid < phi ? a.nodes[t0 + tid] : make_int2(-1, -1);
-        if (DROP && tid < kF32Stage) rKey = drop_col(a.drop, t0 + tid);
-      },
-      [&](int buf) {
-        f32_store<HD>(sK[buf], rK);
-        f32_store<HD>(sV[buf], rV);
-        if (MASKED && nonfinite(rK)) sOdd[buf] = rT;   // the same value from every thread
-        if (MASKED && tid < kF32Stage) sN[buf][tid] = rN;
-        if (DROP && tid < kF32Stage) sKey[buf][tid] = rKey;
-      },
-      [&](int buf, int k0) {
-        const bool tail = k0 + kF32Stage > phi, odd = MASKED && sOdd[buf] == k0;
+  bool odd = false;   // edge mask: this thread staged an infinity or a NaN of a key
+  auto walk = [&](auto checked) {
+    f32_stages(
+        own.plo, phi, own.live,
+        [&](int t0) {
+          f32_load<HD>(rK, a.k, phi, H, head, t0);
+          f32_load<HD>(rV, a.v, phi, H, head, t0);
+          if (MASKED && tid < kF32Stage) rN = t0 + tid < phi ? a.nodes[t0 + tid] : make_int2(-1, -1);
+          if (DROP && tid < kF32Stage) rKey = drop_col(a.drop, t0 + tid);
+        },
+        [&](int buf) {
+          f32_store<HD>(sK[buf], rK);
+          f32_store<HD>(sV[buf], rV);
+          if (MASKED) odd |= nonfinite(rK);
+          if (MASKED && tid < kF32Stage) sN[buf][tid] = rN;
+          if (DROP && tid < kF32Stage) sKey[buf][tid] = rKey;
+        },
+        [&](int buf, int k0) {
+          const bool tail = k0 + kF32Stage > phi;
+          auto block = [&](int kb) {
+            f32x4 x[NR], s[QB], ds[QB];
+            f32_rows<HD>(x, sK[buf], 16 * kb, c16, grp);
 #pragma unroll
-        for (int kb = 0; kb < KB; ++kb) {
-          f32x4 x[NR], s[QB], ds[QB];
-          f32_rows<HD>(x, sK[buf], 16 * kb, c16, grp);
+            for (int b = 0; b < QB; ++b) s[b] = f32_product<HD>(x, q[b]);
+            f32_rows<HD>(x, sV[buf], 16 * kb, c16, grp);
 #pragma unroll
-          for (int b = 0; b < QB; ++b) s[b] = f32_product<HD>(x, q[b]);
-          f32_rows<HD>(x, sV[buf], 16 * kb, c16, grp);
+            for (int b = 0; b < QB; ++b) ds[b] = f32_product<HD>(x, g[b]);
 #pragma unroll
-          for (int b = 0; b < QB; ++b) ds[b] = f32_product<HD>(x, g[b]);
+            for (int r = 0; r < 4; ++r) {
+              const int key = 16 * kb + 4 * grp + r;
+              const int2 pn = MASKED ? sN[buf][key] : make_int2(0, 0);
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int key = 16 * kb + 4 * grp + r;
-            const int2 pn = MASKED ? sN[buf][key] : make_int2(0, 0);
-#pragma unroll
-            for (int b = 0; b < QB; ++b) {
-              const float p = fast_exp2(a.c * s[b][r] - rs[b].x);
-              float dp = ds[b][r];
-              if (DROP) dp = drop_keep(a.drop, rk[b], sKey[buf][key], k0 + key) ? dp * a.drop.inv_keep : 0.f;
-              ds[b][r] = p * (dp - rs[b].y);
-              if (MASKED || tail)
-                ds[b][r] = admissible_f32<MASKED>(k0 + key, phi, own.tok[b], pn, node[b]) ? ds[b][r] : 0.f;
+              for (int b = 0; b < QB; ++b) {
+                const float p = fast_exp2(a.c * s[b][r] - rs[b].x);
+                float dp = ds[b][r];
+                if (DROP) dp = drop_keep(a.drop, rk[b], sKey[buf][key], k0 + key) ? dp * a.drop.inv_keep : 0.f;
+                ds[b][r] = p * (dp - rs[b].y);
+                if (MASKED || tail)
+                  ds[b][r] = admissible_f32<MASKED>(k0 + key, phi, own.tok[b], pn, node[b]) ? ds[b][r] : 0.f;
+              }
             }
+            if constexpr (decltype(checked)::value)
+              f32_gather_admissible<HD>(acc, sK[buf], 16 * kb, ds, c16, grp, sN[buf], k0, phi, own.tok, node);
+            else
+              f32_gather<HD>(acc, sK[buf], 16 * kb, ds, c16, grp);
+          };
+          if constexpr (decltype(checked)::value) {
+#pragma unroll 1
+            for (int kb = 0; kb < KB; ++kb) block(kb);
+          } else {
+#pragma unroll
+            for (int kb = 0; kb < KB; ++kb) block(kb);
           }
-          if (MASKED && odd)
-            f32_gather_admissible<HD>(acc, sK[buf], 16 * kb, ds, c16, grp, sN[buf], k0, phi, own.tok, node);
-          else
-            f32_gather<HD>(acc, sK[buf], 16 * kb, ds, c16, grp);
-        }
-      });
+        });
+  };
+  walk(std::false_type());
+  if (MASKED && __syncthreads_or(odd)) {   // again, over the admissible pairs alone
+#pragma unroll
+    for (int b = 0; b < QB; ++b)
+#pragma unroll
+      for (int c = 0; c < NR; ++c) acc[b][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    walk(std::bool_constant<MASKED>());
+  }
 #pragma unroll
   for (int b = 0; b < QB; ++b)
     if (own.valid[b]) f32_write<HD>(a.dq, acc[b], a.scale, own.tok[b], H, head, grp);
@@ -1957,14 +1971,14 @@ __global__ __launch_bounds__(F32Tile<HD>::kThreads) void attn_dq_f32_kernel(cons
 
 // dV = sum_i P_ij dO_i, dK = scale * sum_i P_ij (dP_ij - D_i) q_i; the partners are queries with their (LSE2, D).
 template <bool MASKED, int HD, bool DROP>
-__global__ __launch_bounds__(F32Tile<HD>::kThreads) void attn_dkdv_f32_kernel(const AttnF32Args a) {
+__global__ __launch_bounds__(F32Tile<HD>::kThreads) __attribute__((amdgpu_waves_per_eu(
+    MASKED ? 4 : 1))) void attn_dkdv_f32_kernel(const AttnF32Args a) {
   using T = F32Tile<HD>;
   constexpr int NR = T::NR, QB = T::QB, KB = kF32Stage / 16;
   __shared__ __align__(16) typename T::Rows sQ[2], sG[2];
   __shared__ __align__(16) float sL[2][kF32Stage], sD[2][kF32Stage];
   __shared__ int2 sN[2][MASKED ? kF32Stage : 1];
   __shared__ uint32_t sKey[2][DROP ? kF32Stage : 1];   // row keys of the staged queries
-  __shared__ int sOdd[2];   // edge mask: the first token of a stage with a nonfinite q or dO row
   const int H = a.heads, item = blockIdx.x / H, head = blockIdx.x - item * H;
   if (item >= *a.count) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1986,72 +2000,82 @@ __global__ __launch_bounds__(F32Tile<HD>::kThreads) void attn_dkdv_f32_kernel(co
   f32x4 rQ[T::kPer], rG[T::kPer];
   float2 rR = make_float2(INFINITY, 0.f);
   int2 rN = make_int2(-1, -1);
-  int rT = 0;
-  if (MASKED) {
-    if (tid < 2) sOdd[tid] = -1;
-    __syncthreads();
-  }
   uint32_t rKey = 0;
-  f32_stages(
-      own.plo, phi, own.live,
-      [&](int t0) {
-        rT = t0;
-        f32_load<HD>(rQ, a.q, phi, H, head, t0);
-        f32_load<HD>(rG, a.dout, phi, H, head, t0);
-        if (tid < kF32Stage) {
-          const bool in = t0 + tid < phi;
-          rR = in ? a.rows[(size_t)head * a.tq_pad + t0 + tid] : make_float2(INFINITY, 0.f);
-          if (MASKED) rN = in ? a.nodes[t0 + tid] : make_int2(-1, -1);
-          if (DROP) rKey = drop_row(a.drop, t0 + tid, head);
-        }
-      },
-      [&](int buf) {
-        f32_store<HD>(sQ[buf], rQ);
-        f32_store<HD>(sG[buf], rG);
-        if (MASKED && (nonfinite(rQ) || nonfinite(rG))) sOdd[buf] = rT;   // the same value from every thread
-        if (tid < kF32Stage) {
-          sL[buf][tid] = rR.x;
-          sD[buf][tid] = rR.y;
-          if (MASKED) sN[buf][tid] = rN;
-          if (DROP) sKey[buf][tid] = rKey;
-        }
-      },
-      [&](int buf, int q0) {
-        const bool odd = MASKED && sOdd[buf] == q0;
+  bool odd = false;   // edge mask: this thread staged an infinity or a NaN of a q or dO row
+  auto walk = [&](auto checked) {
+    f32_stages(
+        own.plo, phi, own.live,
+        [&](int t0) {
+          f32_load<HD>(rQ, a.q, phi, H, head, t0);
+          f32_load<HD>(rG, a.dout, phi, H, head, t0);
+          if (tid < kF32Stage) {
+            const bool in = t0 + tid < phi;
+            rR = in ? a.rows[(size_t)head * a.tq_pad + t0 + tid] : make_float2(INFINITY, 0.f);
+            if (MASKED) rN = in ? a.nodes[t0 + tid] : make_int2(-1, -1);
+            if (DROP) rKey = drop_row(a.drop, t0 + tid, head);
+          }
+        },
+        [&](int buf) {
+          f32_store<HD>(sQ[buf], rQ);
+          f32_store<HD>(sG[buf], rG);
+          if (MASKED) odd |= nonfinite(rQ) || nonfinite(rG);
+          if (tid < kF32Stage) {
+            sL[buf][tid] = rR.x;
+            sD[buf][tid] = rR.y;
+            if (MASKED) sN[buf][tid] = rN;
+            if (DROP) sKey[buf][tid] = rKey;
+          }
+        },
+        [&](int buf, int q0) {
+          auto block = [&](int kb) {
+            f32x4 x[NR], s[QB], ds[QB];
+            f32_rows<HD>(x, sQ[buf], 16 * kb, c16, grp);
 #pragma unroll
-        for (int kb = 0; kb < KB; ++kb) {
-          f32x4 x[NR], s[QB], ds[QB];
-          f32_rows<HD>(x, sQ[buf], 16 * kb, c16, grp);
+            for (int b = 0; b < QB; ++b) s[b] = f32_product<HD>(x, kx[b]);
+            f32_rows<HD>(x, sG[buf], 16 * kb, c16, grp);
 #pragma unroll
-          for (int b = 0; b < QB; ++b) s[b] = f32_product<HD>(x, kx[b]);
-          f32_rows<HD>(x, sG[buf], 16 * kb, c16, grp);
+            for (int b = 0; b < QB; ++b) ds[b] = f32_product<HD>(x, vx[b]);
+            const f32x4 lse2 = ldsf4(&sL[buf][16 * kb + 4 * grp]), d = ldsf4(&sD[buf][16 * kb + 4 * grp]);
 #pragma unroll
-          for (int b = 0; b < QB; ++b) ds[b] = f32_product<HD>(x, vx[b]);
-          const f32x4 lse2 = ldsf4(&sL[buf][16 * kb + 4 * grp]), d = ldsf4(&sD[buf][16 * kb + 4 * grp]);
+            for (int r = 0; r < 4; ++r) {
+              const int qi = 16 * kb + 4 * grp + r;
+              const int2 pn = MASKED ? sN[buf][qi] : make_int2(0, 0);
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int qi = 16 * kb + 4 * grp + r;
-            const int2 pn = MASKED ? sN[buf][qi] : make_int2(0, 0);
-#pragma unroll
-            for (int b = 0; b < QB; ++b) {
-              const float p = fast_exp2(a.c * s[b][r] - lse2[r]);   // a query past the range has LSE2 = inf
-              const bool in = !MASKED || admissible_f32<true>(q0 + qi, phi, own.tok[b], pn, node[b]);
-              const bool keep = !DROP || drop_keep(a.drop, sKey[buf][qi], ck[b], own.tok[b]);
-              float dp = ds[b][r];
-              if (DROP) dp = keep ? dp * a.drop.inv_keep : 0.f;
-              ds[b][r] = in ? p * (dp - d[r]) : 0.f;
-              s[b][r] = in && keep ? p : 0.f;
+              for (int b = 0; b < QB; ++b) {
+                const float p = fast_exp2(a.c * s[b][r] - lse2[r]);   // a query past the range has LSE2 = inf
+                const bool in = !MASKED || admissible_f32<true>(q0 + qi, phi, own.tok[b], pn, node[b]);
+                const bool keep = !DROP || drop_keep(a.drop, sKey[buf][qi], ck[b], own.tok[b]);
+                float dp = ds[b][r];
+                if (DROP) dp = keep ? dp * a.drop.inv_keep : 0.f;
+                ds[b][r] = in ? p * (dp - d[r]) : 0.f;
+                s[b][r] = in && keep ? p : 0.f;
+              }
             }
-          }
-          if (MASKED && odd) {
-            f32_gather_admissible<HD>(dv, sG[buf], 16 * kb, s, c16, grp, sN[buf], q0, phi, own.tok, node);
-            f32_gather_admissible<HD>(dk, sQ[buf], 16 * kb, ds, c16, grp, sN[buf], q0, phi, own.tok, node);
+            if constexpr (decltype(checked)::value) {
+              f32_gather_admissible<HD>(dv, sG[buf], 16 * kb, s, c16, grp, sN[buf], q0, phi, own.tok, node);
+              f32_gather_admissible<HD>(dk, sQ[buf], 16 * kb, ds, c16, grp, sN[buf], q0, phi, own.tok, node);
+            } else {
+              f32_gather<HD>(dv, sG[buf], 16 * kb, s, c16, grp);
+              f32_gather<HD>(dk, sQ[buf], 16 * kb, ds, c16, grp);
+            }
+          };
+          if constexpr (decltype(checked)::value) {
+#pragma unroll 1
+            for (int kb = 0; kb < KB; ++kb) block(kb);
           } else {
-            f32_gather<HD>(dv, sG[buf], 16 * kb, s, c16, grp);
-            f32_gather<HD>(dk, sQ[buf], 16 * kb, ds, c16, grp);
+#pragma unroll
+            for (int kb = 0; kb < KB; ++kb) block(kb);
           }
-        }
-      });
+        });
+  };
+  walk(std::false_type());
+  if (MASKED && __syncthreads_or(odd)) {   // again, over the admissible pairs alone
+#pragma unroll
+    for (int b = 0; b < QB; ++b)
+#pragma unroll
+      for (int c = 0; c < NR; ++c) dk[b][c] = dv[b][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    walk(std::bool_constant<MASKED>());
+  }
 #pragma unroll
   for (int b = 0; b < QB; ++b)
     if (own.valid[b]) {
