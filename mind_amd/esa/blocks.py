@@ -20,6 +20,7 @@ functions, which also serve a backward that is differentiated again.
 from __future__ import annotations
 
 import math
+from types import SimpleNamespace
 
 import torch
 from torch import nn
@@ -83,7 +84,7 @@ class _Setup:
         self.heads, self.max_items, self.cu = mab.num_heads, tokens.max_items, tokens.cu_seqlens
         self.dt, self.amp, self.n_mlp = dt, dt != torch.float32, len(mlp)
         self.dropout = (dropout_p, attention.draw_dropout_seed() if dropout_p > 0.0 else 0)
-        self.again = again   # (x, seed) -> the block's output through the separate functions
+        self.again = again   # (block, x, seed) -> the block's output through the separate functions
         self.mask = {}
         # whole stages of the fused products both ways, for the parameters themselves or (amp) their contiguous casts
         self.fused = all(fc.weight.dim() == 2 and fc.weight.is_contiguous() and max(fc.weight.shape) <= 16384
@@ -104,12 +105,46 @@ def _fitting(d: int, mab, mlp) -> bool:
     return all(fc.weight.shape == (o, i) and (fc.bias is None or fc.bias.shape == (o,)) for fc, o, i in sizes)
 
 
-def _rebuilt(setup, inputs, g, needs):
-    """The inputs' gradients by the separate functions, for a backward that is itself differentiated."""
+def _layer(cls, **attrs):
+    """A module of type ``cls`` with these plain attributes and nothing registered."""
+    m = cls.__new__(cls)
+    nn.Module.__init__(m)
+    m.__dict__.update(attrs)
+    return m
+
+
+def _stand_in(setup, d, params, seeds=None):
+    """The block as its forward found it, for the separate functions: these parameters (``_block_args``' order), its
+    dropout.  The module itself may hold others by now (functional calls) or be in another mode."""
+    it = iter(params)
+
+    def norm(eps):
+        return SimpleNamespace(ln=_layer(nn.LayerNorm, weight=next(it), bias=next(it), normalized_shape=(d,), eps=eps))
+
+    def linear():
+        return _layer(nn.Linear, weight=next(it), bias=next(it))
+
+    blk = SimpleNamespace(idx=1 if setup.mask else 0, use_mlp=setup.n_mlp > 0, residual_dropout=0.0,
+                          norm=norm(setup.eps[0]))
+    mab = SimpleNamespace(fc_q=linear(), fc_k=linear(), fc_v=linear(), fc_o=linear(), num_heads=setup.heads, dim_V=d,
+                          dropout_p=setup.dropout[0], training=True)
+    blk.sab = blk.pma = SimpleNamespace(mab=mab, S=seeds)
+    if setup.n_mlp:
+        blk.norm_mlp = norm(setup.eps[1])
+        layers = [linear()]
+        for _ in range(setup.n_mlp - 1):
+            layers += (Mish(), linear())
+        blk.mlp = _layer(SmallMLP, mlp=layers)
+    return blk
+
+
+def _rebuilt(setup, x, params, g, needs, seeds=None):
+    """The gradients of x, the seeds (where there are any) and the parameters by the separate functions, for a
+    backward that is itself differentiated."""
+    inputs = [x] + ([] if seeds is None else [seeds]) + list(params)
     with torch.enable_grad(), torch.autocast("cuda", setup.dt if setup.amp else None, enabled=setup.amp):
-        out = setup.again(inputs[0], setup.dropout[1])
-        wanted = [t for t, n in zip(inputs, needs) if n]
-        got = iter(torch.autograd.grad(out, wanted, g, create_graph=True, allow_unused=True))
+        out = setup.again(_stand_in(setup, x.shape[1], params, seeds), x, setup.dropout[1])
+        got = iter(torch.autograd.grad(out, [t for t, n in zip(inputs, needs) if n], g, create_graph=True))
     return tuple(next(got) if n else None for n in needs)
 
 
@@ -206,8 +241,8 @@ class _SabBlock(torch.autograd.Function):
     def backward(ctx, g):
         setup, needs, tensors = ctx.setup, ctx.needs_input_grad[1:], ctx.saved_tensors
         if torch.is_grad_enabled():
-            n = ctx.n_keep + 1 + len(ctx.mask_keys)
-            return (None,) + _rebuilt(setup, (tensors[0],) + tensors[n:], g, needs)
+            params = tensors[ctx.n_keep + 1 + len(ctx.mask_keys):]
+            return (None,) + _rebuilt(setup, tensors[0], params, g, needs)
         x, ln_w, stats, xm, q, k, v, o, lse, z, wq, wk, wv, wo = tensors[:14]
         cu, mask = tensors[ctx.n_keep], dict(zip(ctx.mask_keys, tensors[ctx.n_keep + 1:]))
         t, d = x.shape
@@ -234,7 +269,7 @@ class _SabBlock(torch.autograd.Function):
 
 def sab_block(blk, x: torch.Tensor, tokens, masked: bool, attn_p: float, again) -> torch.Tensor | None:
     """The SABComplete block ``blk`` on packed tokens x [T, D], or None where this path does not take the call.
-    ``again(x, seed)`` computes the same through the separate functions."""
+    ``again(blk, x, seed)`` computes a block through the separate functions."""
     mab, ln = blk.sab.mab, blk.norm.ln
     mlp = _mlp_layers(blk)
     if mlp is None or blk.residual_dropout > 0 or x.dim() != 2 or mab.dim_V != x.shape[1]:
@@ -280,7 +315,8 @@ class _PmaBlock(torch.autograd.Function):
     def backward(ctx, g):
         setup, needs, tensors = ctx.setup, ctx.needs_input_grad[1:], ctx.saved_tensors
         if torch.is_grad_enabled():
-            return (None,) + _rebuilt(setup, (tensors[0],) + tensors[ctx.n_keep + 1:], g, needs)
+            seeds, *params = tensors[ctx.n_keep + 1:]
+            return (None,) + _rebuilt(setup, tensors[0], params, g, needs, seeds)
         x, ln_w, stats, xm, s, q, k, v, o, lse, z, wq, wk, wv, wo = tensors[:15]
         cu, seeds = tensors[ctx.n_keep:ctx.n_keep + 2]
         d = x.shape[1]

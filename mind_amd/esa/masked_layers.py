@@ -177,7 +177,7 @@ def _sab_forward_packed(blk: "SABComplete", X: torch.Tensor, tokens: PackedSets)
     """SABComplete.forward (pre-norm, esa/masked_layers.py:418-483) on packed tokens X [T, D]: the masked
     layers (idx 1) apply the descriptor's mask, the unmasked ones (idx 0) attend over each graph's tokens."""
     out = sab_block(blk, X, tokens, blk.idx == 1, attn_dropout(blk.sab.mab),
-                    lambda x, seed: _sab_separate(blk, x, tokens, seed))
+                    lambda b, x, seed: _sab_separate(b, x, tokens, seed))
     return _sab_separate(blk, X, tokens) if out is None else out
 
 
@@ -206,7 +206,7 @@ def _sab_separate(blk: "SABComplete", X: torch.Tensor, tokens: PackedSets, seed:
 def _pma_forward_packed(blk: "PMAComplete", X: torch.Tensor, tokens: PackedSets) -> torch.Tensor:
     """PMAComplete.forward (esa/masked_layers.py:583-610) with packed keys X [T, D] -> [B, k, D]: the seeds
     of each graph attend over its tokens."""
-    out = pma_block(blk, X, tokens, attn_dropout(blk.pma.mab), lambda x, seed: _pma_separate(blk, x, tokens, seed))
+    out = pma_block(blk, X, tokens, attn_dropout(blk.pma.mab), lambda b, x, seed: _pma_separate(b, x, tokens, seed))
     return _pma_separate(blk, X, tokens) if out is None else out
 
 

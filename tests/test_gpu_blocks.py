@@ -173,3 +173,84 @@ def test_parameters_that_do_not_fit(device, amp):
                 assert blocks.sab_block(blk, x, tokens, False, 0.0, None) is None
                 with pytest.raises(RuntimeError):
                     masked_layers._sab_forward_packed(blk, x, tokens)
+
+
+def _packed(blk, tokens):
+    """(the block in one node, through the separate functions): the packed forwards of a SAB or PMA block."""
+    one, apart = ((masked_layers._sab_forward_packed, masked_layers._sab_separate) if hasattr(blk, "sab") else
+                  (masked_layers._pma_forward_packed, masked_layers._pma_separate))
+    return (lambda x: one(blk, x, tokens)), (lambda x: apart(blk, x, tokens))
+
+
+def _pma(device, mlp=True, dropout=0.0, k_seeds=2):
+    torch.manual_seed(5)
+    return masked_layers.PMAComplete(64, 4, k_seeds, "LN", dropout=dropout, use_mlp=mlp, mlp_hidden_size=96,
+                                     num_mlp_layers=2, xformers_or_torch_attn="hip").to(device).train()
+
+
+def _used(blk):
+    return {n: p for n, p in blk.named_parameters() if blk.use_mlp or "norm_mlp" not in n}
+
+
+def _scale(grads, i):
+    """What gradient i is compared with: itself; a Linear's bias, which sums the rows that its weight (the tensor
+    before it) sums against inputs of about 1, with the larger of both (fc_k's is zero but for rounding)."""
+    return max(float(t.double().norm()) for t in grads[max(i - 1, 0):i + 1]) if grads[i].dim() == 1 else float(
+        grads[i].double().norm())
+
+
+def _agree(got, want, bar, names):
+    for i, (a, b, name) in enumerate(zip(got, want, names)):
+        size = _scale(want, i) if name.endswith("bias") and ".ln." not in name else float(b.double().norm())
+        assert a is not None and a.dtype == b.dtype and a.shape == b.shape, name
+        assert float((a.double() - b.double()).norm()) <= bar * size, name
+
+
+class _Held(torch.nn.Module):
+    """A block as a submodule whose forward is its packed one, to be called with other parameters."""
+
+    def __init__(self, blk, fn):
+        super().__init__()
+        self.blk, self.fn = blk, fn
+
+    def forward(self, x):
+        return self.fn(x)
+
+
+@pytest.mark.parametrize("amp", [False, True])
+@pytest.mark.parametrize("pma", [False, True])
+def test_differentiated_again_with_other_parameters(device, amp, pma):
+    """Parameters substituted for a call (fast weights): a backward that is differentiated again gives the gradients
+    of those, and of the weights they are made from."""
+    tokens = _tokens(device, False)
+    blk = _pma(device) if pma else _sab(device, 1, 3)
+    base = {n: (p.detach() * 0.5 + 0.01).requires_grad_(True) for n, p in _used(blk).items()}
+    x = torch.randn(tokens.num_tokens, 64, device=device, requires_grad=True)
+    name, grads, again = "mlp.mlp.2.weight" if pma else "mlp.mlp.4.weight", [], []
+    for fn in _packed(blk, tokens):
+        fast = {n: p * 1.5 for n, p in base.items()}
+        with torch.autocast("cuda", torch.bfloat16, enabled=amp):
+            out = torch.func.functional_call(_Held(blk, fn), {"blk." + n: p for n, p in fast.items()}, (x,))
+        grads.append(torch.autograd.grad(out.float().sin().sum(), [x, *fast.values(), *base.values()], create_graph=True))
+        if not amp:   # the bf16 weight gradients' products (with fp32 results) have no derivative in torch
+            gw = grads[-1][1 + list(fast).index(name)]
+            again.append(torch.autograd.grad(gw.square().sum(), [fast[name], base[name]]))
+    _agree(*grads, 2.0 ** -7 if amp else 1e-5, ["x", *fast, *base])
+    if not amp:
+        _agree(*again, 2e-5, [name, name])
+
+
+@pytest.mark.parametrize("pma", [False, True])
+def test_differentiated_again_in_another_mode(device, pma):
+    """The module leaves training mode between its forward and a backward that is differentiated again: the
+    gradients are those of the forward, attention dropout included."""
+    tokens = _tokens(device, False)
+    blk = _pma(device, dropout=0.3) if pma else _sab(device, 1, 2, 0.3)
+    x = torch.randn(tokens.num_tokens, 64, device=device, requires_grad=True)
+    inputs, grads = [x, *_used(blk).values()], []
+    for again in (True, False):
+        torch.manual_seed(9)
+        out = _packed(blk.train(), tokens)[0](x)
+        blk.eval()
+        grads.append(torch.autograd.grad(out.sin().sum(), inputs, create_graph=again))
+    _agree(*grads, 1e-5, ["x", *_used(blk)])
