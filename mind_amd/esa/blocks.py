@@ -138,9 +138,20 @@ def _stand_in(setup, d, params, seeds=None):
     return blk
 
 
-def _rebuilt(setup, x, params, g, needs, seeds=None):
+def _versions(params, recorded: bool):
+    """How often each parameter has been changed in place so far."""
+    return [p._version for p in params if p is not None] if recorded else None
+
+
+def _rebuilt(ctx, x, params, g, seeds=None):
     """The gradients of x, the seeds (where there are any) and the parameters by the separate functions, for a
-    backward that is itself differentiated."""
+    backward that is itself differentiated.  The parameters are not among the saved tensors: an ordinary backward
+    takes the casts and statistics that the forward kept, so a bias, or under autocast a weight, may be changed in
+    place before it."""
+    setup, needs = ctx.setup, ctx.needs_input_grad[1:]
+    if _versions(ctx.inputs, True) != ctx.versions:
+        raise RuntimeError("one of the variables needed for gradient computation has been modified by an inplace "
+                           "operation: a parameter of a packed block, whose backward is to be differentiated again")
     inputs = [x] + ([] if seeds is None else [seeds]) + list(params)
     with torch.enable_grad(), torch.autocast("cuda", setup.dt if setup.amp else None, enabled=setup.amp):
         out = setup.again(_stand_in(setup, x.shape[1], params, seeds), x, setup.dropout[1])
@@ -234,15 +245,15 @@ class _SabBlock(torch.autograd.Function):
             out, saved = _mlp_forward(ym, params[12:], x2, keeps, setup.fused)
             keep += [x2, f32_values(ln_w2), stats2] + saved
         ctx.setup, ctx.n_keep, ctx.mask_keys = setup, len(keep), list(setup.mask)
-        ctx.save_for_backward(*keep, cu, *setup.mask.values(), *params)
+        ctx.inputs, ctx.versions = params, _versions(params, keeps)
+        ctx.save_for_backward(*keep, cu, *setup.mask.values())
         return out
 
     @staticmethod
     def backward(ctx, g):
         setup, needs, tensors = ctx.setup, ctx.needs_input_grad[1:], ctx.saved_tensors
         if torch.is_grad_enabled():
-            params = tensors[ctx.n_keep + 1 + len(ctx.mask_keys):]
-            return (None,) + _rebuilt(setup, tensors[0], params, g, needs)
+            return (None,) + _rebuilt(ctx, tensors[0], ctx.inputs, g)
         x, ln_w, stats, xm, q, k, v, o, lse, z, wq, wk, wv, wo = tensors[:14]
         cu, mask = tensors[ctx.n_keep], dict(zip(ctx.mask_keys, tensors[ctx.n_keep + 1:]))
         t, d = x.shape
@@ -308,18 +319,17 @@ class _PmaBlock(torch.autograd.Function):
             out, saved = _mlp_forward(ym, params[12:], x2, keeps, setup.fused)
             keep += [x2, f32_values(ln_w2), stats2] + saved
         ctx.setup, ctx.n_keep = setup, len(keep)
-        ctx.save_for_backward(*keep, setup.cu, seeds, *params)
+        ctx.inputs, ctx.versions = (seeds, *params), _versions((seeds, *params), keeps)
+        ctx.save_for_backward(*keep, setup.cu)
         return out.view(-1, k_seeds, d)
 
     @staticmethod
     def backward(ctx, g):
         setup, needs, tensors = ctx.setup, ctx.needs_input_grad[1:], ctx.saved_tensors
         if torch.is_grad_enabled():
-            seeds, *params = tensors[ctx.n_keep + 1:]
-            return (None,) + _rebuilt(setup, tensors[0], params, g, needs, seeds)
+            return (None,) + _rebuilt(ctx, tensors[0], ctx.inputs[1:], g, ctx.inputs[0])
         x, ln_w, stats, xm, s, q, k, v, o, lse, z, wq, wk, wv, wo = tensors[:15]
-        cu, seeds = tensors[ctx.n_keep:ctx.n_keep + 2]
-        d = x.shape[1]
+        cu, seeds, d = tensors[ctx.n_keep], ctx.inputs[0], x.shape[1]
         g, grads = g.contiguous().view(-1, d), _Grads(setup, needs, x.shape[0])
         if setup.n_mlp:
             x2, ln_w2, stats2 = tensors[15:18]

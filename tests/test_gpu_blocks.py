@@ -254,3 +254,27 @@ def test_differentiated_again_in_another_mode(device, pma):
         blk.eval()
         grads.append(torch.autograd.grad(out.sin().sum(), inputs, create_graph=again))
     _agree(*grads, 1e-5, ["x", *_used(blk)])
+
+
+@pytest.mark.parametrize("amp", [False, True])
+@pytest.mark.parametrize("pma", [False, True])
+def test_parameters_changed_before_the_backward(device, amp, pma):
+    """In-place updates between the forward and its backward of parameters whose values the gradients do not take
+    (biases; under autocast the weights, too, of which the cast is kept) leave the gradients as they were.  Where the
+    block would have to run again, the change is an error."""
+    tokens = _tokens(device, False)
+    blk = _pma(device) if pma else _sab(device, 1, 2)
+    x = torch.randn(tokens.num_tokens, 64, device=device, requires_grad=True)
+    used, grads = _used(blk), []
+    changed = [p for n, p in used.items() if n.endswith("bias") or (amp and ".ln." not in n)]
+    for change in (False, True):
+        with torch.autocast("cuda", torch.bfloat16, enabled=amp):
+            out = _packed(blk, tokens)[0](x)
+        if change:
+            with torch.no_grad():
+                for p in changed:
+                    p.add_(0.5)
+            with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+                torch.autograd.grad(out.sum(), x, create_graph=True)
+        grads.append(torch.autograd.grad(out.sin().sum(), [x, *used.values()]))
+    assert all(torch.equal(a, b) for a, b in zip(*grads))
