@@ -32,6 +32,7 @@ from .eager import Unrecorded, call, plain
 from .layer_norm import f32_values, ln_backward, ln_forward, supported
 from .linear import (cast_param, hookless, input_grad, linear_outputs, linear_then_add, linear_then_mab,
                      linear_then_mish, weight_bias_grads)
+from .mha import PMA
 from .mlp_utils import SmallMLP
 
 
@@ -41,7 +42,7 @@ def _mlp_layers(blk) -> list[nn.Linear] | None:
     if not blk.use_mlp:
         return []
     glob = nn.modules.module
-    if (type(blk.mlp) is not SmallMLP or not hookless(blk.mlp) or blk.mlp._backward_hooks
+    if (type(blk.mlp) is not SmallMLP or "forward" in vars(blk.mlp) or not hookless(blk.mlp) or blk.mlp._backward_hooks
             or blk.mlp._backward_pre_hooks or glob._global_forward_hooks or glob._global_forward_pre_hooks
             or glob._global_backward_hooks or glob._global_backward_pre_hooks):
         return None
@@ -62,6 +63,13 @@ def _compute_dtype(x: torch.Tensor, params):
     if not torch.is_autocast_enabled("cuda"):
         return torch.float32
     return torch.bfloat16 if torch.get_autocast_dtype("cuda") == torch.bfloat16 else None
+
+
+def _held(blk, mab) -> bool:
+    """Whether the block's parameters are its modules' own: a subclass, as a parametrization makes it, may compute them
+    with every look (and a spectral norm moves its estimate with it), where the separate functions look once."""
+    return (all(type(fc) is nn.Linear for fc in (mab.fc_q, mab.fc_k, mab.fc_v, mab.fc_o))
+            and all(type(n.ln) is nn.LayerNorm for n in (blk.norm, blk.norm_mlp)))
 
 
 def _block_args(blk, mab, mlp):
@@ -283,7 +291,7 @@ def sab_block(blk, x: torch.Tensor, tokens, masked: bool, attn_p: float, again) 
     ``again(blk, x, seed)`` computes a block through the separate functions."""
     mab, ln = blk.sab.mab, blk.norm.ln
     mlp = _mlp_layers(blk)
-    if mlp is None or blk.residual_dropout > 0 or x.dim() != 2 or mab.dim_V != x.shape[1]:
+    if mlp is None or blk.residual_dropout > 0 or x.dim() != 2 or mab.dim_V != x.shape[1] or not _held(blk, mab):
         return None
     d, h = x.shape[1], mab.num_heads
     params = _block_args(blk, mab, mlp)
@@ -354,12 +362,12 @@ class _PmaBlock(torch.autograd.Function):
 def pma_block(blk, x: torch.Tensor, tokens, attn_p: float, again) -> torch.Tensor | None:
     """The PMAComplete block ``blk`` over packed keys x [T, D] -> [B, k, D], or None where this path does not take
     the call (as ``sab_block``; a seed count equal to the sets' padded size has a residual of its own)."""
-    mab, seeds, ln = blk.pma.mab, blk.pma.S, blk.norm.ln
+    mab, ln = blk.pma.mab, blk.norm.ln
     mlp = _mlp_layers(blk)
-    if mlp is None or blk.residual_dropout > 0 or x.dim() != 2 or seeds.shape[1] == tokens.max_items:
+    if mlp is None or blk.residual_dropout > 0 or x.dim() != 2 or type(blk.pma) is not PMA or not _held(blk, mab):
         return None
-    d, h = x.shape[1], mab.num_heads
-    if mab.dim_V != d or seeds.shape[2] != d or tokens.batch_size < 1:
+    d, h, seeds = x.shape[1], mab.num_heads, blk.pma.S
+    if mab.dim_V != d or seeds.shape[2] != d or seeds.shape[1] == tokens.max_items or tokens.batch_size < 1:
         return None
     params = _block_args(blk, mab, mlp)
     dt = _compute_dtype(x, [seeds] + params)

@@ -278,3 +278,46 @@ def test_parameters_changed_before_the_backward(device, amp, pma):
                 torch.autograd.grad(out.sum(), x, create_graph=True)
         grads.append(torch.autograd.grad(out.sin().sum(), [x, *used.values()]))
     assert all(torch.equal(a, b) for a, b in zip(*grads))
+
+
+class _Halved(torch.nn.Module):
+    """A parametrization that counts how often it is evaluated."""
+
+    def __init__(self):
+        super().__init__()
+        self.calls = 0
+
+    def forward(self, w):
+        self.calls += 1
+        return 0.5 * w
+
+
+@pytest.mark.parametrize("where", ["fc_q", "fc_o", "ln", "S"])
+def test_parametrized_parameters(device, where):
+    """A parametrized tensor is computed as often as the separate functions compute it (a spectral norm's estimate
+    moves with every evaluation) and gets its gradient, also where that is differentiated again."""
+    tokens = _tokens(device, False)
+    grads, calls = [], []
+    for i in range(2):
+        blk = _pma(device) if where == "S" else _sab(device, 0, 2)
+        owner = {"ln": lambda: blk.norm.ln, "S": lambda: blk.pma}.get(where, lambda: getattr(blk.sab.mab, where))()
+        count = _Halved()
+        torch.nn.utils.parametrize.register_parametrization(owner, "S" if where == "S" else "weight", count)
+        gen = torch.Generator(device).manual_seed(2)
+        x = torch.randn(tokens.num_tokens, 64, device=device, generator=gen, requires_grad=True)
+        count.calls = 0
+        out = _packed(blk, tokens)[i](x)
+        calls.append(count.calls)
+        params = [p for n, p in blk.named_parameters()]
+        grads.append(torch.autograd.grad(out.sin().sum(), [x] + params, create_graph=True))
+    assert calls[0] == calls[1]
+    _agree(*grads, 1e-5, ["x"] + [n for n, _ in blk.named_parameters()])
+
+
+def test_replaced_forward_runs(device):
+    """A forward set on the MLP itself (as wrappers set it) is called."""
+    tokens, blk = _tokens(device, False), _sab(device, 0, 2)
+    seen, plain = [], blk.mlp.forward
+    blk.mlp.forward = lambda y: seen.append(1) or plain(y)
+    _packed(blk, tokens)[0](torch.randn(tokens.num_tokens, 64, device=device))
+    assert seen
