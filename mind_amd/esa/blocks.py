@@ -31,7 +31,7 @@ from .attention import HEAD_DIMS, attn_bwd, attn_fwd, pma_backward, pma_forward
 from .eager import Unrecorded, call, plain
 from .layer_norm import f32_values, ln_backward, ln_forward, supported
 from .linear import (cast_param, hookless, input_grad, linear_outputs, linear_then_add, linear_then_mab,
-                     linear_then_mish, weight_bias_grads)
+                     linear_then_mish, on_boundary, weight_bias_grads)
 from .mha import PMA
 from .mlp_utils import SmallMLP
 
@@ -265,7 +265,7 @@ class _SabBlock(torch.autograd.Function):
         x, ln_w, stats, xm, q, k, v, o, lse, z, wq, wk, wv, wo = tensors[:14]
         cu, mask = tensors[ctx.n_keep], dict(zip(ctx.mask_keys, tensors[ctx.n_keep + 1:]))
         t, d = x.shape
-        g, grads = g.contiguous(), _Grads(setup, needs, t)
+        g, grads = on_boundary(g.contiguous()), _Grads(setup, needs, t)
         if setup.n_mlp:
             x2, ln_w2, stats2 = tensors[14:17]
             dy = _mlp_backward(g.to(setup.dt), tensors[17:ctx.n_keep], grads, 13, setup.fused)
@@ -338,7 +338,7 @@ class _PmaBlock(torch.autograd.Function):
             return (None,) + _rebuilt(ctx, tensors[0], ctx.inputs[1:], g, ctx.inputs[0])
         x, ln_w, stats, xm, s, q, k, v, o, lse, z, wq, wk, wv, wo = tensors[:15]
         cu, seeds, d = tensors[ctx.n_keep], ctx.inputs[0], x.shape[1]
-        g, grads = g.contiguous().view(-1, d), _Grads(setup, needs, x.shape[0])
+        g, grads = on_boundary(g.contiguous()).view(-1, d), _Grads(setup, needs, x.shape[0])
         if setup.n_mlp:
             x2, ln_w2, stats2 = tensors[15:18]
             dy = _mlp_backward(g, tensors[18:ctx.n_keep], grads, 14, setup.fused)

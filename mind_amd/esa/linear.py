@@ -70,13 +70,22 @@ def weight_grad(g: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
 _CODES = {torch.float32: _lib.ESA_F32, torch.bfloat16: _lib.ESA_BF16}
 
 
+def _aligned(t: torch.Tensor) -> bool:
+    return t.data_ptr() % 16 == 0
+
+
+def on_boundary(t: torch.Tensor) -> torch.Tensor:
+    """The contiguous t, or its copy where its memory starts off the 16-byte boundary that the kernels ask for."""
+    return t if _aligned(t) else t.clone()
+
+
 def column_sum(g: torch.Tensor) -> torch.Tensor:
     """g.sum(0) of a device [rows, cols] tensor in fp32 through esa_column_sum (fixed order); shapes the kernel
     does not take (cols not a multiple of 4, other dtypes) use torch's sum."""
     rows, cols = g.shape
     if g.dtype not in _CODES or cols % 4 or cols < 4:
         return g.float().sum(0)
-    g = g.contiguous()
+    g = on_boundary(g.contiguous())
     lib = _lib.load()
     n = ctypes.c_size_t(0)
     _lib.check(lib.esa_column_sum_workspace_size(rows, cols, ctypes.byref(n)), "esa_column_sum_workspace_size")
@@ -129,10 +138,6 @@ def esa_weight_grad(pairs, bias) -> list[tuple[torch.Tensor, torch.Tensor | None
                                    o, i, code, vp(*[w.data_ptr() for w in dw]), vp(*[_lib.ptr(b) for b in db]),
                                    ws.data_ptr(), ws.numel(), _lib.stream_of(pairs[0][0])), "esa_weight_grad")
     return list(zip(dw, db))
-
-
-def _aligned(t: torch.Tensor) -> bool:
-    return t.data_ptr() % 16 == 0
 
 
 def weight_bias_grads(pairs, need_w, need_b) -> list[tuple[torch.Tensor | None, torch.Tensor | None]]:
@@ -255,8 +260,8 @@ def _library_rate(x, w, fused_passes: bool) -> bool:
 
 
 # The Linears of the packed blocks.  ``fused``: the caller's word that esa_linear_fwd / esa_linear_dx take the sizes
-# and the weights (``fused_ok`` of both directions).  Rows that come from the caller of the block (the pooling's seeds,
-# the output's gradient) may start anywhere, so the alignment of the rows is looked at here.
+# and the weights (``fused_ok`` of both directions).  Rows that come from the caller of the block (the pooling's seeds)
+# may start anywhere, so the alignment of the rows is looked at here.
 
 def linear_outputs(x, pairs, fused: bool) -> list[torch.Tensor]:
     """[x W^T + b for (W, b) in pairs]: one launch of esa_linear_fwd, or ``linear_fwd``."""

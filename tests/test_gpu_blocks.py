@@ -321,3 +321,22 @@ def test_replaced_forward_runs(device):
     blk.mlp.forward = lambda y: seen.append(1) or plain(y)
     _packed(blk, tokens)[0](torch.randn(tokens.num_tokens, 64, device=device))
     assert seen
+
+
+@pytest.mark.parametrize("amp", [False, True])
+@pytest.mark.parametrize("pma", [False, True])
+@pytest.mark.parametrize("mlp", [False, True])
+def test_output_gradient_off_a_boundary(device, amp, pma, mlp):
+    """An output gradient whose memory starts off a 16-byte boundary gives the same gradients as its copy on one."""
+    tokens = _tokens(device, False)
+    blk = _pma(device, mlp) if pma else _sab(device, 1, 2 * mlp)
+    x = torch.randn(tokens.num_tokens, 64, device=device, requires_grad=True)
+    with torch.autocast("cuda", torch.bfloat16, enabled=amp):
+        out = _packed(blk, tokens)[0](x)
+    flat = torch.randn(out.numel() + 1, device=device).to(out.dtype)
+    g = flat[1:].view(out.shape)
+    assert g.data_ptr() % 16
+    used = _used(blk)
+    got = torch.autograd.grad(out, [x, *used.values()], g, retain_graph=True)
+    want = torch.autograd.grad(out, [x, *used.values()], g.clone())
+    assert all(torch.equal(a, b) for a, b in zip(got, want))

@@ -94,3 +94,15 @@ def test_other_calls_keep_torch_operations(device):
     (dw,) = torch.autograd.grad((L.linear(xr, w) * g).sum(), w, create_graph=True)
     (dx,) = torch.autograd.grad((dw * w).sum(), xr)   # d/dx sum(w * g^T x) = g w
     assert torch.allclose(dx, g @ w.detach(), rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_rows_off_a_boundary(device, dtype):
+    """A gradient and an input that start off a 16-byte boundary: weight and bias gradients, the column sum."""
+    (g, x), = _pairs(device, 301, [(64, 72)], dtype)
+    off = [torch.cat((t.new_zeros(1), t.reshape(-1)))[1:].view(t.shape) for t in (g, x)]
+    assert all(t.data_ptr() % 16 for t in off)
+    for a, b in (off, (off[0], x), (g, off[1])):
+        ((dw, db),) = L.weight_bias_grads([(a, b)], [True], [True])
+        _check([(g, x)], [(dw, db)], [True])
+    assert torch.equal(L.column_sum(off[0]), L.column_sum(g))
