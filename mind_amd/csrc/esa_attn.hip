@@ -2027,6 +2027,7 @@ __global__ __launch_bounds__(F32Tile<HD>::kThreads) __attribute__((amdgpu_waves_
           }
         },
         [&](int buf, int q0) {
+          const bool tail = q0 + kF32Stage > phi;
           auto block = [&](int kb) {
             f32x4 x[NR], s[QB], ds[QB];
             f32_rows<HD>(x, sQ[buf], 16 * kb, c16, grp);
@@ -2042,8 +2043,9 @@ __global__ __launch_bounds__(F32Tile<HD>::kThreads) __attribute__((amdgpu_waves_
               const int2 pn = MASKED ? sN[buf][qi] : make_int2(0, 0);
 #pragma unroll
               for (int b = 0; b < QB; ++b) {
-                const float p = fast_exp2(a.c * s[b][r] - lse2[r]);   // a query past the range has LSE2 = inf
-                const bool in = !MASKED || admissible_f32<true>(q0 + qi, phi, own.tok[b], pn, node[b]);
+                const float p = fast_exp2(a.c * s[b][r] - lse2[r]);
+                // a query past the range has a zero row: an infinity of the key times it would be a NaN
+                const bool in = !(MASKED || tail) || admissible_f32<MASKED>(q0 + qi, phi, own.tok[b], pn, node[b]);
                 const bool keep = !DROP || drop_keep(a.drop, sKey[buf][qi], ck[b], own.tok[b]);
                 float dp = ds[b][r];
                 if (DROP) dp = keep ? dp * a.drop.inv_keep : 0.f;

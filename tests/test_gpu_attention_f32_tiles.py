@@ -81,3 +81,27 @@ def test_edge_mask_nonfinite_row_stays_with_its_neighbours(device, hd, p, what, 
     for name, want, got in zip(("dq", "dk", "dv"), *grads):
         keep = far_q if name == "dq" else far   # dq: the token's own statistics and its keys
         _close(got[keep], want[keep].double(), name)
+
+
+@pytest.mark.parametrize("hd,p", [(16, 0.0), (24, 0.3), (32, 0.0), (64, 0.0)])
+@pytest.mark.parametrize("length", [17, 63, 64, 130])
+def test_key_that_no_query_sees(device, hd, p, length):
+    """A key whose scores are all -inf (an infinite component against positive ones) has zero probability for every
+    query: its own gradients are zeros, the other keys' are those without it, and nothing is a NaN.  (dQ takes the
+    key's row times zero, which an infinity makes a NaN.)"""
+    odd = length // 2
+    rest = [i for i in range(length) if i != odd]
+    q, k, v, g = _inputs(length, length, 11, 2, hd)
+    q[..., 3] = q[..., 3].abs() + 0.1
+    k[odd, :, 3] = -float("inf")
+    qd, kd, vd = (x.to(device).requires_grad_(True) for x in (q, k, v))
+    cu = torch.as_tensor(cu_from_lengths([length])).to(device)
+    out = A.varlen_attention(qd, kd, vd, cu, cu, length, length, dropout_p=p, dropout_seed=3)
+    _, dk, dv = torch.autograd.grad(out, (qd, kd, vd), g.to(device))
+    assert not out.isnan().any() and not dk.isnan().any() and not dv.isnan().any()
+    assert not dk[odd].any() and not dv[odd].any()
+    if p == 0.0:
+        cur = cu_from_lengths([length]), cu_from_lengths([length - 1])
+        want = OA.varlen_attention_bwd(g, q, k[rest], v[rest], *cur, hd ** -0.5)
+        for got, ref, name in zip((dk, dv), want[1:], ("dk", "dv")):
+            _close(got[rest].cpu(), ref, name)
