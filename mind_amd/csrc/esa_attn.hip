@@ -1417,13 +1417,14 @@ struct F32Tile {
 DEVI f32x4 mfma16x4f(float a, float b, const f32x4& c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
 // The stage's rows of a [T][H][HD] tensor from token t0 on, into registers and from there into LDS; tokens at or
-// past `end` are zeros.
-template <int HD>
+// past `end` are zeros, or with REPEAT the last row again.
+template <int HD, bool REPEAT = false>
 DEVI void f32_load(f32x4 (&r)[F32Tile<HD>::kPer], const float* src, int end, int H, int head, int t0) {
   using T = F32Tile<HD>;
 #pragma unroll
   for (int i = 0; i < T::kPer; ++i) {
-    const int x = threadIdx.x + i * T::kThreads, t = t0 + x / (4 * T::NR), part = x % (4 * T::NR);
+    const int x = threadIdx.x + i * T::kThreads, part = x % (4 * T::NR);
+    const int t = REPEAT ? min(t0 + x / (4 * T::NR), end - 1) : t0 + x / (4 * T::NR);
     r[i] = f32x4{0.f, 0.f, 0.f, 0.f};
     if (t < end && part < HD / 4) r[i] = *reinterpret_cast<const f32x4*>(src + ((size_t)t * H + head) * HD + 4 * part);
   }
@@ -2006,7 +2007,9 @@ __global__ __launch_bounds__(F32Tile<HD>::kThreads) __attribute__((amdgpu_waves_
     f32_stages(
         own.plo, phi, own.live,
         [&](int t0) {
-          f32_load<HD>(rQ, a.q, phi, H, head, t0);
+          // past the queries' end, without a mask to select by: the last one again.  An infinity of a key times a zero
+          // row would be a NaN, where this row's score minus its infinite LSE2 is one only if the query's own is
+          f32_load<HD, !MASKED>(rQ, a.q, phi, H, head, t0);
           f32_load<HD>(rG, a.dout, phi, H, head, t0);
           if (tid < kF32Stage) {
             const bool in = t0 + tid < phi;
@@ -2027,7 +2030,6 @@ __global__ __launch_bounds__(F32Tile<HD>::kThreads) __attribute__((amdgpu_waves_
           }
         },
         [&](int buf, int q0) {
-          const bool tail = q0 + kF32Stage > phi;
           auto block = [&](int kb) {
             f32x4 x[NR], s[QB], ds[QB];
             f32_rows<HD>(x, sQ[buf], 16 * kb, c16, grp);
@@ -2043,9 +2045,8 @@ __global__ __launch_bounds__(F32Tile<HD>::kThreads) __attribute__((amdgpu_waves_
               const int2 pn = MASKED ? sN[buf][qi] : make_int2(0, 0);
 #pragma unroll
               for (int b = 0; b < QB; ++b) {
-                const float p = fast_exp2(a.c * s[b][r] - lse2[r]);
-                // a query past the range has a zero row: an infinity of the key times it would be a NaN
-                const bool in = !(MASKED || tail) || admissible_f32<MASKED>(q0 + qi, phi, own.tok[b], pn, node[b]);
+                const float p = fast_exp2(a.c * s[b][r] - lse2[r]);   // a query past the range has LSE2 = inf
+                const bool in = !MASKED || admissible_f32<true>(q0 + qi, phi, own.tok[b], pn, node[b]);
                 const bool keep = !DROP || drop_keep(a.drop, sKey[buf][qi], ck[b], own.tok[b]);
                 float dp = ds[b][r];
                 if (DROP) dp = keep ? dp * a.drop.inv_keep : 0.f;
