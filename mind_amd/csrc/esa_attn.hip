@@ -1489,7 +1489,34 @@ DEVI void f32_gather(f32x4 (&acc)[F32Tile<HD>::QB][F32Tile<HD>::NR], const float
     }
 }
 
-// The same over the admissible pairs alone, by vector FMAs: with the edge mask, where a partner's row holds an infinity
+// acc[b] += over a stage's 64 partners: the products of 32 from zero, then added, so that no rounding of a long sum is
+// taken per partner.  Relative error of the forward's outputs against 64 bits (standard normal q, k, v, head dim 16;
+// 64 / 340 / 3,000 keys): 1.8 / 2.3 / 3.6e-7, in one chain 2.1 / 3.8 / 10.4e-7, in the per-thread kernels' four key
+// splits 1.9 / 2.6 / 5.9e-7.  It takes 8-32 registers more, for which the unmasked forward is held to four waves per
+// SIMD: 8 heads of 32 over 64 small molecules 127 us in one chain, 129 held, 133 at the three waves it would take.
+template <int HD>
+DEVI void f32_add_stage(f32x4 (&acc)[F32Tile<HD>::QB][F32Tile<HD>::NR], const float (*rows)[F32Tile<HD>::kStride],
+                        const f32x4 (&w)[kF32Stage / 16][F32Tile<HD>::QB], int c16, int grp) {
+  constexpr int NR = F32Tile<HD>::NR, QB = F32Tile<HD>::QB;
+#pragma unroll
+  for (int kb = 0; kb < kF32Stage / 16; kb += 2) {
+    f32x4 part[QB][NR];
+#pragma unroll
+    for (int b = 0; b < QB; ++b)
+#pragma unroll
+      for (int c = 0; c < NR; ++c) part[b][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = kb; j < kb + 2; ++j) f32_gather<HD>(part, rows, 16 * j, w[j], c16, grp);
+#pragma unroll
+    for (int b = 0; b < QB; ++b)
+#pragma unroll
+      for (int c = 0; c < NR; ++c)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[b][c][e] += part[b][c][e];
+  }
+}
+
+// f32_gather over the admissible pairs alone, by vector FMAs: with the edge mask, where a partner's row holds an infinity
 // or a NaN, which times the zero weight of a pair that the mask leaves out would reach tokens that do not attend it.
 // A block that has staged one walks its partners again with it: as a branch inside the one walk it took the registers
 // of two of four waves per SIMD (64 small molecules: dK/dV 174 us, 156 with the second walk and 149 without any check;
@@ -1563,7 +1590,8 @@ DEVI void f32_stages(int lo, int hi, bool live, Load load, Store store, Use use)
 }
 
 template <bool MASKED, int HD, bool DROP>
-__global__ __launch_bounds__(F32Tile<HD>::kThreads) void attn_fwd_f32_kernel(const AttnF32Args a) {
+__global__ __launch_bounds__(F32Tile<HD>::kThreads) __attribute__((amdgpu_waves_per_eu(
+    MASKED ? 1 : 4))) void attn_fwd_f32_kernel(const AttnF32Args a) {
   using T = F32Tile<HD>;
   constexpr int NR = T::NR, QB = T::QB, KB = kF32Stage / 16;
   __shared__ __align__(16) typename T::Rows sK[2], sV[2];
@@ -1658,8 +1686,7 @@ __global__ __launch_bounds__(F32Tile<HD>::kThreads) void attn_fwd_f32_kernel(con
               s[kb][b][r] = DROP && !drop_keep(a.drop, rk[b], sKey[buf][key], k0 + key) ? 0.f : p;
             }
         }
-#pragma unroll
-        for (int kb = 0; kb < KB; ++kb) f32_gather<HD>(acc, sV[buf], 16 * kb, s[kb], c16, grp);
+        f32_add_stage<HD>(acc, sV[buf], s, c16, grp);
       });
 #pragma unroll
   for (int b = 0; b < QB; ++b) {

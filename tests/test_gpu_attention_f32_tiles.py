@@ -105,3 +105,19 @@ def test_key_that_no_query_sees(device, hd, p, length):
         want = OA.varlen_attention_bwd(g, q, k[rest], v[rest], *cur, hd ** -0.5)
         for got, ref, name in zip((dk, dv), want[1:], ("dk", "dv")):
             _close(got[rest].cpu(), ref, name)
+
+
+@pytest.mark.parametrize("hd", [16, 24, 32, 64])
+@pytest.mark.parametrize("length", [340, 3000])
+def test_output_error_of_long_segments(device, hd, length):
+    """The outputs' error stays that of short sums: the products with the values are added over 32 keys and then over
+    those sums.  n additions of random signs in a row leave about 2^-24 sqrt(n / 6) of the result, here n = 32 +
+    length / 32 (one row of 3,000: 1.3e-6); four units more for the scores (hd products), the exponentials and the
+    probabilities' sum."""
+    q, k, v, _ = _inputs(length, length, hd, 4, hd)
+    cu = cu_from_lengths([length])
+    cud = torch.as_tensor(cu).to(device)
+    out = A.varlen_attention(*(x.to(device) for x in (q, k, v)), cud, cud, length, length).cpu().double()
+    ref, _ = OA.varlen_attention(q, k, v, cu, cu, hd ** -0.5)
+    bar = 2.0 ** -24 * (((32 + length / 32) / 6) ** 0.5 + 4)
+    assert float((out - ref).norm() / ref.norm()) <= bar
