@@ -40,6 +40,12 @@
 namespace {
 
 constexpr int kGemmMax = 3, kGemmStages = 3;
+// fp32 sums 128 values of a term (eight stages) from zero and adds that to the sums before it, as a product of that
+// length or the library's term by term rounds, and not along the whole contraction.  Relative error against 64 bits of
+// dx of three, 384 long: 3.0e-7 in one chain, 2.05e-7 here and in the library; 1,536 long 6.0, 2.1 and 4.0e-7;
+// y 2,048 long 5.9, 1.6 and 5.9e-7.  It costs 0-3 % (21,752 rows, 128 -> 128: 12.4 -> 12.4 us, dx of three 25.8 -> 26.7);
+// every 64 values took 2-6 %.
+constexpr int kFold = 8;
 
 // What follows the product; kDx*: the input gradient.
 enum Epi { kPlain, kMish, kMab, kMabResidual, kAdd, kDx, kDxBase, kDxMish };
@@ -182,7 +188,22 @@ __global__ __launch_bounds__(256, 2) void linear_gemm_kernel(const GemmArgs a) {
   for (int f = 0; f < NV; ++f)
 #pragma unroll
     for (int t = 0; t < TT; ++t) acc[f][t] = f32x16{};
-  auto multiply = [&](int buf) {
+  f32x16 sum[F32 ? NV : 1][F32 ? TT : 1] = {};   // fp32: the folded values of acc
+  int fold_term = term, term_end = a.p[term].k / KS, fold_at = min(term_end, kFold);   // in stages
+  auto fold = [&](int done) {   // after the products of that many stages
+    if (done != fold_at) return;
+    if (done == term_end && fold_term + 1 < a.n) term_end += a.p[++fold_term].k / KS;
+    fold_at = min(term_end, done + kFold);
+#pragma unroll
+    for (int f = 0; f < NV; ++f)
+#pragma unroll
+      for (int t = 0; t < TT; ++t) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) sum[f][t][e] += acc[f][t][e];
+        acc[f][t] = f32x16{};
+      }
+  };
+  auto multiply = [&](int buf, int stage) {
     const char* bx = lds + buf * kBuf;
     const char* bw = bx + RA::kBytes;
     if constexpr (!F32) {
@@ -228,6 +249,7 @@ __global__ __launch_bounds__(256, 2) void linear_gemm_kernel(const GemmArgs a) {
 #pragma unroll
             for (int t = 0; t < TT; ++t) acc[f][t] = mfma32x2(w[f][j], x[t][j], acc[f][t]);
       }
+      fold(stage + 1);
     }
   };
   auto run = [&](auto use) {
@@ -242,12 +264,18 @@ __global__ __launch_bounds__(256, 2) void linear_gemm_kernel(const GemmArgs a) {
         else wait_vmcnt<0>();
         __syncthreads();   // every wave's have, and every wave is done with stage s - 1, whose buffer is loaded next
         if (s + 2 < stages) load((buf + 2) % kGemmStages);
-        use(buf);
+        use(buf, s);
       }
     }
   };
   if (live) run(multiply);
-  else run([](int) {});
+  else run([](int, int) {});
+  if constexpr (F32) {
+#pragma unroll
+    for (int f = 0; f < NV; ++f)
+#pragma unroll
+      for (int t = 0; t < TT; ++t) acc[f][t] = sum[f][t];
+  }
 
   const GemmPart& out = a.p[part];
   constexpr bool kHasY = EPI == kPlain || EPI == kMish || EPI == kMab || EPI == kMabResidual;

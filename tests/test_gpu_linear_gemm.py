@@ -147,3 +147,19 @@ def test_edge_linear_input_gradient_is_rounded_once(device, out_features):
     wd = w.detach()
     ref, err = _product(torch.cat((gs, gs), 1), torch.cat((wd[:, :f], wd[:, f:]), 0).t())
     _near(dx, ref, err + U[torch.bfloat16] * ref.abs())
+
+
+@pytest.mark.parametrize("widths", [(512, 512, 512), (32, 160, 64), (2048,)])
+def test_fp32_error_of_long_contractions(device, widths):
+    """fp32 adds 128 values of a term at a time, and then those sums: n additions of random signs in a row leave about
+    2^-24 sqrt(n / 6) of the result, here n = 128 + length / 128 (one row of 1,536: 9.5e-7), and one rounding more."""
+    gen = torch.Generator().manual_seed(sum(widths))
+    rows, cols = 1000, 96
+    pairs = [(torch.randn(rows, k, generator=gen).to(device), torch.randn(k, cols, generator=gen).to(device))
+             for k in widths]
+    ref = sum(g.double() @ w.double() for g, w in pairs)
+    bar = 2.0 ** -24 * (((128 + sum(widths) / 128) / 6) ** 0.5 + 1)
+    assert float((L.fused_dx(pairs).double() - ref).norm() / ref.norm()) <= bar
+    (g, w), = pairs[:1]
+    ref = g.double() @ w.double()
+    assert float((L.fused_fwd(g, [(w.t().contiguous(), None)])[0].double() - ref).norm() / ref.norm()) <= bar
