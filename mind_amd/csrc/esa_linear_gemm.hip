@@ -43,7 +43,7 @@ constexpr int kGemmMax = 3, kGemmStages = 3;
 // fp32 sums 128 values of a term (eight stages) from zero and adds that to the sums before it, as a product of that
 // length or the library's term by term rounds, and not along the whole contraction.  Relative error against 64 bits of
 // dx of three, 384 long: 3.0e-7 in one chain, 2.05e-7 here and in the library; 1,536 long 6.0, 2.1 and 4.0e-7;
-// y 2,048 long 5.9, 1.6 and 5.9e-7.  It costs 0-3 % (21,752 rows, 128 -> 128: 12.4 -> 12.4 us, dx of three 25.8 -> 26.7);
+// y 2,048 long 5.9, 1.6 and 5.9e-7.  It costs 0-4 % (21,752 rows, 128 -> 128: 12.6 -> 12.6 us, dx of three 26.0 -> 27.1);
 // every 64 values took 2-6 %.
 constexpr int kFold = 8;
 
@@ -189,15 +189,16 @@ __global__ __launch_bounds__(256, 2) void linear_gemm_kernel(const GemmArgs a) {
 #pragma unroll
     for (int t = 0; t < TT; ++t) acc[f][t] = f32x16{};
   f32x16 sum[F32 ? NV : 1][F32 ? TT : 1] = {};   // fp32: the folded values of acc
-  int fold_term = term, term_end = a.p[term].k / KS, fold_at = min(term_end, kFold);   // in stages
-  auto fold = [&](int done) {   // after the products of that many stages
-    if (done != fold_at) return;
-    if (done == term_end && fold_term + 1 < a.n) term_end += a.p[++fold_term].k / KS;
-    fold_at = min(term_end, done + kFold);
+  const int end0 = DX ? a.p[0].k / KS : stages, end1 = DX && a.n > 1 ? end0 + a.p[1].k / KS : stages;   // of the terms
+  int fold_at = min(end0, kFold);
+  auto fold = [&](int done) {   // after the products of that many stages; the last of them are added below
+    if (done != fold_at || done == stages) return;
+    fold_at = min(done + kFold, done < end0 ? end0 : done < end1 ? end1 : stages);
 #pragma unroll
     for (int f = 0; f < NV; ++f)
 #pragma unroll
       for (int t = 0; t < TT; ++t) {
+        mfma_settled(acc[f][t]);
 #pragma unroll
         for (int e = 0; e < 16; ++e) sum[f][t][e] += acc[f][t][e];
         acc[f][t] = f32x16{};
@@ -274,7 +275,11 @@ __global__ __launch_bounds__(256, 2) void linear_gemm_kernel(const GemmArgs a) {
 #pragma unroll
     for (int f = 0; f < NV; ++f)
 #pragma unroll
-      for (int t = 0; t < TT; ++t) acc[f][t] = sum[f][t];
+      for (int t = 0; t < TT; ++t) {
+        mfma_settled(acc[f][t]);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[f][t][e] += sum[f][t][e];
+      }
   }
 
   const GemmPart& out = a.p[part];

@@ -13,6 +13,11 @@ DEVI f32x16 mfma32x2(float a, float b, const f32x16& c) {
   return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
 }
 
+// The 18 wait states that v_mfma_f32_32x32x2_f32 (16 passes) asks for before a vector instruction touches its result,
+// written out where that instruction stands in a block of its own that several paths reach: the compiler then counts
+// the longest of them and has put none (a sum took an accumulator register before the matrix pipe had written it).
+DEVI void mfma_settled(f32x16& acc) { asm volatile("s_nop 15\n\ts_nop 1" : "+v"(acc)); }
+
 // An operand whose contraction runs over the rows in memory, staged as [rows
 // of the stage][COLS]: the operands of dW = g^T x (rows = tokens) and W in
 // dx = g W.  bf16 operands come from ds_read_b64_tr_b16, and a row's 16-byte
