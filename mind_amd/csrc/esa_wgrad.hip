@@ -47,6 +47,15 @@ constexpr int kMaxPairs = 8;
 constexpr int kWTileO = 128;                 // block tile along `out` (two waves of 64); along `in`: 64 NV (two of 32 NV)
 constexpr int kStages = 3;
 constexpr int kCus = 256, kMinRows = 128;
+// The bias sums of this many stages are added to those before them, instead of a row range's tokens in one chain
+// (relative error against 64 bits, fp32 21,752 x 128: 2.05e-7 in one chain, 1.44 here, 1.76 in the column sum;
+// 129,850 x 512: 7.7, 1.9 and 2.5e-7).
+constexpr int kBiasFold = 4;
+// In fp32 ranges of more than kFoldRows rows the sums of kFold stages are added to those before them, too (FOLD):
+// 129,850 x 2048 x 512, 16,256 rows a range: 2.3e-6 in one chain, 4.2e-7 folded, the library's token-chunk products
+// 1.6e-6.  It takes 50 registers and 4 % (2,005 -> 2,086 us; shorter ranges by more splits: 2,450), which ranges up to
+// 4,096 rows are spared: 1.1e-6 in one chain.
+constexpr int kFold = 32, kFoldRows = 4096;
 
 struct WgradPair {
   const void* g; const void* x;
@@ -62,7 +71,7 @@ struct WgradArgs {
 struct ReducePart { const float* src; float* dst; int64_t n; int block0; };
 struct ReduceArgs { int splits, n; ReducePart p[2 * kMaxPairs]; };
 
-template <typename T, int NV>
+template <typename T, int NV, bool FOLD>
 __global__ __launch_bounds__(256, 2) void wgrad_kernel(const WgradArgs a) {
   constexpr int kTileI = 64 * NV;
   using RG = Rows<T, kWTileO>;
@@ -107,9 +116,11 @@ __global__ __launch_bounds__(256, 2) void wgrad_kernel(const WgradArgs a) {
   for (int u = 0; u < 2; ++u)
 #pragma unroll
     for (int v = 0; v < NV; ++v) acc[u][v] = f32x16{};
-  float bs[2] = {0.f, 0.f};
+  float bs[2] = {0.f, 0.f}, bias_sum[2] = {0.f, 0.f};   // of the last stages, of those before them
+  f32x16 sum[FOLD ? 2 : 1][FOLD ? NV : 1] = {};         // of acc and bias_sum, before the last kFold stages
+  float bias_before[2] = {0.f, 0.f};
   // One stage's products; all operands of the stage are read first, so the reads of a step overlap the last one's MFMAs.
-  auto multiply = [&](int buf, auto with_bias) {
+  auto multiply = [&](int buf, int stage, auto with_bias) {
     typename RG::Op og[kSteps][2], ox[kSteps][NV];
 #pragma unroll
     for (int k = 0; k < kSteps; ++k) {
@@ -128,6 +139,26 @@ __global__ __launch_bounds__(256, 2) void wgrad_kernel(const WgradArgs a) {
 #pragma unroll
         for (int u = 0; u < 2; ++u) bs[u] = RG::add_tokens(og[k][u], bs[u]);
     }
+    if (with_bias.value && stage % kBiasFold == kBiasFold - 1)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        bias_sum[u] += bs[u];
+        bs[u] = 0.f;
+      }
+    if constexpr (FOLD)
+      if (stage % kFold == kFold - 1)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          bias_before[u] += bias_sum[u];
+          bias_sum[u] = 0.f;
+#pragma unroll
+          for (int v = 0; v < NV; ++v) {
+            mfma_settled(acc[u][v]);
+#pragma unroll
+            for (int e = 0; e < 16; ++e) sum[u][v][e] += acc[u][v][e];
+            acc[u][v] = f32x16{};
+          }
+        }
   };
   // Every wave runs the same stages and barriers; `use` is what it does with a stage.
   auto run = [&](auto use) {
@@ -142,14 +173,23 @@ __global__ __launch_bounds__(256, 2) void wgrad_kernel(const WgradArgs a) {
         else wait_vmcnt<0>();
         __syncthreads();   // every wave's have, and every wave is done with stage s - 1, whose buffer is loaded next
         if (s + 2 < stages) load(s + 2, (buf + 2) % kStages);
-        use(buf);
+        use(buf, s);
       }
     }
   };
-  if (!live) run([](int) {});
-  else if (bias) run([&](int buf) { multiply(buf, std::true_type{}); });
-  else run([&](int buf) { multiply(buf, std::false_type{}); });
+  if (!live) run([](int, int) {});
+  else if (bias) run([&](int buf, int s) { multiply(buf, s, std::true_type{}); });
+  else run([&](int buf, int s) { multiply(buf, s, std::false_type{}); });
   if (!live) return;
+  if constexpr (FOLD)
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int v = 0; v < NV; ++v) {
+        mfma_settled(acc[u][v]);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[u][v][e] += sum[u][v][e];
+      }
   const int col = lane & 31, half = lane >> 5;
   // rows past `out` lie past the buffer, columns past `in` are sent there: both stores are dropped
   const rsrc_t ro = make_rsrc(p.part + (size_t)split * p.out * p.in, (uint32_t)p.out * p.in * 4u);
@@ -168,9 +208,9 @@ __global__ __launch_bounds__(256, 2) void wgrad_kernel(const WgradArgs a) {
   if (bias)
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      const float sum = bs[u] + __shfl_xor(bs[u], 32);   // the lane halves hold different tokens
+      const float b = bias_before[u] + (bias_sum[u] + bs[u]), both = b + __shfl_xor(b, 32);   // the lane halves hold different tokens
       const int o = o0 + wo + 32 * u + col;
-      if (half == 0 && o < p.out) p.bpart[(size_t)split * p.out + o] = sum;
+      if (half == 0 && o < p.out) p.bpart[(size_t)split * p.out + o] = both;
     }
 }
 
@@ -189,11 +229,17 @@ __global__ __launch_bounds__(256) void wgrad_reduce_kernel(const ReduceArgs a) {
   const int64_t e = ((int64_t)((int)blockIdx.x - p.block0) * 64 + lane) * 4;
   f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};
   if (e < p.n) {
-#pragma unroll 8
-    for (int k = wave; k < a.splits; k += 4) {
-      const f32x4 v = *reinterpret_cast<const f32x4*>(p.src + (size_t)k * p.n + e);
+    for (int k0 = wave; k0 < a.splits; k0 += 32) {   // eight at a time, their loads in flight together
+      f32x4 v[8], part = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int j = 0; j < 4; ++j) s[j] += v[j];
+      for (int i = 0; i < 8; ++i)
+        v[i] = *reinterpret_cast<const f32x4*>(p.src + (size_t)min(k0 + 4 * i, a.splits - 1) * p.n + e);
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) part[j] += k0 + 4 * i < a.splits ? v[i][j] : 0.f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) s[j] += part[j];
     }
   }
   if (wave) sums[wave - 1][lane] = s;
@@ -313,12 +359,13 @@ int esa_weight_grad(long long rows, int n, const void* const* g, const void* con
   const int64_t items = (int64_t)w.tiles * w.splits;
   if (items > 0x7fffffffLL || blocks > 0x7fffffffLL) return ESA_ERR_SHAPE;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-#define ESA_WGRAD(T, NV) \
+#define ESA_WGRAD(T, NV, FOLD) \
   ESA_TIMED(esa_profile::kWeightGrad, st, \
-            hipLaunchKernelGGL((wgrad_kernel<T, NV>), dim3((unsigned)items), dim3(256), 0, st, a))
-  if (dtype == ESA_F32) ESA_WGRAD(float, 2);
-  else if (w.nv == 4) ESA_WGRAD(bf16, 4);
-  else ESA_WGRAD(bf16, 2);
+            hipLaunchKernelGGL((wgrad_kernel<T, NV, FOLD>), dim3((unsigned)items), dim3(256), 0, st, a))
+  if (dtype == ESA_F32 && w.chunk > kFoldRows) ESA_WGRAD(float, 2, true);
+  else if (dtype == ESA_F32) ESA_WGRAD(float, 2, false);
+  else if (w.nv == 4) ESA_WGRAD(bf16, 4, false);
+  else ESA_WGRAD(bf16, 2, false);
 #undef ESA_WGRAD
   ESA_LAUNCH_CHECK();
   if (w.splits > 1) {

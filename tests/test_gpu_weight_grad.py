@@ -106,3 +106,21 @@ def test_rows_off_a_boundary(device, dtype):
         ((dw, db),) = L.weight_bias_grads([(a, b)], [True], [True])
         _check([(g, x)], [(dw, db)], [True])
     assert torch.equal(L.column_sum(off[0]), L.column_sum(g))
+
+
+@pytest.mark.parametrize("rows,shape", [(900, (128, 128)), (21752, (256, 128)), (66000, (1024, 1024))])
+def test_fp32_error(device, rows, shape):
+    """n additions of random signs in a row leave about 2^-24 sqrt(n / 6) of the result.  A bias column is 32 tokens
+    (four stages, half of their rows), those sums over a range (up to 4,096 rows, or 512 and those), and at most 512
+    ranges in four slices of eights: n = 52 + 64; a weight is the range's rows, or 512 and those sums.  Two units more
+    for the last additions."""
+    pairs = _pairs(device, rows, [shape], torch.float32)
+    ((dw, db),) = L.esa_weight_grad(pairs, [True])
+    g, x = (t.double() for t in pairs[0])
+
+    def off(got, ref):
+        return float((got.double() - ref).norm() / ref.norm())
+    tiles = -(-shape[0] // 128) * -(-shape[1] // 128)
+    span = max(128, rows // max(1, 512 // tiles))   # rows of a range
+    assert off(db, g.sum(0)) <= 2.0 ** -24 * (((52 + min(span, 4096) / 64) / 6) ** 0.5 + 2)
+    assert off(dw, g.t() @ x) <= 2.0 ** -24 * (((span if span <= 4096 else 512 + span / 512) / 6) ** 0.5 + 2)
