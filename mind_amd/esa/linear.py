@@ -105,10 +105,10 @@ _MAX_FEATURES = 16384
 
 def _wgrad_ok(pairs) -> bool:
     """Whether esa_weight_grad takes every (g, x): fp32 or bf16 device tensors of one dtype, [rows, features]
-    contiguous with the same rows >= 1, feature counts multiples of 8 (bf16) or 4 (fp32), 16-byte aligned."""
+    contiguous with the same 1 to 2^31 - 1 rows, feature counts multiples of 8 (bf16) or 4 (fp32), 16-byte aligned."""
     g0 = pairs[0][0]
     code = _CODES.get(g0.dtype)
-    if code is None or not g0.is_cuda or g0.shape[0] < 1:
+    if code is None or not g0.is_cuda or not 1 <= g0.shape[0] < 2 ** 31:
         return False
     unit = 8 if code == _lib.ESA_BF16 else 4
     for g, x in pairs:

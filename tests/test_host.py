@@ -216,3 +216,15 @@ def test_torch_library_ops_have_fake_implementations():
         ip, perm = torch.ops.esa_hip.csr_build(idx, 10)
         assert ip.shape == (11,) and perm.shape == (30,)
         assert torch.ops.esa_hip.csr_segment_sum(torch.empty(30, 8), ip, perm).shape == (10, 8)
+
+
+def test_weight_grad_rows_beyond_the_kernel():
+    """esa_weight_grad counts rows in 31 bits: larger inputs stay with the token-chunk products."""
+    from types import SimpleNamespace
+    from mind_amd.esa import linear as L
+
+    def rows(n):
+        return SimpleNamespace(dtype=torch.bfloat16, device="cuda:0", is_cuda=True, shape=(n, 8), dim=lambda: 2,
+                               is_contiguous=lambda: True, data_ptr=lambda: 256)
+    for n, taken in ((0, False), (1, True), (2 ** 31 - 1, True), (2 ** 31, False)):
+        assert L._wgrad_ok([(rows(n), rows(n))]) is taken
