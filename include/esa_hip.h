@@ -454,7 +454,9 @@ ESA_API int esa_column_sum(const void* x, int dtype, int64_t rows, int cols, flo
 /* a [rows, cols] tensor, and dbias = the fp32 column sums of dz, equal to   */
 /* esa_column_sum over dz, in one pass.  Workspace size from                 */
 /* esa_column_sum_workspace_size(rows, cols).  cols % 4 == 0; 16-byte        */
-/* aligned pointers.                                                         */
+/* aligned pointers.  For callers of this interface that need no weight      */
+/* gradient (a frozen Linear with a trained bias, one pass over z and grad): */
+/* the Python modules take the bias gradient from esa_weight_grad.           */
 ESA_API int esa_mish_bwd_colsum(const void* z, const void* grad, int64_t rows, int cols,
                         int dtype, void* dz, float* dbias, void* workspace,
                         size_t workspace_bytes, void* stream);

@@ -1518,9 +1518,11 @@ DEVI void f32_add_stage(f32x4 (&acc)[F32Tile<HD>::QB][F32Tile<HD>::NR], const fl
 
 // f32_gather over the admissible pairs alone, by vector FMAs: with the edge mask, where a partner's row holds an infinity
 // or a NaN, which times the zero weight of a pair that the mask leaves out would reach tokens that do not attend it.
-// A block that has staged one walks its partners again with it: as a branch inside the one walk it took the registers
-// of two of four waves per SIMD (64 small molecules: dK/dV 174 us, 156 with the second walk and 149 without any check;
-// dQ 127, 123 and 119).  The masked backward kernels are held to the four waves for it; neither spills.
+// The backward kernels take it where a block has staged one, in a second walk over its partners: as a branch inside the
+// one walk it took the registers of two of four waves per SIMD (64 small molecules: dK/dV 174 us, 156 with the second
+// walk and 149 without any check; dQ 127, 123 and 119).  They are held to the four waves for it; neither spills.  The
+// forward has no such walk: an infinite or NaN row of V reaches every query of its segment, as it does in the softmax of
+// a mask of -inf, whose zeros multiply V.
 template <int HD>
 DEVI void f32_gather_admissible(f32x4 (&acc)[F32Tile<HD>::QB][F32Tile<HD>::NR],
                                 const float (*rows)[F32Tile<HD>::kStride], int p0, const f32x4 (&w)[F32Tile<HD>::QB],
@@ -1701,8 +1703,9 @@ __global__ __launch_bounds__(F32Tile<HD>::kThreads) __attribute__((amdgpu_waves_
 
 // fp32 calls with segments of a few queries (the PMA's seeds: the expanded
 // call has k queries per set).  The tiled fp32 kernels give each (segment,
-// head) a 128-thread block in which k lanes are live and that walks every
-// key of the segment, so their time is that of the longest segment's walk.
+// head) a block of whose waves the first alone has queries, k of its 16 or 32
+// columns, and that walks every key of the segment, so their time is that of
+// the longest segment's walk.
 // Here the forward and dQ take one wave per (segment, query slot, head): its
 // 64 lanes take the segment's keys in turn (key kb + lane + 64 i) with
 // per-lane partials (running maximum and sum, or the dQ sum) that merge by a

@@ -10,9 +10,10 @@
 // us of host time (10-40 us are the kernels of a small batch) and the element-
 // wise passes around it read and write what its epilogue holds in registers.
 //
-// Block = 128 tokens x 64 NV features, four waves of 64 x 32 NV; operands are
-// staged by LDS-direct loads (esa_stage.h), 64 bytes of the contraction per
-// row and stage, three buffers deep, one barrier per stage.  bf16:
+// Block = 64 TT tokens x 64 NV features, four waves of 32 TT x 32 NV: 64 x 64
+// in fp32 and on small bf16 launches, else 128 x 128 or 256 (gemm_tile).
+// Operands are staged by LDS-direct loads (esa_stage.h), 64 bytes of the
+// contraction per row and stage, three buffers deep, one barrier per stage.  bf16:
 // v_mfma_f32_32x32x16_bf16 with the features as the MFMA's rows, so that a
 // lane holds four consecutive features of a token; the 32-token halves of the
 // accumulators pass through the wave's part of the (then free) stage buffers

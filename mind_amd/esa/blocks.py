@@ -1,16 +1,18 @@
 """The packed pre-norm blocks as one autograd function each.
 
 ``sab_block`` and ``pma_block`` run the computation of
-``masked_layers._sab_forward_packed`` / ``_pma_forward_packed`` (the
-reference's SABComplete.forward and PMAComplete.forward,
-esa/masked_layers.py:418-483, 574-621) on the same kernels, in the same order,
-but record one autograd node for a block instead of seven, and call the
-kernels without the layers between.  A small batch's step is bound by the
-host: a block's forward and backward issue about 35 launches, and an autograd
-function around each costs more than the launch (64 small molecules in fp32,
-three blocks: 3.3 -> 2.2 ms per train step).  The gradients of a block's
-shared inputs are added inside its GEMMs and kernels, with at most the
-roundings of the separate nodes.
+``masked_layers._sab_separate`` / ``_pma_separate`` (the reference's
+SABComplete.forward and PMAComplete.forward, esa/masked_layers.py:418-483,
+574-621), but record one autograd node for a block instead of seven, and call
+the kernels without the layers between: the norms and the attention are the
+separate functions', a Linear runs with what follows it in one kernel, and so
+do its input gradients, where linear.py says so.  A small batch's step is
+bound by the host: a block's forward and backward issue about 35 launches,
+and an autograd function around each costs more than the launch (64 small
+molecules in fp32, three blocks, with the attention's dispatch, on the
+separate functions' kernels: 3.48 -> 2.76 ms per train step).  The gradients
+of a block's shared inputs are added inside its GEMMs and kernels, with at
+most the roundings of the separate nodes.
 
 They take the calls that nothing else has to see as single operations
 (``eager.plain``), over the dtypes the kernels compute in: bf16 autocast with

@@ -50,7 +50,7 @@ class SmallMLP(nn.Module):
             nxt = layers[i + 1] if i + 1 < len(layers) else None
             if (type(layers[i]) is nn.Linear and type(nxt) in (Mish, nn.Mish) and hookless(layers[i])
                     and hookless(nxt)):
-                x = linear_mish(x, layers[i])   # Linear -> Mish: the bias gradient comes with Mish's backward
+                x = linear_mish(x, layers[i])   # one autograd function for Linear -> Mish
                 i += 2
             else:
                 x = apply(layers[i], x)

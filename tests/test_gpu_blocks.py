@@ -1,7 +1,7 @@
 """The packed blocks recorded as one autograd node (mind_amd.esa.blocks) against the separate functions: outputs
 and gradients of every input.
 
-Bar, norm-wise per tensor: the two differ in the order of the Linears' sums and in where partial gradients are added
+Bar, norm-wise per tensor (``_scale``): the two differ in the order of the Linears' sums and in where partial gradients are added
 and rounded.  fp32: roundings of 2^-24 per addition, far below 1e-5.  bf16 autocast: a value rounded to bf16 the
 other way, or a gradient rounded once more or once less, 2^-9 of its magnitude per rounding, at most four of them on
 any path: 2^-7."""
@@ -10,7 +10,7 @@ import pytest
 import torch
 
 from mind_amd import generators
-from mind_amd.esa import attention, blocks, masked_layers
+from mind_amd.esa import attention, blocks, linear, masked_layers
 from mind_amd.esa.packing import EdgeAdjacency, NodeAdjacency
 
 pytestmark = pytest.mark.gpu
@@ -30,7 +30,21 @@ def _sab(device, idx, mlp_layers, dropout=0.0, d=64):
     return blk.train()
 
 
-def _both(one, separate, x, params, g, amp):
+def _scale(grads, names, i):
+    """What gradient i is compared with: itself; a Linear's bias, which sums the rows that its weight (the tensor
+    before it) sums against inputs of about 1, with the larger of both (fc_k's is zero but for rounding)."""
+    own = float(grads[i].double().norm())
+    return max(own, float(grads[i - 1].double().norm())) if names[i].endswith("bias") and ".ln." not in names[i] else own
+
+
+def _agree(got, want, bar, names):
+    for i, (a, b, name) in enumerate(zip(got, want, names)):
+        assert a is not None and a.dtype == b.dtype and a.shape == b.shape, name
+        assert float((a.double() - b.double()).norm()) <= bar * _scale(want, names, i), name
+
+
+def _both(one, separate, x, params, g, amp, blk):
+    named = {id(p): n for n, p in blk.named_parameters()}
     res = []
     for fn in (one, separate):
         with torch.autocast("cuda", torch.bfloat16, enabled=amp):
@@ -40,13 +54,7 @@ def _both(one, separate, x, params, g, amp):
     (o1, g1), (o2, g2) = res
     bar = 2.0 ** -7 if amp else 1e-5
     assert o1.dtype == o2.dtype and float((o1.double() - o2.double()).norm()) <= bar * float(o2.double().norm())
-    size = 0.0
-    for a, b in zip(g1, g2):
-        assert a.dtype == b.dtype and a.shape == b.shape
-        # a bias sums the rows that its weight (the tensor before it) sums against inputs of about 1; fc_k's is zero
-        # but for rounding, the softmax being unchanged by it
-        size = max(float(b.double().norm()), size if b.dim() == 1 else 0.0)
-        assert float((a.double() - b.double()).norm()) <= bar * size
+    _agree(g1, g2, bar, ["x"] + [named[id(p)] for p in params])
 
 
 @pytest.mark.parametrize("amp", [False, True])
@@ -68,7 +76,7 @@ def test_sab_block(device, amp, idx, node, mlp_layers, dropout):
     state = torch.get_rng_state()
     seed = attention.draw_dropout_seed() if dropout else None   # what the block draws from the same state
     torch.set_rng_state(state)
-    _both(one, separate, x, params, g, amp)
+    _both(one, separate, x, params, g, amp, blk)
 
 
 @pytest.mark.parametrize("amp", [False, True])
@@ -84,7 +92,7 @@ def test_pma_block(device, amp, k_seeds, dropout):
     seed = attention.draw_dropout_seed() if dropout else None
     torch.set_rng_state(state)
     _both(lambda: blocks.pma_block(blk, x, tokens, dropout, None),
-          lambda: masked_layers._pma_separate(blk, x, tokens, seed), x, list(blk.parameters()), g, amp)
+          lambda: masked_layers._pma_separate(blk, x, tokens, seed), x, list(blk.parameters()), g, amp, blk)
 
 
 def test_frozen_parameters_and_input(device):
@@ -135,7 +143,8 @@ def test_strided_and_misaligned_parameters(device, amp):
         x = torch.randn(tokens.num_tokens, 64, device=device, requires_grad=True)
         g = torch.randn(tokens.num_tokens, 64, device=device)
         _both(lambda: blocks.sab_block(blk, x, tokens, False, 0.0, None),
-              lambda: masked_layers._sab_separate(blk, x, tokens), x, [blk.mlp.mlp[2].weight, blk.norm.ln.weight], g, amp)
+              lambda: masked_layers._sab_separate(blk, x, tokens), x, [blk.mlp.mlp[2].weight, blk.norm.ln.weight], g,
+              amp, blk)
 
 
 def _off_boundary(t):
@@ -156,7 +165,7 @@ def test_rows_off_a_boundary(device, amp):
     g = _off_boundary(torch.randn(tokens.batch_size, 2, 64, device=device))
     params = [p for n, p in blk.named_parameters() if "norm_mlp" not in n]
     _both(lambda: blocks.pma_block(blk, x, tokens, 0.0, None), lambda: masked_layers._pma_separate(blk, x, tokens), x,
-          params, g, amp)
+          params, g, amp, blk)
 
 
 @pytest.mark.parametrize("amp", [False, True])
@@ -190,20 +199,6 @@ def _pma(device, mlp=True, dropout=0.0, k_seeds=2):
 
 def _used(blk):
     return {n: p for n, p in blk.named_parameters() if blk.use_mlp or "norm_mlp" not in n}
-
-
-def _scale(grads, i):
-    """What gradient i is compared with: itself; a Linear's bias, which sums the rows that its weight (the tensor
-    before it) sums against inputs of about 1, with the larger of both (fc_k's is zero but for rounding)."""
-    return max(float(t.double().norm()) for t in grads[max(i - 1, 0):i + 1]) if grads[i].dim() == 1 else float(
-        grads[i].double().norm())
-
-
-def _agree(got, want, bar, names):
-    for i, (a, b, name) in enumerate(zip(got, want, names)):
-        size = _scale(want, i) if name.endswith("bias") and ".ln." not in name else float(b.double().norm())
-        assert a is not None and a.dtype == b.dtype and a.shape == b.shape, name
-        assert float((a.double() - b.double()).norm()) <= bar * size, name
 
 
 class _Held(torch.nn.Module):
@@ -340,3 +335,21 @@ def test_output_gradient_off_a_boundary(device, amp, pma, mlp):
     got = torch.autograd.grad(out, [x, *used.values()], g, retain_graph=True)
     want = torch.autograd.grad(out, [x, *used.values()], g.clone())
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("amp", [False, True])
+@pytest.mark.parametrize("pma", [False, True])
+@pytest.mark.parametrize("which", ["one by one", "library"])
+def test_large_block_routes(device, monkeypatch, amp, pma, which):
+    """What only large blocks take, at a small size: weight gradients computed one by one, products that stay with
+    the library."""
+    if which == "library":
+        monkeypatch.setattr(linear, "_library_rate", lambda *a: True)
+    else:
+        monkeypatch.setattr(blocks, "_TOGETHER", 0)
+    tokens = _tokens(device, False)
+    blk = _pma(device) if pma else _sab(device, 1, 3)
+    x = torch.randn(tokens.num_tokens, 64, device=device, requires_grad=True)
+    g = torch.randn(tokens.batch_size, 2, 64, device=device) if pma else torch.randn(tokens.num_tokens, 64, device=device)
+    one, separate = _packed(blk, tokens)
+    _both(lambda: one(x), lambda: separate(x), x, list(_used(blk).values()), g, amp, blk)
