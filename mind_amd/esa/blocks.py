@@ -194,9 +194,11 @@ def _mlp_forward(x, params, residual, keep, fused):
 
 # Token counts up to which a block's weight gradients wait for the end of its backward and run in one launch: the
 # launches of single weights leave the chip partly idle at their ends and each costs the host.  Six weights of a SAB
-# block with an MLP, apart and together, us: fp32 21,752 x 128 105 / 63; bf16 33,000 x 256 99 / 56, 65,536 x 512
-# (MLP 2048) 478 / 448; 129,850 x 512 864 / 934, where a weight alone fills the chip and takes longer row ranges.
-# Above the line the operands are freed early, too.
+# block with an MLP, together / apart, us: fp32 128 wide (MLP 256) 92 / 136 at 33,000 tokens; bf16 256 (1024) 91 / 135
+# at 33,000 and 145 / 203 at 65,000; 512 (2048) 230 / 304 at 33,000 and 457 / 491 at 65,000.  Up to the line every
+# width gains.  Beyond, that is the width's matter: 512 loses from 100,000 tokens on (710 / 703; 131,000: 935 / 903),
+# where a weight alone fills the chip, 192 (768) at 262,000 (482 / 456), while 256 and 128 gain still (131,000: 256 /
+# 337, 92 / 143); and the operands of all six stay allocated to the end.
 _TOGETHER = 65536
 
 
