@@ -1228,41 +1228,11 @@ def cpu_baseline_block(gb, types, emb, proj, model, heads) -> dict:
                        f"2 warm-ups")}
 
 
-def count_gemm_flops(step) -> int:
-    """FLOPs of the matrix products one call of `step` runs (forward and backward): every aten mm / addmm /
-    bmm / baddbmm dispatched (in-place forms included), 2 m n k each (batch included), from its operands'
-    shapes."""
-    from torch.utils._python_dispatch import TorchDispatchMode
-
-    class GemmCount(TorchDispatchMode):
-        flops = 0
-
-        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
-            name = func._overloadpacket.__name__.rstrip("_")
-            if name in ("mm", "bmm"):
-                a, b = args[0], args[1]
-            elif name in ("addmm", "baddbmm"):
-                a, b = args[1], args[2]
-            else:
-                a = b = None
-            if a is not None:
-                batch = a.shape[0] if a.dim() == 3 else 1
-                GemmCount.flops += 2 * batch * a.shape[-2] * a.shape[-1] * b.shape[-1]
-            return func(*args, **(kwargs or {}))
-
-    with GemmCount():
-        step()
-    return GemmCount.flops
-
-
-def stack_flops(step, gb, d: int, layers: str, k_seeds: int, mlp: int) -> dict:
-    """Exact FLOPs of one configuration-4 train step: the GEMMs counted as they are dispatched over one step
-    (projections, MLPs, weight and input gradients, each product with its real shape), plus the attention by
-    pair counts, 14 D per (query, key) pair for forward + backward (QK^T and PV; QK^T recomputation, dP, dV,
-    dK, dQ): the S layers' pairs are sum L^2, the masked M layers' the mask's nnz (effective), PMA's
-    k_seeds * T.  gemm_analytic restates the GEMMs from the layer shapes (3x the forward products: forward,
-    input and weight gradients) as a check of the count."""
-    gemm = count_gemm_flops(step)
+def stack_flops(gb, d: int, layers: str, k_seeds: int, mlp: int) -> dict:
+    """Exact FLOPs of one configuration-4 train step: the GEMMs from the layer shapes (3x the forward products:
+    forward, input and weight gradients, whether the library or this framework's kernels run them), plus the
+    attention by pair counts, 14 D per (query, key) pair for forward + backward (QK^T and PV; QK^T recomputation, dP,
+    dV, dK, dQ): the S layers' pairs are sum L^2, the masked M layers' the mask's nnz (effective), PMA's k_seeds * T."""
     stats = edge_mask_stats(gb.edge_index[0].astype(np.int64), gb.edge_index[1].astype(np.int64), gb.cu_seqlens)
     t, b = gb.num_tokens, gb.num_graphs
     n_enc = sum(1 for lt in layers[: layers.index("P")] if lt in "MS")
@@ -1271,7 +1241,8 @@ def stack_flops(step, gb, d: int, layers: str, k_seeds: int, mlp: int) -> dict:
     pma += 2 * 2 * b * k_seeds * d * mlp + 2 * b * d * d                      # PMA MLP; decoder_linear
     attn = {"S": 14 * d * gb.sum_sq * layers.count("S"), "M": 14 * d * stats["nnz"] * layers.count("M"),
             "P": 14 * d * k_seeds * t * layers.count("P")}
-    return {"gemm": gemm, "gemm_analytic": 3 * (enc + pma), "attention": attn, "total": gemm + sum(attn.values()),
+    gemm = 3 * (enc + pma)
+    return {"gemm": gemm, "attention": attn, "total": gemm + sum(attn.values()),
             "mask_nnz": stats["nnz"], "sum_L2": gb.sum_sq}
 
 
@@ -1321,11 +1292,11 @@ def bench_stack(args, sub: bool = False):
     ms, wall_ms, kern, ms_prof = timed(step, args.steps, args.warmup)
     lib_ms = sum(k["avg_us"] * k["launches"] for k in kern.values()) / 1e3 / args.steps
     attn_ms = sum(k["avg_us"] * k["launches"] for n, k in kern.items() if n.startswith("attn")) / 1e3 / args.steps
-    fl = stack_flops(step, gb, d, layers, 4, 2048)
+    fl = stack_flops(gb, d, layers, 4, 2048)
     achieved = fl["total"] / (ms * 1e-3) / 1e12
     roofline = {"bound": "mfma", "kernel": "whole train step (GEMMs + attention)", "achieved": achieved,
                 "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s", "frac": achieved / PEAK_BF16_TFLOPS, "traffic": None,
-                "flops": "exact: GEMMs counted as dispatched over one step, attention 14 D per pair "
+                "flops": "exact: GEMMs from the layer shapes, attention 14 D per pair "
                          "(S: sum L^2, M: mask nnz, P: seeds x tokens)"}
     split = {"library_kernels_ms": lib_ms, "attention_ms": attn_ms, "other_ms": ms - lib_ms,
              "what": "library_kernels: this library's launches by HIP events (attention, LayerNorm, Mish, column "
