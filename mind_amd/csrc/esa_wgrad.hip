@@ -209,9 +209,10 @@ __global__ __launch_bounds__(256, 2) void wgrad_kernel(const WgradArgs a) {
   if (bias)
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      const float b = bias_before[u] + (bias_sum[u] + bs[u]), both = b + __shfl_xor(b, 32);   // the lane halves hold different tokens
+      const float b = bias_before[u] + (bias_sum[u] + bs[u]);
+      const float sum_b = b + __shfl_xor(b, 32);   // the lane halves hold different tokens
       const int o = o0 + wo + 32 * u + col;
-      if (half == 0 && o < p.out) p.bpart[(size_t)split * p.out + o] = both;
+      if (half == 0 && o < p.out) p.bpart[(size_t)split * p.out + o] = sum_b;
     }
 }
 
